@@ -1847,11 +1847,14 @@ struct ModelStep {
   ModelOp op;
   ModelAppendParams append{};
   bgtq_encode_job encode{};
-  ModelScoresParams scores{};
-  int kv_count = 0, lds = 0;
+  ModelScoresParams scores;  // set by the op that uses it (one of scores and attn)
+  int kv_count = 0, book_bytes = 0;
+  size_t packed_bytes = 0, norm_bytes = 0, q_bytes = 0, score_bytes = 0;  // bytes a scores step reads and spans
   ModelAttnParams attn{};
-  int64_t score_rows = 0;
 };
+
+// Query floats per dimension in the LDS budget that bounds a scores step's books.
+constexpr int kMaxScoresQueryFloats = 16;
 
 bool aligned(const void *p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
 
@@ -1948,6 +1951,7 @@ bgtq_status plan_model_dispatch(const bgtq_model_dispatch &D, size_t idx, ModelS
       const uint64_t n_tok = std::min<uint64_t>(tokens, x);
       const uint64_t read = std::min<uint64_t>(n_tok, start + rows);
       ModelScoresParams &sp = st->scores;
+      std::memset(&sp, 0, sizeof(sp));
       st->op = ModelOp::Scores;
       sp.rows = (int32_t)rows;
       sp.start = (int32_t)start;
@@ -1972,13 +1976,15 @@ bgtq_status plan_model_dispatch(const bgtq_model_dispatch &D, size_t idx, ModelS
         q_heads_used = (head + 1) * gqa;
         if (bgtq_status s = need(3, read * (uint64_t)t->info.row_bytes, 1)) return s;
         if (bgtq_status s = need(4, read * (uint64_t)t->info.norm_stride * 2, 2)) return s;
-        sp.tables = t->dev();
-        sp.packed = static_cast<const uint8_t *>(D.bindings[3].ptr);
-        sp.norms = static_cast<const uint16_t *>(D.bindings[4].ptr);
-        sp.head0 = (int32_t)head;
+        sp.jobs[0].tables = t->dev();
+        sp.jobs[0].packed = static_cast<const uint8_t *>(D.bindings[3].ptr);
+        sp.jobs[0].norms = static_cast<const uint16_t *>(D.bindings[4].ptr);
+        sp.jobs[0].head = (int32_t)head;
         st->kv_count = 1;
-        st->lds = model_scores_lds_bytes((int)d, t->info.n_books * t->info.max_centroids);
-        if (st->lds > 64 * 1024)
+        st->packed_bytes = (size_t)(read * (uint64_t)t->info.row_bytes);
+        st->norm_bytes = (size_t)(read * (uint64_t)t->info.norm_stride * 2);
+        st->book_bytes = t->info.n_books * t->info.max_centroids * 4;
+        if (st->book_bytes > 64 * 1024 - kMaxScoresQueryFloats * (int)d * 4)
           return fail(BGTQ_ERR_UNSUPPORTED, "dispatch %zu (compressed_dot): centroid books too large", idx);
       } else {
         if (read > capacity)
@@ -1989,17 +1995,19 @@ bgtq_status plan_model_dispatch(const bgtq_model_dispatch &D, size_t idx, ModelS
         sp.capacity = (int32_t)capacity;
         sp.head0 = 0;
         st->kv_count = (int)kvh;
-        st->lds = model_scores_lds_bytes((int)d, 0);
       }
       if (rows && n_tok) {
-        if (bgtq_status s = need(qb, ((rows - 1) * qh + q_heads_used) * d * 4, 4)) return s;
-        if (bgtq_status s = need(sb, (((rows - 1) * qh + q_heads_used - 1) * tokens + n_tok) * 4, 4)) return s;
+        st->q_bytes = (size_t)(((rows - 1) * qh + q_heads_used) * d * 4);
+        st->score_bytes = (size_t)((((rows - 1) * qh + q_heads_used - 1) * tokens + n_tok) * 4);
+        if (bgtq_status s = need(qb, st->q_bytes, 4)) return s;
+        if (bgtq_status s = need(sb, st->score_bytes, 4)) return s;
       }
       sp.q = static_cast<const float *>(D.bindings[qb].ptr);
       sp.scores = static_cast<float *>(D.bindings[sb].ptr);
       return BGTQ_OK;
     }
     ModelAttnParams &ap = st->attn;
+    ap.rows = (int32_t)rows;
     ap.tokens = (int32_t)tokens;
     ap.start = (int32_t)start;
     ap.q_heads = (int32_t)qh;
@@ -2012,19 +2020,19 @@ bgtq_status plan_model_dispatch(const bgtq_model_dispatch &D, size_t idx, ModelS
     ap.out = static_cast<float *>(D.bindings[5].ptr);
     if (name == "softmax") {
       st->op = ModelOp::Softmax;
-      st->score_rows = (int64_t)std::min<uint64_t>(x, rows * qh);
-      if (bgtq_status s = need(3, (uint64_t)st->score_rows * tokens * 4, 4)) return s;
-      if (bgtq_status s = need(4, (uint64_t)st->score_rows * tokens * 4, 4)) return s;
+      ap.score_rows = (int64_t)std::min<uint64_t>(x, rows * qh);
+      if (bgtq_status s = need(3, (uint64_t)ap.score_rows * tokens * 4, 4)) return s;
+      if (bgtq_status s = need(4, (uint64_t)ap.score_rows * tokens * 4, 4)) return s;
       return BGTQ_OK;
     }
     st->op = ModelOp::Weighted;
     const uint64_t outs = std::min<uint64_t>(x, rows * qh * d);
     ap.x_limit = (int64_t)outs;
-    st->score_rows = (int64_t)((outs + d - 1) / d);
+    ap.score_rows = (int64_t)((outs + d - 1) / d);
     if (outs && span > capacity)
       return fail(BGTQ_ERR_RANGE, "dispatch %zu (weighted): tokens beyond capacity %llu", idx,
                   (unsigned long long)capacity);
-    if (bgtq_status s = need(4, (uint64_t)st->score_rows * tokens * 4, 4)) return s;
+    if (bgtq_status s = need(4, (uint64_t)ap.score_rows * tokens * 4, 4)) return s;
     if (bgtq_status s = need(2, outs ? kvh * capacity * d * 2 : 0, 2)) return s;
     if (bgtq_status s = need(5, outs * 4, 4)) return s;
     return BGTQ_OK;
@@ -2034,6 +2042,32 @@ bgtq_status plan_model_dispatch(const bgtq_model_dispatch &D, size_t idx, ModelS
     if (name == o)
       return fail(BGTQ_ERR_UNSUPPORTED, "model kernel %s is outside the attention path this library serves", D.name);
   return fail(BGTQ_ERR_RANGE, "dispatch %zu: unknown model kernel %s", idx, D.name);
+}
+
+// Whether the bytes [a, a + na) and [b, b + nb) share any.
+bool overlap(const void *a, size_t na, const void *b, size_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return na && nb && x < y + nb && y < x + na;
+}
+
+// Whether a compressed_dot can run beside the `heads` before it (first[0 ..
+// heads)) in one launch: the same rows, tokens, queries and scores buffer,
+// a KV head of its own, and no step's scores on what another one reads.
+bool scores_join(const ModelStep *first, int heads, const ModelStep &next) {
+  if (next.op != ModelOp::Scores || next.scores.k) return false;
+  const ModelScoresParams &a = first[0].scores, &b = next.scores;
+  if (a.q != b.q || a.scores != b.scores || a.rows != b.rows || a.start != b.start || a.q_heads != b.q_heads ||
+      a.gqa != b.gqa || a.dim != b.dim || a.tokens != b.tokens || a.n_tok != b.n_tok || a.y_limit != b.y_limit)
+    return false;
+  auto reads = [](const ModelStep &w, const ModelStep &r) {  // r reads what w writes
+    const ModelScoresJob &j = r.scores.jobs[0];
+    return overlap(w.scores.scores, w.score_bytes, j.packed, r.packed_bytes) ||
+           overlap(w.scores.scores, w.score_bytes, j.norms, r.norm_bytes) ||
+           overlap(w.scores.scores, w.score_bytes, r.scores.q, r.q_bytes);
+  };
+  for (int h = 0; h < heads; ++h)
+    if (first[h].scores.jobs[0].head == b.jobs[0].head || reads(first[h], next) || reads(next, first[h])) return false;
+  return true;
 }
 
 }  // namespace
@@ -2054,7 +2088,8 @@ bgtq_status bgtq_model_submit(bgtq_context *ctx, const bgtq_model_dispatch *disp
     jobs.clear();
     return s;
   };
-  for (const ModelStep &st : steps) {
+  for (size_t i = 0; i < n; ++i) {
+    const ModelStep &st = steps[i];
     if (st.op == ModelOp::Encode) {
       jobs.push_back(st.encode);
       continue;
@@ -2062,12 +2097,24 @@ bgtq_status bgtq_model_submit(bgtq_context *ctx, const bgtq_model_dispatch *disp
     if (bgtq_status s = flush()) return s;
     switch (st.op) {
       case ModelOp::Append: HIP_TRY(launch_model_append(st.append, ctx->stream), "model append"); break;
-      case ModelOp::Scores:
-        HIP_TRY(launch_model_scores(st.scores, st.kv_count, st.lds, ctx->stream), "model scores");
+      case ModelOp::Scores: {
+        // The KV heads' compressed_dot dispatches of one layer, one after
+        // another, share a launch.
+        ModelScoresParams sp = st.scores;
+        int heads = st.kv_count, book_bytes = st.book_bytes;
+        while (!sp.k && heads < kMaxKvHeads && i + 1 < n && scores_join(steps.data() + i + 1 - heads, heads, steps[i + 1])) {
+          ++i;
+          sp.jobs[heads++] = steps[i].scores.jobs[0];
+          book_bytes = std::max(book_bytes, steps[i].book_bytes);
+        }
+        HIP_TRY(launch_model_scores(sp, heads, book_bytes, ctx->stream), "model scores");
         break;
-      case ModelOp::Softmax: HIP_TRY(launch_model_softmax(st.attn, st.score_rows, ctx->stream), "model softmax"); break;
+      }
+      case ModelOp::Softmax:
+        HIP_TRY(launch_model_softmax(st.attn, ctx->stream), "model softmax");
+        break;
       case ModelOp::Weighted:
-        HIP_TRY(launch_model_weighted(st.attn, st.score_rows, ctx->stream), "model weighted");
+        HIP_TRY(launch_model_weighted(st.attn, ctx->stream), "model weighted");
         break;
       default: break;
     }

@@ -73,6 +73,15 @@ __device__ __forceinline__ float row_max(float v) {
   return v;
 }
 
+// Sum over the 16 lanes of each row, in every lane (the same rotations).
+__device__ __forceinline__ float row_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));
+  return v;
+}
+
 // Minimum over the wave's 64 lanes, in every lane: DPP row rotations, then
 // the row swaps (no LDS round trip).
 __device__ __forceinline__ int wave_min(int v) {

@@ -229,3 +229,67 @@ def test_model_dispatch_coverage_and_checks(device, oracle):
     finally:
         for t, _ in heads:
             t.destroy()
+
+
+@pytest.mark.parametrize("key_format,kvh,gqa,d,steps", [
+    ("packed", 3, 3, 64, ((0, 1), (1, 16), (17, 31), (48, 85), (133, 1))),   # tile edges of tokens and items
+    ("packed", 2, 16, 128, ((0, 5), (5, 129), (134, 2))),                    # the widest GQA, d=128, ragged tiles
+    ("fp16", 1, 5, 128, ((0, 127), (127, 1), (128, 13))),
+])
+def test_model_dispatch_tile_edges(device, oracle, key_format, kvh, gqa, d, steps):
+    import bgtq
+    from bgtq import calibrate
+    heads = []
+    if key_format == "packed":
+        for make in (calibrate.layout_a, calibrate.layout_b, calibrate.layout_a)[:kvh]:
+            integer, floating = bgtq.tables(make(d))
+            heads.append((bgtq.Tables(device, integer=integer, floating=floating),
+                          oracle.Layout.from_model_config(integer, floating)))
+    try:
+        print("model dispatch edges", key_format, kvh, gqa, d, flush=True)
+        _attention_case(device, oracle, key_format, heads, kvh=kvh, gqa=gqa, d=d, steps=steps, seed=11)
+    finally:
+        for t, _ in heads:
+            t.destroy()
+
+
+@pytest.mark.parametrize("kvh,gqa,rows,start", [(2, 3, 21, 180), (2, 1, 3, 4600), (1, 5, 13, 4400)])
+def test_model_dispatch_weighted_causal_ends(device, kvh, gqa, rows, start):
+    """softmax and weighted over more tokens than one pass of either weighted
+    kernel holds, for chunks whose later V rows hold an infinity that the
+    earlier query rows do not attend to and whose cache rows past the chunk
+    are NaN: against FP64, within an FP32 sum of `tokens` terms
+    (tokens 2^-24 of the largest value; the exponentials and the division
+    add a few 2^-24 of each probability)."""
+    import torch
+    import bgtq
+    ops = bgtq.ModelOps.create(device)
+    d = 64
+    qh, tokens = kvh * gqa, start + rows
+    cap = tokens + 23
+    g = torch.Generator(device="cuda").manual_seed(5)
+    scores = torch.randn((rows, qh, tokens), generator=g, device="cuda") * 3
+    v = torch.randn((kvh, cap, d), generator=g, device="cuda").half()
+    odd = rows // 2
+    v[kvh - 1, start + odd, 7] = float("inf")  # rows odd.. of the last KV head meet it
+    v[:, tokens:] = float("nan")               # cache rows not written yet
+    p = [rows, tokens, cap, start, qh, kvh, gqa, d]
+    probs = torch.full((rows, qh, tokens), float("nan"), device="cuda")
+    attn = torch.full((rows, qh, d), float("nan"), device="cuda")
+    bufs = [scores, None, v.view(torch.int16), scores, probs, attn]
+    cmd = ops.commands()
+    cmd.dispatch("softmax", p, bufs, rows * qh)
+    cmd.dispatch("weighted", p, bufs, rows * qh * d)
+    cmd.submit()
+    probs, attn = probs.cpu(), attn.cpu()
+    live = torch.arange(tokens)[None, :] <= start + torch.arange(rows)[:, None]
+    ref = torch.softmax(scores.cpu().double().masked_fill(~live[:, None], float("-inf")), -1)
+    assert torch.all(probs[~live[:, None].expand_as(probs)] == 0)
+    torch.testing.assert_close(probs.double(), ref, rtol=tokens * 2.0 ** -24, atol=1e-30)
+    vf = v.cpu().double()[:, :tokens]
+    hit = vf.isinf()
+    out = torch.einsum("rkgt,ktd->rkgd", ref.view(rows, kvh, gqa, tokens), vf.masked_fill(hit, 0.0)).reshape(rows, qh, d)
+    inf = torch.zeros_like(out, dtype=torch.bool)
+    inf[odd:, (kvh - 1) * gqa:, 7] = True
+    assert torch.isposinf(attn[inf]).all()
+    torch.testing.assert_close(attn.double()[~inf], out[~inf], rtol=0, atol=2 * tokens * 2.0 ** -24)
