@@ -26,7 +26,7 @@ OBJ_DIR = PKG / "_build"
 INCLUDE = PKG.parent / "include"
 ARCH = os.environ.get("BGTQ_OFFLOAD_ARCH", "gfx950")
 
-DEVICE_SOURCES = ["encode.hip", "encode_bulk.hip", "encode_wave.hip", "decode.hip", "decode_fast.hip",
+DEVICE_SOURCES = ["encode.hip", "encode_bulk.hip", "encode_tile.hip", "encode_wave.hip", "decode.hip", "decode_fast.hip",
                   "decode_fast_any64.hip", "decode_fast_any64_append.hip", "decode_fast_any64_prefill.hip",
                   "decode_fast_any128.hip",
                   "decode_fast_d64.hip", "decode_fast_d64_append.hip", "decode_fast_d64_prefill.hip",

@@ -177,6 +177,7 @@ struct bgtq_tables {
   bgtq_tables_info info{};
   DeviceBuffer blob;
   std::vector<uint8_t> host;  // the DevTables image uploaded to blob
+  bool tile_encode = false;   // encode_tile_layout of the image
   const DevTables *dev() const { return static_cast<const DevTables *>(blob.ptr); }
   const DevTables *h() const { return reinterpret_cast<const DevTables *>(host.data()); }
 };
@@ -595,6 +596,7 @@ bgtq_status bgtq_tables_create(bgtq_context *ctx, const uint32_t *integer, size_
           }
         }
   }
+  t->tile_encode = encode_tile_layout(T);
   t->info = bgtq_tables_info{(int32_t)d, (int32_t)ng, (int32_t)rb, (int32_t)nstride, (int32_t)nib, (int32_t)mc, ncb, nb,
                              (uint64_t)total};
   bgtq_status s = ctx->use();
@@ -878,10 +880,18 @@ static int device_cus() {
   return cached[dev];
 }
 
-// Below this many rows per launch the wave-per-row encoder (short latency per
-// row) runs; larger launches use a thread-per-row encoder (more rows per
-// instruction): the bulk one where the layout qualifies, else the generic one.
-constexpr int64_t kEncodeWaveMaxRows = 16384;
+// Below a number of rows per launch the wave-per-row encoder (short latency
+// per row) runs, above it an encoder that takes more rows per instruction.
+// Measured in microseconds per call, wave against tile encoder: d=64, 6144
+// rows 9.4 / 11.4, 12,288 rows 13.3 / 11.1; d=128, 1000 rows 9.5 / 23.9, 8000
+// rows 44.2 / 21.9. The thread-per-row encoder of the layouts the tile encoder
+// does not take starts later.
+constexpr int kEncodeTile = 3;  // encoder kind beside encode_bulk_kind's
+static int64_t encode_wave_max_rows(int dim, bool tile) { return !tile ? 16384 : dim == 64 ? 8192 : 4096; }
+// Layout B at d=64 from this many rows: the thread-per-row encoder with the
+// layout's structure at compile time (51 us for 368,640 rows, 57 with the tile
+// encoder; 44 against 41 for 262,144, 20 against 13 for 32,768).
+constexpr int64_t kEncodeBulkMinRows = 300000;
 
 // ---------------------------------------------------------------- batched entry points
 bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq_encode_job *jobs, size_t n_jobs) {
@@ -899,16 +909,18 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
     if (j.src_row_stride > INT32_MAX) return fail(BGTQ_ERR_RANGE, "encode job %zu: row stride above 2^31 - 1", i);
   }
   if (bgtq_status s = ctx->use()) return s;
-  // Group jobs by dimension and bulk-encoder kind. Few rows in all (a decode
+  // Group jobs by dimension and encoder kind. Few rows in all (a decode
   // step's appended tokens) go to the wave-per-row encoder, its jobs in kernel
-  // arguments (kEncodeJobsPerLaunch per launch); otherwise one thread-per-row
+  // arguments (kEncodeJobsPerLaunch per launch); otherwise one tile or thread-per-row
   // launch covers up to kEncodeJobTable jobs through the context's job table,
   // so every job's rows share one grid and one round of workgroups.
   std::map<std::pair<int, int>, std::vector<size_t>> by_kind;
   for (size_t i = 0; i < n_jobs; ++i)
     if (jobs[i].rows > 0) {
       const bgtq_tables *t = jobs[i].tables;
-      by_kind[{t->info.dim, encode_bulk_kind(t->h())}].push_back(i);
+      const bool tile = t->tile_encode && jobs[i].src_row_stride <= kTileMaxStride;
+      const int bulk = encode_bulk_kind(t->h());
+      by_kind[{t->info.dim, bulk ? bulk : tile ? kEncodeTile : 0}].push_back(i);
     }
   const bool src_f32 = src_dtype == BGTQ_DTYPE_F32;
   auto job_dev = [&](const bgtq_encode_job &j) {
@@ -930,11 +942,14 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
     const std::vector<size_t> &idx = kv.second;
     int64_t total_rows = 0;
     int wave_lds = 0;
+    bool tile = true;
     for (size_t i : idx) {
       total_rows += jobs[i].rows;
+      tile &= jobs[i].tables->tile_encode && jobs[i].src_row_stride <= kTileMaxStride;
       wave_lds = std::max(wave_lds, encode_wave_lds_bytes(dim, (int)jobs[i].tables->h()->off_rot));
     }
-    if (wave_lds <= 160 * 1024 && total_rows < kEncodeWaveMaxRows) {
+    if (kind == 1 && total_rows >= kEncodeBulkMinRows) tile = false;
+    if (wave_lds <= 160 * 1024 && total_rows < encode_wave_max_rows(dim, tile)) {
       for (size_t b = 0; b < idx.size(); b += kEncodeJobsPerLaunch) {
         EncodeLaunch L{};
         int64_t max_rows = 0, rows = 0;
@@ -958,7 +973,7 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
     for (size_t b = 0; b < idx.size(); b += kEncodeJobTable) {
       const size_t e = std::min(idx.size(), b + kEncodeJobTable);
       int64_t max_rows = 0;
-      int lut_max = 0, books_max = 0;
+      int lut_max = 0, books_max = 0, cb_max = 0, groups_max = 0, rb_max = 0;
       for (size_t c = b; c < e; c += kEncodeJobsPerLaunch) {
         EncodeLaunch L{};
         for (size_t k = c; k < std::min(e, c + kEncodeJobsPerLaunch); ++k) {
@@ -967,15 +982,19 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
           max_rows = std::max(max_rows, j.rows);
           lut_max = std::max(lut_max, j.tables->info.n_codebooks * 256);
           books_max = std::max(books_max, j.tables->info.n_books * j.tables->info.max_centroids);
+          cb_max = std::max(cb_max, j.tables->info.n_codebooks);
+          groups_max = std::max(groups_max, j.tables->info.groups);
+          rb_max = std::max(rb_max, j.tables->info.row_bytes);
         }
         HIP_TRY(launch_encode_upload(L, table, (int)(c - b), ctx->stream), "encode job upload");
       }
       const int n = (int)(e - b);
-      const int wg = kind == 1 ? 256 : 128;
-      if (kind && encode_bulk_lds_bytes(kind, wg, lut_max, books_max) <= 64 * 1024) {
-        // Bulk encodes of layout-B-shaped tables: thread per row, structure at compile time.
-        HIP_TRY(launch_encode_bulk(table, n, kind, wg, src_f32, max_rows, lut_max, books_max, ctx->stream),
+      if (tile && encode_tile_lds_bytes(dim, cb_max, groups_max, rb_max) <= 160 * 1024) {
+        HIP_TRY(launch_encode_tile(table, n, dim, src_f32, max_rows, device_cus(), cb_max, groups_max, rb_max, ctx->stream),
                 "encode launch");
+      } else if (kind == 1 && encode_bulk_lds_bytes(lut_max, books_max) <= 64 * 1024) {
+        // Bulk encodes of layout-B-shaped tables: thread per row, structure at compile time.
+        HIP_TRY(launch_encode_bulk(table, n, src_f32, max_rows, lut_max, books_max, ctx->stream), "encode launch");
       } else {
         HIP_TRY(launch_encode(table, n, dim, src_f32, max_rows, ctx->stream), "encode launch");
       }

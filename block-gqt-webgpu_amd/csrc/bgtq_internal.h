@@ -353,15 +353,24 @@ int encode_wave_lds_bytes(int dim, int enc_bytes);
 hipError_t launch_encode_wave(const EncodeLaunch &launch, int dim, int src_f32, int wgs_per_job, int lds_bytes,
                               hipStream_t stream);
 // Bulk thread-per-row encode (encode_bulk.hip) for layouts of two equal
-// contiguous groups with nibble codes in the first (layout B at d 64 / 128):
-// kind 1 (d=64) or 2 (d=128), 0 when the layout does not qualify. wg rows per
-// workgroup: 256 (d=64) or 128 (d=128). The launch needs
+// contiguous groups at d=64 with nibble codes in the first (layout B): kind
+// 1, 0 when the layout does not qualify. The launch needs
 // encode_bulk_lds_bytes of dynamic LDS for the largest LUT (bytes) and book
 // set (floats) among its jobs.
 int encode_bulk_kind(const DevTables *T);
-int encode_bulk_lds_bytes(int kind, int wg, int lut_bytes, int book_floats);
-hipError_t launch_encode_bulk(const EncodeJobDev *jobs, int n_jobs, int kind, int wg, int src_f32, int64_t max_rows,
-                              int lut_bytes, int book_floats, hipStream_t stream);
+int encode_bulk_lds_bytes(int lut_bytes, int book_floats);
+hipError_t launch_encode_bulk(const EncodeJobDev *jobs, int n_jobs, int src_f32, int64_t max_rows, int lut_bytes,
+                              int book_floats, hipStream_t stream);
+// Tile encode (encode_tile.hip, 16 rows per wave, rotations on the matrix
+// cores): whether a table set's layout qualifies (ascending contiguous groups
+// with even boundaries, one centroid book per codebook, its LDS within
+// bounds), the LDS of a launch's largest codebook count, group count and row
+// bytes, and its launcher. Source row strides up to kTileMaxStride elements.
+constexpr int64_t kTileMaxStride = 1 << 24;
+bool encode_tile_layout(const DevTables *T);
+int encode_tile_lds_bytes(int dim, int n_codebooks, int groups, int row_bytes);
+hipError_t launch_encode_tile(const EncodeJobDev *jobs, int n_jobs, int dim, int src_f32, int64_t max_rows, int cus,
+                              int max_codebooks, int max_groups, int max_row_bytes, hipStream_t stream);
 hipError_t launch_rotate_q(const DecodeParams &p, const float *q, float *qr, hipStream_t stream);
 // Device address of this device's bgtq_decode_noalloc scratch (decode_scratch.hip).
 hipError_t decode_scratch_setup(int device, hipStream_t stream, uint8_t **out);

@@ -11,8 +11,8 @@
 //  * y_j = sum_i xn_i R[j][i] (production_math.py:16) is one FMA chain over
 //    the group of j in ascending i from +0, the order of the CPU sgemm (the
 //    off-group rotation entries are exact zeros); the group's chains advance
-//    together, column i of R (a row of the stored transpose) a wave-uniform
-//    operand read through the scalar cache;
+//    together, column i of R (a row of the stored transpose) one broadcast
+//    LDS read;
 //  * division and square root are IEEE (built with -ffp-contract=off and
 //    correctly rounded fp32 division/sqrt); a group's 32 divisions by its
 //    norm use its correctly rounded reciprocal and one FMA correction each,
@@ -63,10 +63,7 @@ struct Bulk {
   static constexpr int ROWS = WG;     // rows (threads) per workgroup
   static constexpr int SSTR = D + 2;  // staged halfs per row: odd dword stride
   static constexpr int STAGE = ROWS * SSTR * 2;
-  // d <= 64: the two diagonal rotation blocks in LDS (8 KB); at d=128 (32 KB)
-  // the columns are read through the scalar cache instead.
-  static constexpr bool ROT_LDS = D <= 64;
-  static constexpr int ROT = ROT_LDS ? 2 * (D / 2) * (D / 2) * 4 : 0;
+  static constexpr int ROT = 2 * (D / 2) * (D / 2) * 4;  // the two diagonal rotation blocks (8 KB)
   // The LUT and book areas are whole 256-byte pieces (the LDS DMA's unit).
   static constexpr int lut_area(int lut_bytes) { return (lut_bytes + 255) & ~255; }
   static constexpr int book_area(int book_floats) { return ((book_floats + 63) & ~63) * 4; }
@@ -175,15 +172,13 @@ __global__ __launch_bounds__(WG) void encode_bulk_kernel(const EncodeJobDev *__r
     const __amdgpu_buffer_rsrc_t rb = rsrc(tb + T->off_books, nbb);
     for (int c = wave; c * 256 < nbb; c += NW)
       dma4(rb, reinterpret_cast<uint8_t *>(books) + c * 256, c * 256 + lane * 4, 0);
-    if constexpr (Bulk<D, WG>::ROT_LDS) {
-      // Eight rows i of block g (GW = 32 floats each) per instruction:
-      // lane l brings Rt[(g GW + i0 + l / 8) D + g GW + 4 (l % 8) ...+3].
-      static_assert(GW == 32, "eight 128-byte block rows per 16-byte DMA");
-      const __amdgpu_buffer_rsrc_t rr = rsrc(tb + T->off_rot_t, D * D * 4);
-      for (int c = wave; c < NG * GW / 8; c += NW) {
-        const int g = c / (GW / 8), i = 8 * c - g * GW + lane / 8;
-        dma16(rr, reinterpret_cast<uint8_t *>(rot) + c * 1024, ((g * GW + i) * D + g * GW + 4 * (lane % 8)) * 4, 0);
-      }
+    // Eight rows i of block g (GW = 32 floats each) per instruction:
+    // lane l brings Rt[(g GW + i0 + l / 8) D + g GW + 4 (l % 8) ...+3].
+    static_assert(GW == 32, "eight 128-byte block rows per 16-byte DMA");
+    const __amdgpu_buffer_rsrc_t rr = rsrc(tb + T->off_rot_t, D * D * 4);
+    for (int c = wave; c < NG * GW / 8; c += NW) {
+      const int g = c / (GW / 8), i = 8 * c - g * GW + lane / 8;
+      dma16(rr, reinterpret_cast<uint8_t *>(rot) + c * 1024, ((g * GW + i) * D + g * GW + 4 * (lane % 8)) * 4, 0);
     }
   }
   if (vec) {
@@ -206,7 +201,6 @@ __global__ __launch_bounds__(WG) void encode_bulk_kernel(const EncodeJobDev *__r
   __syncthreads();
   if (tid >= nr) return;  // no barrier below
 
-  const BGTQ_CONST float *Rt = to_const<float>(reinterpret_cast<const uint8_t *>(job.t) + T->off_rot_t);  // Rt[i * D + j] = R[j][i]
   uint32_t packed[LOGICAL / 4];
 #pragma unroll
   for (int w = 0; w < LOGICAL / 4; ++w) packed[w] = 0u;
@@ -236,27 +230,21 @@ __global__ __launch_bounds__(WG) void encode_bulk_kernel(const EncodeJobDev *__r
     }
     // production_math.py:16: y_j = FMA chain over i ascending from +0 for
     // every output j of the group, the chains advanced together (input i
-    // outer: column i of the group's block one broadcast LDS read, or one
-    // scalar read at d=128), each in its own order.
+    // outer: column i of the group's block one broadcast LDS read), each in
+    // its own order.
     float y[GW];
 #pragma unroll
     for (int j = 0; j < GW; ++j) y[j] = 0.0f;
 #pragma unroll
     for (int i = 0; i < GW; ++i) {
-      if constexpr (Bulk<D, WG>::ROT_LDS) {
-        const float4 *Ci = reinterpret_cast<const float4 *>(rot + (g * GW + i) * GW);
+      const float4 *Ci = reinterpret_cast<const float4 *>(rot + (g * GW + i) * GW);
 #pragma unroll
-        for (int j4 = 0; j4 < GW / 4; ++j4) {
-          const float4 c = Ci[j4];
-          y[4 * j4 + 0] = __builtin_fmaf(x[i], c.x, y[4 * j4 + 0]);
-          y[4 * j4 + 1] = __builtin_fmaf(x[i], c.y, y[4 * j4 + 1]);
-          y[4 * j4 + 2] = __builtin_fmaf(x[i], c.z, y[4 * j4 + 2]);
-          y[4 * j4 + 3] = __builtin_fmaf(x[i], c.w, y[4 * j4 + 3]);
-        }
-      } else {
-        const BGTQ_CONST float *Ci = Rt + (P0 + i) * D + P0;
-#pragma unroll
-        for (int j = 0; j < GW; ++j) y[j] = __builtin_fmaf(x[i], Ci[j], y[j]);
+      for (int j4 = 0; j4 < GW / 4; ++j4) {
+        const float4 c = Ci[j4];
+        y[4 * j4 + 0] = __builtin_fmaf(x[i], c.x, y[4 * j4 + 0]);
+        y[4 * j4 + 1] = __builtin_fmaf(x[i], c.y, y[4 * j4 + 1]);
+        y[4 * j4 + 2] = __builtin_fmaf(x[i], c.z, y[4 * j4 + 2]);
+        y[4 * j4 + 3] = __builtin_fmaf(x[i], c.w, y[4 * j4 + 3]);
       }
     }
     // production_math.py:17-23: output j's bin, LUT code and centroid are
@@ -291,46 +279,35 @@ __global__ __launch_bounds__(WG) void encode_bulk_kernel(const EncodeJobDev *__r
   for (int g = NG; g < NSTR; ++g) nrow[g] = 0;
 }
 
-template <int D, int NG, int NS, int WG>
-hipError_t launch_kind(const EncodeJobDev *jobs, int n_jobs, int src_f32, int64_t max_rows, int lut_area,
-                       int book_floats, hipStream_t stream) {
-  const int lds = Bulk<D, WG>::STAGE + lut_area + Bulk<D, WG>::book_area(book_floats) + Bulk<D, WG>::ROT;
-  dim3 grid((unsigned)((max_rows + WG - 1) / WG), (unsigned)n_jobs);
-  if (src_f32)
-    hipLaunchKernelGGL((encode_bulk_kernel<D, NG, NS, true, WG>), grid, dim3(WG), lds, stream, jobs, lut_area,
-                       book_floats);
-  else
-    hipLaunchKernelGGL((encode_bulk_kernel<D, NG, NS, false, WG>), grid, dim3(WG), lds, stream, jobs, lut_area,
-                       book_floats);
-  return hipGetLastError();
-}
+// Layout B at d=64: two groups, 32 nibble dimensions; 256 rows per workgroup.
+constexpr int kDim = 64, kWg = 256;
 
 }  // namespace
 
 int encode_bulk_kind(const DevTables *T) {
   const int d = T->dim, ng = T->groups;
-  if ((d != 64 && d != 128) || ng != 2 || T->nibble_dims != d / 2) return 0;
+  if (d != kDim || ng != 2 || T->nibble_dims != d / 2) return 0;
   if (T->gstart[0] != 0 || T->gend[0] != d / 2 || T->gstart[1] != d / 2 || T->gend[1] != d) return 0;
   if (T->row_bytes % 4 || T->row_bytes < d / 4 + d / 2) return 0;
-  return d == 64 ? 1 : 2;
+  return 1;
 }
 
-int encode_bulk_lds_bytes(int kind, int wg, int lut_bytes, int book_floats) {
-  const int d = kind == 1 ? 64 : 128;
-  return wg * (d + 2) * 2 + Bulk<64, 256>::lut_area(lut_bytes) + Bulk<64, 256>::book_area(book_floats) +
-         (d <= 64 ? 2 * (d / 2) * (d / 2) * 4 : 0);
+int encode_bulk_lds_bytes(int lut_bytes, int book_floats) {
+  using B = Bulk<kDim, kWg>;
+  return B::STAGE + B::lut_area(lut_bytes) + B::book_area(book_floats) + B::ROT;
 }
 
-hipError_t launch_encode_bulk(const EncodeJobDev *jobs, int n_jobs, int kind, int wg, int src_f32, int64_t max_rows,
-                              int lut_bytes, int book_floats, hipStream_t stream) {
-  const int lut_area = Bulk<64, 256>::lut_area(lut_bytes);
-#define BGTQ_BULK(K, DD, NS, W)                                                                           \
-  if (kind == K && wg == W)                                                                               \
-    return launch_kind<DD, 2, NS, W>(jobs, n_jobs, src_f32, max_rows, lut_area, book_floats, stream);
-  BGTQ_BULK(1, 64, 32, 256)
-  BGTQ_BULK(2, 128, 64, 128)
-#undef BGTQ_BULK
-  return hipErrorInvalidValue;
+hipError_t launch_encode_bulk(const EncodeJobDev *jobs, int n_jobs, int src_f32, int64_t max_rows, int lut_bytes,
+                              int book_floats, hipStream_t stream) {
+  const int lut_area = Bulk<kDim, kWg>::lut_area(lut_bytes), lds = encode_bulk_lds_bytes(lut_bytes, book_floats);
+  const dim3 grid((unsigned)((max_rows + kWg - 1) / kWg), (unsigned)n_jobs);
+  if (src_f32)
+    hipLaunchKernelGGL((encode_bulk_kernel<kDim, 2, kDim / 2, true, kWg>), grid, dim3(kWg), lds, stream, jobs, lut_area,
+                       book_floats);
+  else
+    hipLaunchKernelGGL((encode_bulk_kernel<kDim, 2, kDim / 2, false, kWg>), grid, dim3(kWg), lds, stream, jobs,
+                       lut_area, book_floats);
+  return hipGetLastError();
 }
 
 }  // namespace bgtq

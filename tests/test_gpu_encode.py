@@ -277,6 +277,79 @@ def test_bulk_encoder_unaligned_source(device, oracle):
         tables.destroy()
 
 
+@pytest.mark.parametrize("src_kind", ["f16", "f32"])
+@pytest.mark.parametrize("dim,layouts", [(64, ("B", "A", "mixed_d64", "smollm2_h0", "smollm2_h17", "smollm2_h89")),
+                                         (128, ("B", "A", "mixed_d128", "low_d128"))])
+def test_tile_encoder_bit_exact(device, oracle, dim, layouts, src_kind):
+    """One launch of jobs above the wave encoder's row limit takes the tile encoder (16 rows per wave):
+    layouts of one to six groups, row counts around whole tiles, jobs with and without rows, interleaved
+    heads, unaligned sources with odd strides, destinations at odd bytes with guard rows on both sides."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    rng = np.random.default_rng(77 + dim)
+    known = dict(_layouts(oracle), B=calibrate.layout_b(dim), A=calibrate.layout_a(dim))
+    print("tile encoder", dim, src_kind, flush=True)
+    jobs, checks, tabs = [], [], []
+    try:
+        for i, name in enumerate(layouts):
+            p = known[name]
+            tabs.append(bgtq.Tables(device, p))
+            for j, rows in enumerate((1, 15, 16, 17, 63, 1039, 3001) if i else (0, 5, 32, 4100)):
+                stride = dim + (0, 8, 1)[j % 3]
+                lead = (j % 2) * (1 if src_kind == "f32" else 3)  # elements before the first row
+                row0, guard = (3, 0, 1, 2)[j % 4], 2
+                k = _random_half_rows(rng, rows, dim)
+                flat = np.zeros(lead + max(1, rows) * stride, dtype=np.float16)
+                flat[lead:].reshape(-1, stride)[:rows, :dim] = k.view(np.float16)
+                src = torch.from_numpy(flat if src_kind == "f16" else flat.astype(np.float32)).cuda()
+                packed = torch.full((row0 + rows + guard, p.rowBytes), 0xA5, dtype=torch.uint8, device="cuda")
+                norms = torch.full((row0 + rows + guard, p.normStride), 0x5A5A, dtype=torch.int16, device="cuda")
+                jobs.append(dict(tables=tabs[-1], src=src[lead:], src_row_stride=stride, rows=rows, packed=packed,
+                                 norms=norms, dst_row0=row0))
+                checks.append((name, p, rows, row0, k, packed, norms))
+        batched.encode(device, jobs, src_kind)
+        device.synchronize()
+        for name, p, rows, row0, k, packed, norms in checks:
+            got_p, got_n = packed.cpu().numpy(), norms.cpu().numpy().view(np.uint16)
+            outside = np.r_[0:row0, row0 + rows:len(got_p)]
+            assert np.all(got_p[outside] == 0xA5) and np.all(got_n[outside] == 0x5A5A), f"{name} {rows}: guard rows"
+            if rows:
+                ref_p, ref_n = oracle.encode_pack(_olayout(oracle, p), np.ascontiguousarray(k))
+                bad = np.nonzero(np.any(got_p[row0:row0 + rows] != ref_p, axis=1)
+                                 | np.any(got_n[row0:row0 + rows] != ref_n, axis=1))[0]
+                assert bad.size == 0, f"{name} {rows} rows: {bad.size} differ, first {bad[:5]}"
+    finally:
+        for t in tabs:
+            t.destroy()
+
+
+def test_bulk_layout_b_largest_calls(device, oracle):
+    """Layout B at d=64 from 300,000 rows a call: the thread-per-row encoder with the layout's structure
+    compiled in, FP16 and FP32 sources, a partial last workgroup."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    rng = np.random.default_rng(5)
+    p, rows = calibrate.layout_b(64), 300077
+    k = _random_half_rows(rng, rows, 64)
+    ref_p, ref_n = oracle.encode_pack(_olayout(oracle, p), k)
+    tables = bgtq.Tables(device, p)
+    try:
+        for src_kind in ("f16", "f32"):
+            src = torch.from_numpy(k.view(np.float16) if src_kind == "f16" else
+                                   k.view(np.float16).astype(np.float32)).cuda()
+            packed = torch.zeros((rows, p.rowBytes), dtype=torch.uint8, device="cuda")
+            norms = torch.zeros((rows, p.normStride), dtype=torch.int16, device="cuda")
+            batched.encode(device, [dict(tables=tables, src=src, src_row_stride=64, rows=rows, packed=packed,
+                                         norms=norms)], src_kind)
+            device.synchronize()
+            assert np.array_equal(packed.cpu().numpy(), ref_p), src_kind
+            assert np.array_equal(norms.cpu().numpy().view(np.uint16), ref_n), src_kind
+    finally:
+        tables.destroy()
+
+
 def test_calibration_load_encodes_every_head(device, oracle):
     """Calibration.load (src/model/calibration.ts:7-21) puts the 90 SmolLM2 heads on the device;
     each head's tables then encode its KV head's post-RoPE rows bit for bit as the oracle does
