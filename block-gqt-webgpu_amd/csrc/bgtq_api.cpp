@@ -76,21 +76,7 @@ uint16_t f32_to_f16(float x) {
   return (uint16_t)(sign | ((he > 0 ? (uint32_t)he << 10 : 0u) + base + inc));
 }
 
-// FP32 -> FP16 bits rounded toward zero (subnormals kept, overflow to the
-// largest finite value), and FP16 bits -> FP32.
-uint16_t f32_to_f16_rtz(float x) {
-  uint32_t b;
-  std::memcpy(&b, &x, 4);
-  const uint32_t sign = (b >> 16) & 0x8000u, e = (b >> 23) & 0xffu, m = b & 0x7fffffu;
-  const int32_t he = (int32_t)e - 112;
-  if (e == 0xffu) return (uint16_t)(sign | 0x7c00u | (m ? 0x200u : 0u));
-  if (he >= 31) return (uint16_t)(sign | 0x7bffu);
-  if (he <= 0) {
-    if (he < -10) return (uint16_t)sign;
-    return (uint16_t)(sign | ((m | 0x800000u) >> (14 - he)));
-  }
-  return (uint16_t)(sign | ((uint32_t)he << 10) | (m >> 13));
-}
+// FP16 bits -> FP32.
 float f16_to_f32(uint16_t h) {
   const uint32_t sign = ((uint32_t)h & 0x8000u) << 16, e = (h >> 10) & 31u, m = h & 1023u;
   float v;
@@ -200,10 +186,6 @@ struct bgtq_values {
   uint32_t dim = 0, capacity = 0, length = 0;
   int32_t dtype = BGTQ_DTYPE_F32;
   DeviceBuffer buf;
-  // FP32 V: every appended |v| < 65504, so the fused kernel can split each
-  // value into FP16 parts; a larger value sends the store to the general
-  // kernels.
-  bool fp16_range = true;
   Ledger ledger;
 };
 
@@ -555,7 +537,8 @@ bgtq_status bgtq_tables_create(bgtq_context *ctx, const uint32_t *integer, size_
   float *rot_t = reinterpret_cast<float *>(h + off_rot_t);
   for (int64_t j = 0; j < d; ++j)
     for (int64_t i = 0; i < d; ++i) rot_t[i * d + j] = rot[j * d + i];
-  // MFMA lookup tables: c * 2^cent_exp = hi + lo, hi and lo fp16 rounded toward zero.
+  // MFMA lookup tables: c * 2^cent_exp = hi + lo, both fp16 rounded to nearest
+  // (within 2^-22; rounding toward zero left up to 2^-20).
   const float csc = std::ldexp(1.0f, T->cent_exp);
   for (int b = 0; b < nb; ++b) {
     const float *c = cent + book_rows[b] * mc;
@@ -564,8 +547,8 @@ bgtq_status bgtq_tables_create(bgtq_context *ctx, const uint32_t *integer, size_
     uint32_t *code = reinterpret_cast<uint32_t *>(tb + 2048);  // [256] hi | lo << 16
     auto split = [&](int e, uint16_t *hi, uint16_t *lo) {
       const float x = e < mc ? c[e] * csc : 0.0f;
-      *hi = f32_to_f16_rtz(x);
-      *lo = f32_to_f16_rtz(x - f16_to_f32(*hi));
+      *hi = f32_to_f16(x);
+      *lo = f32_to_f16(x - f16_to_f32(*hi));
     };
     for (int e = 0; e < 256; ++e) {
       uint16_t h0, l0, h1, l1;
@@ -591,8 +574,8 @@ bgtq_status bgtq_tables_create(bgtq_context *ctx, const uint32_t *integer, size_
           uint16_t *dst = op + ((n * (d / 32) + s) * 64 + l) * 16;
           for (int jv = 0; jv < 8; ++jv) {
             const float x = rq[(16 * n + l % 16) * d + 32 * s + 8 * (l / 16) + jv];
-            dst[jv] = f32_to_f16_rtz(x);
-            dst[8 + jv] = f32_to_f16_rtz(x - f16_to_f32(dst[jv]));
+            dst[jv] = f32_to_f16(x);
+            dst[8 + jv] = f32_to_f16(x - f16_to_f32(dst[jv]));
           }
         }
   }
@@ -842,8 +825,6 @@ bgtq_status bgtq_values_append(bgtq_values *v, const float *values, size_t n) {
     HIP_TRY(hipMemcpy(static_cast<float *>(v->buf.ptr) + (size_t)v->length * v->dim, values, n * 4,
                       hipMemcpyHostToDevice),
             "V upload");
-    for (size_t i = 0; i < n; ++i)
-      if (std::fabs(values[i]) >= 65504.0f) v->fp16_range = false;
   } else {
     std::vector<uint16_t> h(n);
     for (size_t i = 0; i < n; ++i) h[i] = f32_to_f16(values[i]);
@@ -1087,12 +1068,11 @@ bgtq_status bgtq_decode_workspace_size(const bgtq_decode_desc *d, size_t *bytes)
   return BGTQ_OK;
 }
 
-// Whether the fused kernel reads p's V: FP16 rows, or FP32 rows known to
-// lie within FP16's range in a decode without an appended token; 16-byte
-// aligned base and strides.
+// Whether the fused kernel reads p's V: FP16 rows, or FP32 rows in a decode
+// without an appended token; 16-byte aligned base and strides.
 static bool fused_v(const DecodeParams &p) {
   const bool f32 = p.v_dtype == BGTQ_DTYPE_F32;
-  if (f32 ? !p.v_f32_split || p.k_new || p.starts : p.v_dtype != BGTQ_DTYPE_F16) return false;
+  if (f32 ? p.k_new || p.starts : p.v_dtype != BGTQ_DTYPE_F16) return false;
   const int64_t vb = f32 ? 4 : 2;
   return (reinterpret_cast<uintptr_t>(p.v) & 15) == 0 && (p.v_seq_stride * vb) % 16 == 0 &&
          (p.v_head_stride * vb) % 16 == 0;
@@ -1736,7 +1716,6 @@ static bgtq_status attention_record(bgtq_attention *a, bgtq_timestamps *ts, uint
   }
   p.v = v->buf.ptr;
   p.v_dtype = v->dtype;
-  p.v_f32_split = v->dtype == BGTQ_DTYPE_F32 && v->fp16_range;
   p.qr = static_cast<float *>(a->qr.ptr);
   p.lengths = static_cast<const uint32_t *>(a->small.ptr);
   p.max_length = (int32_t)T;

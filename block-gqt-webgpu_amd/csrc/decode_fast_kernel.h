@@ -334,7 +334,7 @@ __device__ __forceinline__ void merge_rows(float *part, float *out, const MergeR
 // only as many of its splits as its history needs (p.split_floor tokens per
 // split at least); the others exit before their first chunk.
 // VF: V rows of FP32 values (1; decode without an appended token) or FP16
-// (0). FP32 V enters the PV MFMAs as three FP16 parts per value.
+// (0). FP32 V takes its PV products on the FP32 matrix cores.
 // NW: waves per workgroup (4; row-wise prefill at d=64, 8: a unit's splits
 // then cover twice the tokens each and half as many partials are merged).
 // Every kernel argument the set-up reads, loaded at once (one asm statement,
@@ -372,6 +372,8 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   static_assert(KF == 0 || row_enc::scratch_bytes(D) <= Sl::BYTES, "append scratch fits a ring slot");
   constexpr int KS = Gm::KS, DT = Gm::DT, PR = Gm::PR, VI = Sl::VI, KRI = Gm::KRI;
   constexpr int VB = VF ? 4 : 2;  // bytes per V value
+  // P is carried times 2^15 where it is split into FP16 parts; unscaled for FP32 V.
+  constexpr float kPShift = VF ? 0.0f : 15.0f, kPFactor = VF ? 1.0f : kPScale;
   constexpr int RB = Sl::RB, KI = Sl::KI, L = Sl::L, AHEAD = Sl::AHEAD;
   static_assert(NN >= 0 && NN <= KS && SG >= 1 && SG <= KS, "layout");
   static_assert(Sl::BYTES >= 16 * (D + 4) * 4, "q staging fits one ring slot");
@@ -1377,42 +1379,30 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       }
     }
   };
-  // PV of the chunk in ring slot sb: O += P V, P split into fp16 hi (pha) and
-  // lo (pla) parts in A-operand order.
-  auto chunk_pv = [&](const uint8_t *sb, const half8 pha, const half8 pla) {
+  // PV of the chunk in ring slot sb: O += P V. FP16 V: P split into fp16 hi
+  // (pha) and lo (pla) parts in A-operand order. FP32 V: the probabilities
+  // pr themselves, on the FP32 matrix cores.
+  auto chunk_pv = [&](const uint8_t *sb, const half8 pha, const half8 pla, const float *pr) {
     if constexpr (VF) {
-      // FP32 V: lane (gq, col) reads V[16 (j >> 2) + 4 gq + (j & 3)][16 dt + col],
-      // the B operand of its P slots j = 0..7 (row reads; the four lane groups
-      // hit different banks through swz32), and splits each value into FP16
-      // parts v = h0 + 2^-11 h1 + 2^-22 h2: each part holds the next 11 bits
-      // of what the ones before left, so the parts are exact for
-      // 2^-23 <= |v| < 65504 (the host keeps larger V off this path). The
-      // MFMAs weight h1 and h2 with P's hi part scaled by 2^-11 and 2^-22
-      // (exact powers of two; P lo times those terms is below 2^-22 of the
-      // result and left out).
-      const half8 ph1 = pha * (_Float16)0x1p-11f, ph2 = pha * (_Float16)0x1p-22f;
-      // Row 4 gq + (j & 3) + 16 (j >> 2), its piece 4 (dt ^ gq) + col / 4.
+      // Lane (gq, col) reads V[16 (j >> 2) + 4 gq + (j & 3)][16 dt + col], the
+      // B operand of its probability j = 0..7 (row reads; the four lane
+      // groups hit different banks through swz32). The 16x16x4 FP32 product
+      // takes P and V as they are, so it serves any FP32 value and spends no
+      // vector instructions on splitting (each value into three FP16 parts
+      // served |V| < 65504 only, and batched calls, whose values the library
+      // does not see, took the general kernels: 8 sequences x 14 heads x 4096
+      // tokens 65 us against 17.7).
       const uint8_t *vl = sb + 16 * gq * D + 4 * col;
+      float v[8][DT];
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const uint8_t *vd = vl + 64 * (dt ^ gq);
-        half8 h0, h1, h2;
+      for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float v = *reinterpret_cast<const float *>(vd + (16 * (j >> 2) + (j & 3)) * (4 * D));
-          const _Float16 a = (_Float16)v;
-          const float r1 = v - (float)a;
-          const _Float16 c = (_Float16)(r1 * 0x1p11f);
-          const float r2 = __builtin_fmaf(-(float)c, 0x1p-11f, r1);
-          h0[j] = a;
-          h1[j] = c;
-          h2[j] = (_Float16)(r2 * 0x1p22f);
-        }
-        O[dt] = mfma(pha, h0, O[dt]);
-        O[dt] = mfma(pla, h0, O[dt]);
-        O[dt] = mfma(ph1, h1, O[dt]);
-        O[dt] = mfma(ph2, h2, O[dt]);
-      }
+        for (int dt = 0; dt < DT; ++dt)
+          v[j][dt] = *reinterpret_cast<const float *>(vl + 64 * (dt ^ gq) + (16 * (j >> 2) + (j & 3)) * (4 * D));
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) O[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[j], v[j][dt], O[dt], 0, 0, 0);
     } else {
       u32x2 vt[DT][2];
 #pragma unroll
@@ -1491,8 +1481,8 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
           for (int dt = 0; dt < DT; ++dt) O[dt][r] *= ar;
         }
       }
-      chunk_pv(slot_base(0), __builtin_bit_cast(half8, ph[0]), __builtin_bit_cast(half8, pl[0]));
-      if (!app_wg) chunk_pv(slot_base(1), __builtin_bit_cast(half8, ph[1]), __builtin_bit_cast(half8, pl[1]));
+      chunk_pv(slot_base(0), __builtin_bit_cast(half8, ph[0]), __builtin_bit_cast(half8, pl[0]), nullptr);
+      if (!app_wg) chunk_pv(slot_base(1), __builtin_bit_cast(half8, ph[1]), __builtin_bit_cast(half8, pl[1]), nullptr);
     }
   } else {
     for (int i = 0; i < n_chunks; ++i) {
@@ -1533,7 +1523,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       float mloc = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
       const float m_new = fmaxf(m_run, col_max(mloc));
       const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-      const float mb = (m_new == -INFINITY ? 0.0f : m_new) - 15.0f;
+      const float mb = (m_new == -INFINITY ? 0.0f : m_new) - kPShift;
       float pr[8], psum = 0.0f;
   #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -1542,9 +1532,9 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       }
       l_run = __builtin_fmaf(l_run, alpha, psum);
       m_run = m_new;
-      u32x4 ph, pl;
+      u32x4 ph{}, pl{};
   #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < (VF ? 0 : 4); ++k) {
         uint32_t h, l;
         split2(pr[2 * k], pr[2 * k + 1], h, l);
         ph[k] = h;
@@ -1571,12 +1561,12 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       // computed is waited for (at the top of the iteration).
       if (!PF) wait_vm<0>();
       const half8 pha = __builtin_bit_cast(half8, ph), pla = __builtin_bit_cast(half8, pl);
-      chunk_pv(sb, pha, pla);
+      chunk_pv(sb, pha, pla, pr);
     }
   }
 
   // ---------------- epilogue ----------------
-  const float l_tot = col_sum(l_run) * (1.0f / kPScale);
+  const float l_tot = col_sum(l_run) * (1.0f / kPFactor);
   wait_vm<0>();     // a wave without chunks still has its prologue's zero-sized chunk loads to retire
   __syncthreads();  // every wave is done with the ring
   float *comb = reinterpret_cast<float *>(smem);  // [wave][16 heads][2 + D]
@@ -1588,7 +1578,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      comb[(wave * 16 + 4 * gq + r) * (D + 2) + 2 + 16 * dt + col] = O[dt][r] * (1.0f / kPScale);
+      comb[(wave * 16 + 4 * gq + r) * (D + 2) + 2 + 16 * dt + col] = O[dt][r] * (1.0f / kPFactor);
   __syncthreads();
   if constexpr (!PF) {
     // Decode: the waves' states of each of the G heads merged by log-sum-exp,

@@ -142,9 +142,8 @@ void bgtq_keys_destroy(bgtq_keys *k);
 /* ---- Values (src/runtime/values.ts:3-16) --------------------------------- *
  * dtype BGTQ_DTYPE_F32 stores FP32 V exactly (the synthetic path); F16 stores
  * RNE-rounded FP16 V (src/model/append.wgsl:6-10). append() is synchronous.
- * Attention over F32 V runs on the fused kernel, which splits each value into
- * three FP16 parts that add back to it exactly, while every appended
- * |v| < 65504; a larger value sends the store to the general kernels. */
+ * Attention over F32 V runs on the fused kernel, its PV products on the FP32
+ * matrix cores. */
 typedef struct bgtq_values bgtq_values;
 bgtq_status bgtq_values_create(bgtq_context *ctx, uint32_t dim, uint32_t capacity, int32_t dtype,
                                bgtq_values **out);

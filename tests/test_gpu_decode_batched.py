@@ -341,3 +341,71 @@ def test_batch_beyond_grid_refused(device):
                 v_seq_stride=0, v_head_stride=0, k_f16=z, k_seq_stride=0, k_head_stride=0, splits=1)
     with pytest.raises(bgtq.UnsupportedError, match="65535 sequences"):
         batched.workspace_bytes(batched.decode_desc(**args))
+
+
+@pytest.mark.parametrize("key_format,layout,dim,hq,hkv,lengths", [
+    ("packed", "B", 64, 14, 2, [1, 31, 33, 1000]), ("packed", "A", 64, 3, 1, [700, 129]),
+    ("packed", "B", 128, 16, 4, [257, 64]), ("packed", "A", 128, 2, 2, [1, 500]),
+    ("fp16", None, 64, 5, 1, [127, 128, 300]), ("fp16", None, 128, 8, 8, [65]),
+])
+def test_fp32_values_batched(device, oracle, key_format, layout, dim, hq, hkv, lengths):
+    """bgtq_decode over FP32 V (its PV products on the FP32 matrix cores): values of ordinary size and, in
+    one dimension, near the largest FP32, whose products with the probabilities must not overflow on the
+    way. The rows past a sequence's length are NaN (never read into the result)."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    batched.bind_torch_stream(device)
+    print("fp32 V batched", key_format, layout, dim, lengths, flush=True)
+    g = torch.Generator().manual_seed(3)
+    B, cap, G = len(lengths), max(lengths) + 9, hq // hkv
+    k = (torch.randn((B, hkv, cap, dim), generator=g) * 0.8).half()
+    v = torch.randn((B, hkv, cap, dim), generator=g)
+    v[..., 5] *= 2.0e37
+    q = torch.randn((B, hq, dim), generator=g)
+    for b, n in enumerate(lengths):
+        v[b, :, n:] = float("nan")
+    kd, vd, qd = k.cuda(), v.cuda(), q.cuda()
+    lens = torch.tensor(lengths, dtype=torch.int32).cuda()
+    out = torch.empty((B, hq, dim), device="cuda")
+    tabs = []
+    if key_format == "packed":
+        p = calibrate.layout_b(dim) if layout == "B" else calibrate.layout_a(dim)
+        tabs = [bgtq.Tables(device, p) for _ in range(hkv)]
+        packed = torch.zeros((B, hkv, (cap * p.rowBytes + 79) // 16 * 16), dtype=torch.uint8, device="cuda")
+        norms = torch.zeros((B, hkv, (cap * p.normStride + 39) // 8 * 8), dtype=torch.int16, device="cuda")
+        batched.encode(device, [dict(tables=tabs[h], src=kd[b, h], src_row_stride=dim, rows=cap, packed=packed[b, h],
+                                     norms=norms[b, h]) for b in range(B) for h in range(hkv)], "f16")
+        kw = dict(tables=tabs, packed=packed, packed_seq_stride=packed.stride(0), packed_head_stride=packed.stride(1),
+                  norms=norms, norms_seq_stride=norms.stride(0), norms_head_stride=norms.stride(1))
+    else:
+        kw = dict(k_f16=kd, k_seq_stride=kd.stride(0), k_head_stride=kd.stride(1))
+    args = dict(batch=B, q_heads=hq, kv_heads=hkv, dim=dim, q=qd, out=out, lengths=lens, max_length=max(lengths), v=vd,
+                v_dtype="f32", v_seq_stride=vd.stride(0), v_head_stride=vd.stride(1), **kw)
+    try:
+        for splits in (0, 1, 3):
+            ws = torch.zeros(batched.workspace_bytes(batched.decode_desc(splits=splits, **args)), dtype=torch.uint8,
+                             device="cuda")
+            out.fill_(float("nan"))
+            batched.decode(device, batched.decode_desc(splits=splits, workspace=ws, **args))
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()
+            for b, T in enumerate(lengths):
+                for h in range(hkv):
+                    if key_format == "packed":
+                        pk = packed[b, h, :T * p.rowBytes].cpu().numpy().reshape(T, p.rowBytes)
+                        nm = norms[b, h, :T * p.normStride].cpu().numpy().view(np.float16).reshape(T, p.normStride)
+                        keff = oracle.reconstruct(_olayout(oracle, p), oracle.unpack(pk, dim, p.nibbleDims),
+                                                  nm.astype(np.float32))
+                    else:
+                        keff = k[b, h, :T].float().numpy()
+                    vv = v[b, h, :T].numpy()
+                    _, _, ref = oracle.attention(q[b, h * G:(h + 1) * G].numpy(), keff, vv, np.full(G, T - 1), False)
+                    # The usual bar in units of each dimension's largest value (the sums' terms).
+                    err = np.abs(got[b, h * G:(h + 1) * G].astype(np.float64) - ref)
+                    big = np.maximum(1.0, np.abs(vv.astype(np.float64)).max(0))
+                    lim = ATOL * big + RTOL * np.abs(ref.astype(np.float64))
+                    assert np.all(err <= lim), f"splits {splits} b{b} kv{h}: worst ratio {(err / lim).max():.2f}"
+    finally:
+        for t in tabs:
+            t.destroy()
