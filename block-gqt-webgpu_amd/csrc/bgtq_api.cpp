@@ -1331,6 +1331,8 @@ struct PrefillPlan {
   int tiles, tile_queries, ranges, range_blocks;
   size_t records;    // bytes of the workgroups' partial records
   size_t workspace;  // records, then the tile table (16 bytes per tile)
+  size_t operands;   // bytes of the built K operands and their exponents after those, 0 = built per tile
+  int operand_blocks;
   bool rowwise;      // the fused decode kernel, units of 16 (row, head) query columns
   int qgroups;       // rowwise: units per (sequence, KV head)
   int unit_cols;     // rowwise: query columns per unit
@@ -1438,6 +1440,16 @@ static bgtq_status plan_prefill(const bgtq_prefill_desc *d, PrefillPlan *plan, b
   plan->records = plan->ranges > 1 ? sizeof(float) * (size_t)plan->ranges * 2 * tq * (d->dim + 2) : 0;
   const size_t info = plan->ranges > 1 ? 16 * (size_t)d->batch * d->kv_heads * plan->tiles : 0;
   plan->workspace = kPrefillCounterBytes + plan->records + info;
+  if (d->key_format == BGTQ_KEYS_PACKED && plan->tiles > 1 &&
+      prefill_operands_once(d->dim, false, nq)) {
+    plan->operand_blocks = (int)(((int64_t)d->max_length + 31) / 32);
+    const size_t blocks = (size_t)d->batch * d->kv_heads * plan->operand_blocks;
+    const size_t bytes = blocks * 32 * 4 * d->dim + (blocks * 4 + 15) / 16 * 16;
+    if (bytes <= kPrefillOperandBytes) {
+      plan->workspace = (plan->workspace + 15) / 16 * 16;
+      plan->operands = bytes;
+    }
+  }
   return BGTQ_OK;
 }
 
@@ -1445,7 +1457,7 @@ bgtq_status bgtq_prefill_workspace_size(const bgtq_prefill_desc *d, size_t *byte
   PrefillPlan plan{};
   if (bgtq_status s = plan_prefill(d, &plan)) return s;
   if (!bytes) return fail(BGTQ_ERR_RANGE, "null output");
-  *bytes = std::max<size_t>(plan.workspace, 256);
+  *bytes = std::max<size_t>(plan.workspace + plan.operands, 256);
   return BGTQ_OK;
 }
 
@@ -1593,6 +1605,19 @@ static bgtq_status prefill_impl(bgtq_context *ctx, const bgtq_prefill_desc *d, c
   p.part = reinterpret_cast<float *>(static_cast<uint8_t *>(d->workspace) + kPrefillCounterBytes);
   p.tile_info = reinterpret_cast<int32_t *>(static_cast<uint8_t *>(d->workspace) + kPrefillCounterBytes + plan.records);
   p.out = d->out;
+  // A workspace of the partials alone leaves the operands to each tile's own
+  // build, as do books beyond the build's LDS.
+  bool once = prefill_operands_once(d->dim, nn >= 0, (int64_t)d->rows * dp.G);
+  for (int h = 0; h < d->kv_heads && d->key_format == BGTQ_KEYS_PACKED; ++h) {
+    const DevTables *T = d->tables[h]->h();
+    if (T->n_books * T->max_centroids * 4 > prefill_general_book_bytes(d->dim)) once = false;
+  }
+  if (plan.operands && d->workspace_bytes >= plan.workspace + plan.operands && once) {
+    p.operand_blocks = plan.operand_blocks;
+    p.operands = static_cast<uint8_t *>(d->workspace) + plan.workspace;
+    p.operand_exp = reinterpret_cast<int32_t *>(
+        p.operands + (size_t)d->batch * d->kv_heads * plan.operand_blocks * 32 * 4 * d->dim);
+  }
   HIP_TRY(launch_prefill(p, fl, nn, sg, ctx->stream), "prefill launch");
   return BGTQ_OK;
 }

@@ -231,12 +231,27 @@ struct PrefillParams {
   int32_t first_round;      // > 0: the first first_round ranges are 1.5 times the others
   float *part;              // two records per workgroup: (m, l, o[dim]) per query of a tile
   int32_t *tile_info;       // per (KV head, sequence, tile): first and last workgroup, first one's record
+  uint8_t *operands;        // built K operands, [B][kv_heads][operand_blocks][32 tokens x 4 dim bytes]; null: built per tile
+  int32_t *operand_exp;     // their scale exponents, [B][kv_heads][operand_blocks]
+  int32_t operand_blocks;   // 32-token blocks of max_length
   float *out;               // [B*rows*Hq*dim]
 };
 // Most 16-query MFMA column blocks per wave of the prefill kernel (four waves per tile).
 __host__ __device__ constexpr int prefill_column_blocks(int dim) { return dim == 64 ? 4 : 2; }
 constexpr int kPrefillMinRange = 2;       // cost units per workgroup range the kernel picks at least
 constexpr int kPrefillSegmentCost = 4;    // cost units of a tile's set-up (a 32-token block is one)
+// A tiled chunk's K operands built once (prefill_operand_kernel, about 5 us) instead of by every query tile.
+// us per call, once / per tile (MI355X, same outputs bit for bit):
+//   any packed layout, d=128: 33 rows x 4 heads after 2000 tokens 26.5 / 29.2, 1001 rows x 4 after 3077 77 / 343: always;
+//   any packed layout, d=64: from the 256-query tiles on (1001 rows x 3 after 3077: 54.8 / 81.2; 300 rows x 7 after
+//   300: 27.2 / 24.6 structured); with 64-query tiles the build launch costs what it saves (771 queries 30.7 / 31.4,
+//   900 after 300 tokens 21.8 / 19.6);
+//   structured layouts build cheaply per tile: d=128 2100 queries 37.9 / 36.5, 4200 73.2 / 76.8, 14336 79.1 / 87.6;
+//   d=64 28672 queries 109.4 / 110.1, 2100 27.2 / 24.6: never.
+__host__ __device__ constexpr bool prefill_operands_once(int dim, bool structured, int64_t queries) {
+  return dim == 128 ? !structured || queries >= 4096 : !structured && queries >= 2048;
+}
+constexpr size_t kPrefillOperandBytes = (size_t)1 << 30;  // workspace bytes of built operands at most
 constexpr int kPrefillMaxRanges = 2048;   // workgroups of one launch at most (bounds the records)
 // Chunks of at most this many rows run row-wise through the fused decode
 // kernel (a unit per query row and KV head, its split merge); longer chunks

@@ -68,31 +68,35 @@ constexpr float kPOut = 1 << (15 - kTauLog2);
 // buffers of built K operands. The ring is as deep as lets two workgroups
 // share a compute unit. KF 2 (any packed layout): K rows of up to D bytes,
 // up to 8 scales per token, every book (n_books x max_centroids floats).
+// KF 3: the block's K operand as prefill_operand_kernel left it, 4 * D bytes a
+// token; no books, operand buffers or scales.
 template <int D, int KF, int NN>
 struct PSlot {
   static constexpr int KS = D / 32, DT = D / 16, PR = D / 8;
   static constexpr int VBYTES = kChunk * D * 2;
   static constexpr int VI = VBYTES / 1024;  // 16-byte DMA instructions per V block
   static constexpr int VW = VI / kWaves;    // ... per wave
-  static constexpr int RB = KF == 1 ? NN * 16 + (KS - NN) * 32 : KF == 2 ? D : 2 * D;  // K row bytes
+  static constexpr int RB = KF == 1 ? NN * 16 + (KS - NN) * 32 : KF == 2 ? D : KF == 3 ? 4 * D : 2 * D;  // K row bytes
   static constexpr int KBYTES = kChunk * RB;
   // Packed K and its scales move as 4-byte DMAs with every lane of every wave
   // busy (no lane-masked instructions, so the compiler's waits for register
   // loads issued before the ring stay exact): the K block padded to a
   // multiple of 1 KB, the scales to 1 KB (past the block's tokens the range
   // check reads zeros).
-  static constexpr int KPAD = KF >= 1 ? (KBYTES + 1023) / 1024 * 1024 : KBYTES;
-  static constexpr int KW = KF >= 1 ? KPAD / 1024 : VW;  // K DMA instructions per wave
+  static constexpr bool CODES = KF == 1 || KF == 2;
+  static constexpr int KPAD = CODES ? (KBYTES + 1023) / 1024 * 1024 : KBYTES;
+  static constexpr int KW = CODES ? KPAD / 1024 : KBYTES / 1024 / kWaves;  // K DMA instructions per wave
   static constexpr int NUSED = KF == 1 ? kChunk * 4 : KF == 2 ? kChunk * 16 : 0;  // scale bytes of a block
-  static constexpr int NBYTES = KF >= 1 ? 1024 : 0;
+  static constexpr int NBYTES = CODES ? 1024 : 0;
   static constexpr int BYTES = VBYTES + KPAD + NBYTES;
-  static constexpr int LW = VW + KW + (KF >= 1 ? 1 : 0);  // DMA instructions per wave per block
-  static constexpr int BOOKS = KF >= 1 ? KS * 1024 * KF : 0;  // KF 1: 256 fp32 centroids per K-step
-  static constexpr int KOP = KF >= 1 ? 2 * 2 * KS * 2048 : 0;  // [buffer][u][s]: hi 1 KB, lo 1 KB
+  static constexpr int LW = VW + KW + (CODES ? 1 : 0);  // DMA instructions per wave per block
+  static constexpr int BOOKS = CODES ? KS * 1024 * KF : 0;  // KF 1: 256 fp32 centroids per K-step
+  static constexpr int KOP = CODES ? 2 * 2 * KS * 2048 : 0;  // [buffer][u][s]: hi 1 KB, lo 1 KB
   static constexpr int CURSOR = kWaves * 32;  // each wave's segment cursor (8 ints), after the operands
   static constexpr int FIXED = BOOKS + KOP + CURSOR;
   static constexpr int RING = 6 * BYTES + FIXED <= kLdsLimit / 2 ? 6 : 4 * BYTES + FIXED <= kLdsLimit / 2 ? 4 : 3;
-  static constexpr int AHEAD = RING - 2;
+  // With a build the block after the one computed on has landed too.
+  static constexpr int AHEAD = CODES ? RING - 2 : RING - 1;
   static constexpr int LDS = RING * BYTES + FIXED;
   static_assert(VI % kWaves == 0 && KBYTES % 16 == 0 && NUSED <= NBYTES, "DMA split over four waves");
   static_assert(LDS <= kLdsLimit, "LDS of one workgroup");
@@ -160,7 +164,8 @@ __device__ __forceinline__ int64_t query_row(int b, int rows, int Hq, int kv, in
 }
 
 // KF: 1 = packed codes of a structured layout, 2 = packed codes of any
-// layout, 0 = FP16 K rows. NN: leading nibble K-steps. SG: K-steps in group 0. NCB: 16-query column blocks per wave. At least two
+// layout, 3 = packed codes whose operands prefill_operand_kernel built, 0 =
+// FP16 K rows. NN: leading nibble K-steps. SG: K-steps in group 0. NCB: 16-query column blocks per wave. At least two
 // waves per SIMD (at most 256 registers each), so that one wave's softmax
 // overlaps another's matrix-core work; up to four for single-block tiles.
 //
@@ -289,6 +294,12 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
     const int e_tile = start + (q0 + n_valid - 1) / G + 1;  // exclusive end of the tile's last query
     const int t_lo = blk_lo * kChunk, t_hi = min(t_lo + n_blocks * kChunk, e_tile);
     const DevTables *T = KF >= 1 ? p.tables[kv] : nullptr;
+    // KF 3: the unit's built operands and scale exponents from the segment's first block on.
+    const int64_t kb0 = KF == 3 ? (int64_t)(b * p.kv_heads + kv) * p.operand_blocks + blk_lo : 0;
+    const uint8_t *const kop_g = KF == 3 ? p.operands + kb0 * Sl::KBYTES : nullptr;
+    // Scalar loads (constant address space): a vector load's wait would cover the ring's DMAs.
+    typedef const __attribute__((address_space(4))) int32_t const_i32;
+    const_i32 *const kexp_g = KF == 3 ? (const_i32 *)(p.operand_exp + kb0) : nullptr;
     // Row bytes and scales per token (runtime for KF 2).
     // Table fields are wave-uniform: scalar values, so buffer descriptors built
     // from them need no per-lane loop.
@@ -325,7 +336,14 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
 #pragma unroll
       for (int kk = 0; kk < Sl::VW; ++kk) dma16(rV, sb + (wave * Sl::VW + kk) * 1024, voff_rows[kk], 0);
       uint8_t *kb = sb + Sl::VBYTES;
-      if (KF >= 1) {
+      if (KF == 3) {
+        const __amdgpu_buffer_rsrc_t rK = rsrc(kop_g + (int64_t)i * Sl::KBYTES, Sl::KBYTES);
+#pragma unroll
+        for (int kk = 0; kk < Sl::KW; ++kk) {
+          const int off = (wave * Sl::KW + kk) * 1024;
+          dma16(rK, kb + off, off + ln * 16, 0);
+        }
+      } else if (KF >= 1) {
         // Ranges end on the access size: the range check zeroes a whole access
         // reaching past the range; the bytes past the last row lie in the same
         // aligned 4 bytes as its end (16-byte aligned bases, c0 a multiple of 32).
@@ -512,8 +530,10 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
     lim_min = wave_min(lim_min);
     // Block 0 (and the books before it) landed for every wave; the later
     // blocks stay in flight.
-    wait_blocks<Sl::LW, AHEAD - 1>(min(n_blocks, AHEAD) - 1);
-    lds_barrier();
+    if constexpr (Sl::CODES) {
+      wait_blocks<Sl::LW, AHEAD - 1>(min(n_blocks, AHEAD) - 1);
+      lds_barrier();
+    }
 
     // Builds block i's K operand into buffer i & 1; returns E (2^E >= every
     // FP16 scale of the block). Thread (wave w, lane) builds the (u, s) steps
@@ -603,6 +623,8 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
           *reinterpret_cast<half8 *>(dst + 1024) = lo;
         }
         return E;
+      } else if constexpr (KF == 3) {
+        return kexp_g[min(i, n_blocks - 1)];
       } else {
         return 0;
       }
@@ -653,7 +675,7 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
           if constexpr (KF >= 1) {
-            const uint8_t *src = kop + (i & 1) * (2 * KS * 2048) + (u * KS + s) * 2048 + lane * 16;
+            const uint8_t *src = (KF == 3 ? sb + Sl::VBYTES : kop + (i & 1) * (2 * KS * 2048)) + (u * KS + s) * 2048 + lane * 16;
             const half8 ah = *reinterpret_cast<const half8 *>(src), al = *reinterpret_cast<const half8 *>(src + 1024);
 #pragma unroll
             for (int cb = 0; cb < NCB; ++cb) {
@@ -753,6 +775,16 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
     auto run = [&](auto nib_c) {
       int E_cur = build(0, nib_c);
       for (int i = 0; i < n_blocks; ++i) {
+        if constexpr (!Sl::CODES) {
+          // Block i landed for every wave and block i - 1 done with: its buffer
+          // takes block i - 1 + RING = i + AHEAD.
+          wait_blocks<Sl::LW, AHEAD - 1>(min(n_blocks - 1 - i, AHEAD - 1));
+          lds_barrier();
+          if (i + AHEAD < n_blocks) issue(i + AHEAD);
+          if (t_lo + i * kChunk + kChunk > lim_min) E_cur = step(i, E_cur, std::true_type{}, nib_c);
+          else E_cur = step(i, E_cur, std::false_type{}, nib_c);
+          continue;
+        }
         // Block i + AHEAD goes to the buffer of block i - 2, whose V every wave
         // read before the barrier of iteration i - 1. Wait for block i + 1
         // (built below); block i has landed already.
@@ -856,6 +888,87 @@ prefill_kernel(PrefillParams p, FastLayout fl) {
       first = false;
     }
   }
+}
+
+// The K operands of a chunk's whole history, built once for all its query
+// tiles: the arithmetic of the KF 2 build above (any packed layout), a
+// workgroup per (32-token block, sequence x KV head), a wave per 16-token x
+// 32-dim piece. Block: [u][s] pieces of 2 KB, hi 1 KB then lo 1 KB in the
+// MFMA A-operand lane order; operand_exp holds its E. Latency bound (a 32-token
+// block is about 3 KB in and 8 KB out, 384 blocks one round of workgroups):
+// 5 us for 4078 tokens x 3 heads. The attention kernel then only streams:
+// 1001 rows x 3 heads after 3077 tokens on the SmolLM2 heads 76 -> 42 us, layout
+// A at d=128 (4 heads) 343 -> 77 us with both launches.
+template <int D>
+__global__ __launch_bounds__(kThreads) void prefill_operand_kernel(PrefillParams p) {
+  using Sl = PSlot<D, 2, 0>;
+  constexpr int KS = Sl::KS;
+  __shared__ __align__(16) uint8_t smem[Sl::BOOKS + Sl::KPAD + Sl::NBYTES];
+  float *books = reinterpret_cast<float *>(smem);
+  uint8_t *kraw = smem + Sl::BOOKS;
+  uint16_t *nrm = reinterpret_cast<uint16_t *>(kraw + Sl::KPAD);
+  const int tid = threadIdx.x, lane = tid & 63, gq = lane >> 4, col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int blk = (int)blockIdx.x, unit = (int)blockIdx.y, b = unit / p.kv_heads, kv = unit - b * p.kv_heads;
+  const int rest = min(seq_start(p, b) + p.rows - blk * kChunk, kChunk);
+  if (rest <= 0) return;  // workgroup-uniform: past the history
+  const DevTables *T = p.tables[kv];
+  const int rb = __builtin_amdgcn_readfirstlane(T->row_bytes), ns = __builtin_amdgcn_readfirstlane(T->norm_stride);
+  const int mc = __builtin_amdgcn_readfirstlane(T->max_centroids), ec = __builtin_amdgcn_readfirstlane(T->cent_exp);
+  const int groups = __builtin_amdgcn_readfirstlane(T->groups);
+  const uint32_t book_bytes = (uint32_t)__builtin_amdgcn_readfirstlane(T->n_books * T->max_centroids * 4);
+  const __amdgpu_buffer_rsrc_t rB = rsrc(tables_books(T), book_bytes);
+  const __amdgpu_buffer_rsrc_t rK = rsrc(p.packed + b * p.packed_seq_stride + kv * p.packed_head_stride +
+                                             (int64_t)blk * kChunk * rb, ((uint32_t)rest * rb + 3u) & ~3u);
+  const __amdgpu_buffer_rsrc_t rN = rsrc(p.norms + b * p.norms_seq_stride + kv * p.norms_head_stride +
+                                             (int64_t)blk * kChunk * ns, ((uint32_t)rest * ns * 2 + 3u) & ~3u);
+  for (int k = wave; k < Sl::BOOKS / 256; k += kWaves)
+    if ((uint32_t)k * 256 < book_bytes) dma4(rB, smem + 256 * k, 256 * k + lane * 4, 0);
+#pragma unroll
+  for (int kk = 0; kk < Sl::KW; ++kk) {
+    const int off = (kk * kWaves + wave) * 256;
+    dma4(rK, kraw + off, off + lane * 4, 0);
+  }
+  dma4(rN, kraw + Sl::KPAD + wave * 256, wave * 256 + lane * 4, 0);
+  const u32x4 *gd = reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint8_t *>(T) + T->off_gdesc);
+  u32x4 gdl[KS / 2][2];  // this wave's pieces: wave + 4 k, K-step (wave + 4 k) % KS
+#pragma unroll
+  for (int k = 0; k < KS / 2; ++k) {
+    const int s = (wave + kWaves * k) % KS;
+    gdl[k][0] = gd[8 * s + gq];
+    gdl[k][1] = gd[8 * s + 4 + gq];
+  }
+  wait_vm<0>();
+  __syncthreads();
+  // E bounds the scales of the block's tokens inside the history.
+  float smax = 0.0f;
+  const int tl = lane & 31;
+  for (int g = lane >> 5; g < groups; g += 2) smax = fmaxf(smax, tl < rest ? fabsf(h2f(nrm[tl * ns + g])) : 0.0f);
+  smax = wave_max(smax);
+  const int E = smax > 0.0f ? (int)ceilf(__builtin_log2f(smax)) : 0;
+  const int64_t slot = (int64_t)unit * p.operand_blocks + blk;
+  float one = 1.0f;
+  asm volatile("" : "+s"(one));
+#pragma unroll
+  for (int k = 0; k < KS / 2; ++k) {
+    const int combo = wave + kWaves * k, u = combo / KS, t = 16 * u + col;
+    float v[8];
+#pragma unroll
+    for (int k2 = 0; k2 < 8; ++k2) {
+      const uint32_t dsc = gdl[k][k2 >> 2][k2 & 3];
+      const uint32_t byte = kraw[t * rb + (int)(dsc & 255u)];
+      const uint32_t code = (dsc >> 11) & 1u ? (byte >> ((dsc >> 8) & 7u)) & 15u : byte;
+      const float c = books[(int)((dsc >> 12) & 15u) * mc + (int)code];
+      const float sc = t < rest ? h2f(nrm[t * ns + (int)((dsc >> 16) & 15u)]) : 0.0f;
+      v[k2] = c * __builtin_ldexpf(sc, ec - E);
+    }
+    half8 hi, lo;
+    split8_mix(v, one, hi, lo);
+    uint8_t *dst = p.operands + (slot * 2 * KS + combo) * 2048 + lane * 16;
+    *reinterpret_cast<half8 *>(dst) = hi;
+    *reinterpret_cast<half8 *>(dst + 1024) = lo;
+  }
+  if (tid == 0) p.operand_exp[slot] = E;
 }
 
 // LSE merge of the tiles whose history several ranges shared. Grid (unit,
@@ -1049,6 +1162,14 @@ int prefill_general_book_bytes(int dim) { return dim == 64 ? PSlot<64, 2, 0>::BO
 
 hipError_t launch_prefill(const PrefillParams &p, const FastLayout &fl, int nn, int sg, hipStream_t stream) {
   const int D = p.dim;
+  if (p.operands) {
+    const dim3 grid((unsigned)p.operand_blocks, (unsigned)(p.batch * p.kv_heads));
+    if (D == 64) hipLaunchKernelGGL(prefill_operand_kernel<64>, grid, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL(prefill_operand_kernel<128>, grid, dim3(kThreads), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return D == 64 ? launch_one<64, 3, 0, 1>(p, fl, stream) : launch_one<128, 3, 0, 1>(p, fl, stream);
+  }
   if (nn < 0) return D == 64 ? launch_one<64, 2, 0, 1>(p, fl, stream) : launch_one<128, 2, 0, 1>(p, fl, stream);
   if (p.key_format == 0) return D == 64 ? launch_one<64, 0, 0, 2>(p, fl, stream) : launch_one<128, 0, 0, 4>(p, fl, stream);
 #define BGTQ_PREFILL(DD, N, S) \

@@ -306,7 +306,10 @@ bgtq_status bgtq_decode_noalloc(bgtq_context *ctx, const bgtq_decode_desc *d);
  *   v: FP16. Key formats and strides are those of bgtq_decode.
  *   workspace: 16-byte aligned device memory of at least
  *   bgtq_prefill_workspace_size() bytes for the partial results of query
- *   rows or tiles whose history several workgroups share. Its first
+ *   rows or tiles whose history several workgroups share and, in long tiled
+ *   chunks, the history's rebuilt K operands (4 * dim bytes per token and KV
+ *   head, at most 1 GiB; a workspace of the partial results alone still works,
+ *   every tile then rebuilding K itself: same outputs, slower). Its first
  *   BGTQ_PREFILL_COUNTER_BYTES bytes (split arrival counters) must be zero
  *   before the first call on it, and every call leaves them zero, whatever
  *   its geometry; the rest needs no initial contents. Calls sharing a

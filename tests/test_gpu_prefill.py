@@ -5,12 +5,15 @@ causally to the sequence's history (src/model/decoder.ts:46-56 per chunk,
 src/model/compressed-dot.wgsl:28). Outputs must match the oracle's causal
 attention on the same effective K within |gpu - oracle| <= 1e-5 + 1e-4 |oracle|.
 """
+from pathlib import Path
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 ATOL, RTOL = 1e-5, 1e-4
+GOLDEN = Path(__file__).parent / "golden" / "reference"
 
 
 def _olayout(oracle, p):
@@ -347,5 +350,54 @@ def test_workspace_shared_across_paths(device, oracle):
                 for h in range(2):
                     ref = _reference(oracle, cache, q, eff, b, h, G)
                     _check(got[b, :, h * G:(h + 1) * G], ref.astype(np.float64), f"rows {rows} b{b} kv{h}")
+    finally:
+        cache.destroy()
+
+
+@pytest.mark.parametrize("layout,dim,hq,rows,starts", [
+    ("S", 64, 9, 683, [0, 300]),      # 2049 queries: just past the 256-query tiles' line, odd lengths
+    ("A", 64, 8, 512, [1, 33]),       # 2048 queries, a history one token into a block
+    ("A", 128, 2, 65, [0, 158]),      # two 64-query tiles, the smallest launch of this route
+    ("A", 128, 8, 513, [31, 64]),
+    ("B", 128, 16, 256, [0, 95]),     # a structured layout at its line (4096 queries)
+])
+def test_operands_built_once_match_per_tile_build(device, oracle, layout, dim, hq, rows, starts):
+    """The K operands built once per call and by every tile are the same numbers: outputs bit for bit
+    equal (one byte less workspace selects the per-tile build), and within tolerance of the oracle."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate, calibration
+    hkv = 3 if layout == "S" else 2 if hq % 2 == 0 and hq < 16 else 1
+    if layout == "S":
+        blobs = calibration.read(GOLDEN / "model")[2]
+        params = [bgtq.BlockGTQParameters.from_serialized(b.config, b.table) for b in blobs[:hkv]]
+    else:
+        params = [(calibrate.layout_a if layout == "A" else calibrate.layout_b)(dim)] * hkv
+    cap = max(starts) + rows
+    one = max(params, key=lambda p: p.rowBytes)
+    cache = Cache(device, params=[one] * hkv, batch=2, hkv=hkv, dim=dim, cap=cap, pad16=True)
+    try:
+        g = torch.Generator().manual_seed(rows)
+        q = torch.randn((2, rows, hq, dim), generator=g)
+        outs = []
+        for cut in (0, 1):
+            out = torch.full((2, rows, hq, dim), float("nan"), device="cuda")
+            kw = dict(batch=2, rows=rows, q_heads=hq, kv_heads=hkv, dim=dim, q=q.cuda(), out=out,
+                      starts=torch.tensor(starts, dtype=torch.int32).cuda(), max_length=cap, v=cache.vd,
+                      v_seq_stride=cache.vd.stride(0), v_head_stride=cache.vd.stride(1), **cache.kw)
+            need = batched.prefill_workspace_bytes(batched.prefill_desc(**kw))
+            assert need > 2 * hkv * cap * 4 * dim, "no operand space: this size does not reach the route"
+            ws = torch.full((need,), 0xff, dtype=torch.uint8, device="cuda")
+            ws[:262144] = 0
+            print("prefill operands", layout, dim, rows, starts, "cut", cut, flush=True)
+            batched.prefill(device, batched.prefill_desc(workspace=ws[:need - cut], **kw))
+            torch.cuda.synchronize()
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1])
+        got, G = outs[0].cpu().numpy(), hq // hkv
+        sel = np.array([0, 1, rows // 2, rows - 1])
+        for b in range(2):
+            ref = _reference(oracle, cache, q, starts, b, hkv - 1, G, sel)
+            _check(got[b, sel][:, (hkv - 1) * G:], ref.astype(np.float64), f"b{b}")
     finally:
         cache.destroy()
