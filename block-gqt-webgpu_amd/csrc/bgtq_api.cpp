@@ -997,6 +997,39 @@ static int choose_splits(int64_t units, uint32_t max_length, int32_t requested) 
   return (int)std::min<int64_t>(want, max_splits);
 }
 
+// The fused decode's splits, by the rounds the launch takes on the chip's
+// workgroup slots (two resident workgroups per compute unit): choose_splits
+// rounds the splits up, and 63 units x 9 left 55 workgroups of 567 to a second
+// round of their own. Cost in tokens of one workgroup: every round has a set-up
+// and merge worth 512 tokens (6 us), a full round its share of the sequence,
+// a last round filled to f 0.6 + 0.4 f of that (HBM feeds the fewer workgroups
+// faster). Fewest splits win ties within 1%. us per call, rounded up / this rule:
+// 63 units x 8191 tokens (SmolLM2 heads) 35.7 (9) / 25.0 (8), 42 x 8191 22.4 (13) /
+// 17.5 (12), 200 x 8191 68.1 (3) / 53.4 (2), 120 x 2000 24.6 (5) / 18.1 (4), d=128
+// 40 x 5000 25.9 (13) / 23.4 (12); above half the slots 270 x 8000 102.8 (2) / 84.4
+// (3), 300 x 1000 19.8 (2) / 16.6 (1), 320 x 4000 53.6 (2) / 43.7 (3). More units
+// than slots keep one split (640 sequences of 250 to 2000 tokens 32.6 us, two
+// splits 37.0: the short ones' workgroups already make room). extra: more
+// workgroups per unit beside the splits (an appended token's).
+static int fused_decode_splits(int64_t units, uint32_t max_length, int extra) {
+  const int64_t max_splits = std::min<int64_t>(256, std::max<int64_t>(1, (max_length + 127) / 128));
+  const int64_t slots = 2 * (int64_t)device_cus();
+  const int64_t first = std::min(max_splits, std::max<int64_t>(1, slots / units - extra));
+  const int64_t last = units > slots ? 1 : std::min(max_splits, std::max<int64_t>(first, 3 * slots / units));
+  int64_t best = first;
+  double best_cost = 0;
+  for (int64_t s = first; s <= last; ++s) {
+    const int64_t wgs = units * (s + extra), full = wgs / slots, rest = wgs % slots;
+    const double part = rest ? 0.6 + 0.4 * (double)rest / (double)slots : 0.0;
+    const double cost = ((double)full + part) * max_length / (double)s + 512.0 * (double)(full + (rest ? 1 : 0));
+    if (s == first || cost < 0.99 * best_cost) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return (int)best;
+}
+
 // Decodes of few (sequence, KV head) units at d=64 on a structured layout or
 // FP16 K (at most one four-wave workgroup per compute unit): eight-wave
 // workgroups, each split covering twice the tokens (256), so the last
@@ -1064,7 +1097,9 @@ bgtq_status bgtq_decode_workspace_size(const bgtq_decode_desc *d, size_t *bytes)
   int splits = 1;
   if (bgtq_status s = validate_decode(d, &splits)) return s;
   if (!bytes) return fail(BGTQ_ERR_RANGE, "null output");
-  *bytes = decode_ws((int64_t)d->batch * d->kv_heads, (int64_t)d->batch * d->q_heads, d->dim, splits).total;
+  const int64_t units = (int64_t)d->batch * d->kv_heads;
+  if (d->splits <= 0) splits = std::max(splits, fused_decode_splits(units, d->max_length, 0));
+  *bytes = decode_ws(units, (int64_t)d->batch * d->q_heads, d->dim, splits).total;
   return BGTQ_OK;
 }
 
@@ -1194,6 +1229,7 @@ static bgtq_status launch_decode_common(bgtq_context *ctx, DecodeParams &p, cons
     fused = true;
   }
   if (fused) {
+    if (p.fused_splits) p.splits = p.fused_splits;
     if (!p.starts) choose_waves(p, nn);
     HIP_TRY(launch_decode_fast(p, fl, nn, sg, ctx->stream), "decode launch");
     if (p.probs) HIP_TRY(launch_decode_probs(p, ctx->stream), "probabilities launch");
@@ -1254,9 +1290,18 @@ static bgtq_status decode_impl(bgtq_context *ctx, const bgtq_decode_desc *d, con
   int splits = 1;
   if (bgtq_status s = validate_decode(d, &splits)) return s;
   const int64_t heads = (int64_t)d->batch * d->q_heads;
-  const DecodeWorkspace w = decode_ws((int64_t)d->batch * d->kv_heads, heads, d->dim, splits);
+  const int64_t units = (int64_t)d->batch * d->kv_heads;
+  DecodeWorkspace w = decode_ws(units, heads, d->dim, splits);
   if (!d->workspace || d->workspace_bytes < w.total)
     return fail(BGTQ_ERR_RANGE, "workspace of %zu bytes required", w.total);
+  // The fused kernel's own choice, as long as its partials fit the workspace
+  // (one sized for another call need only hold the general kernel's).
+  int fused_splits = d->splits > 0 ? splits : fused_decode_splits(units, d->max_length, a ? 1 : 0);
+  if (fused_splits > splits) {
+    const DecodeWorkspace wf = decode_ws(units, heads, d->dim, fused_splits);
+    if (d->workspace_bytes >= wf.total) w = wf;
+    else fused_splits = splits;
+  }
   if (bgtq_status s = ctx->use()) return s;
   DecodeParams p{};
   for (int h = 0; h < d->kv_heads; ++h) p.tables[h] = d->key_format == BGTQ_KEYS_PACKED ? d->tables[h]->dev() : nullptr;
@@ -1291,6 +1336,7 @@ static bgtq_status decode_impl(bgtq_context *ctx, const bgtq_decode_desc *d, con
   p.ends = nullptr;
   p.splits = splits;
   p.splits_forced = d->splits > 0;
+  p.fused_splits = fused_splits;
   p.split_tokens = (int)((d->max_length + p.splits - 1) / p.splits);
   p.split_tokens = ((p.split_tokens + 127) / 128) * 128;
   p.inv_sqrt_d = (float)(1.0 / std::sqrt((double)d->dim));
@@ -1319,6 +1365,7 @@ static bgtq_status decode_impl(bgtq_context *ctx, const bgtq_decode_desc *d, con
     if (!fused)
       return fail(BGTQ_ERR_UNSUPPORTED,
                   "decode_append needs the fused kernel's layouts; use bgtq_encode_batched and bgtq_decode");
+    p.splits = fused_splits;
     choose_waves(p, nn);
     HIP_TRY(launch_decode_fast(p, fl, nn, sg, ctx->stream), "decode append launch");
     return BGTQ_OK;
@@ -1633,7 +1680,11 @@ bgtq_status bgtq_attention_create(bgtq_keys *k, bgtq_values *v, uint32_t max_que
   a->values = v;
   a->max_queries = max_queries;
   a->materialize = materialize ? 1 : 0;
-  a->max_splits = (uint32_t)std::min<int64_t>(256, std::max<int64_t>(1, ((int64_t)k->capacity + 255) / 256));
+  // Splits of one 32-token chunk per wave of the fused kernel (4096 tokens, d=128,
+  // FP32 V, 3 queries: 20.6 us with two chunks per wave, 17.7 with one);
+  // the general kernel keeps 256 tokens.
+  const int64_t floor_tok = k->kind != BGTQ_KEYS_COMPRESSED && (k->dim == 64 || k->dim == 128) ? 128 : 256;
+  a->max_splits = (uint32_t)std::min<int64_t>(256, std::max<int64_t>(1, ((int64_t)k->capacity + floor_tok - 1) / floor_tok));
   const size_t d = k->dim, Q = max_queries;
   bgtq_status s = k->ctx->use();
   struct Item {

@@ -155,6 +155,7 @@ struct DecodeParams {
   int32_t v_dtype;  // 0 = FP32, 1 = FP16
   int32_t waves;          // decode workgroup waves of the fused kernel: 8 (d=64, few units), else 4
   int32_t splits_forced;  // the caller fixed the split count
+  int32_t fused_splits;     // the fused kernel's splits, 0 = splits (bgtq_decode's general kernel always takes splits)
   int64_t v_seq_stride, v_head_stride;  // elements
   const float *q;         // [B*Hq*dim] queries
   int32_t q_rotated;      // 1: q is already R q[perm] (code domain); the kernels do not rotate it

@@ -409,3 +409,45 @@ def test_fp32_values_batched(device, oracle, key_format, layout, dim, hq, hkv, l
     finally:
         for t in tabs:
             t.destroy()
+
+
+@pytest.mark.parametrize("batch,hkv,ctx,fewer", [
+    (150, 2, 3000, 2),  # 300 units: three splits where the rounded-up count is two
+    (150, 2, 3000, 0),
+    (257, 2, 200, 0),   # 514 units, just past the workgroup slots: one split
+    (32, 8, 129, 0),    # 256 units, two splits of which the second holds one token
+    (21, 3, 1500, 0),   # 63 units: eight splits, one workgroup per slot at most
+])
+def test_default_splits_by_rounds(device, batch, hkv, ctx, fewer):
+    """The library's split choice at the edges of its rule, and a workspace sized for `fewer` splits
+    (the call then takes those), against float64 attention."""
+    import torch
+    from bgtq import batched
+    batched.bind_torch_stream(device)
+    G, dim = 2, 64
+    g = torch.Generator().manual_seed(batch)
+    k = torch.randn((hkv, ctx, dim), generator=g).half()  # every sequence reads the same rows (stride 0)
+    v = torch.randn((hkv, ctx, dim), generator=g).half()
+    q = torch.randn((batch, hkv * G, dim), generator=g)
+    lengths = [ctx if b % 50 == 0 else 1 + (37 * b) % min(ctx, 300) for b in range(batch)]
+    out = torch.full((batch, hkv * G, dim), float("nan"), device="cuda")
+    kd, vd = k.cuda(), v.cuda()
+    kw = dict(batch=batch, q_heads=hkv * G, kv_heads=hkv, dim=dim, q=q.cuda(), out=out,
+              lengths=torch.tensor(lengths, dtype=torch.int32).cuda(), max_length=ctx, v=vd, v_seq_stride=0,
+              v_head_stride=ctx * dim, k_f16=kd, k_seq_stride=0, k_head_stride=ctx * dim)
+    need = batched.workspace_bytes(batched.decode_desc(**kw))
+    if fewer:
+        small = batched.workspace_bytes(batched.decode_desc(splits=fewer, **kw))
+        assert small < need
+        need = small
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    print("default splits", batch, hkv, ctx, fewer, flush=True)
+    for _ in range(2):
+        batched.decode(device, batched.decode_desc(workspace=ws, **kw))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    for b in range(batch):
+        n = lengths[b]
+        for h in range(hkv):
+            s = q[b, h * G:(h + 1) * G].double() @ k[h, :n].double().t() / dim ** 0.5
+            _check(got[b, h * G:(h + 1) * G], (torch.softmax(s, 1) @ v[h, :n].double()).numpy(), f"b{b} kv{h} T={n}")
