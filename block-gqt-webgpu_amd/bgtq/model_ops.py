@@ -17,6 +17,7 @@ tables (a Calibration head's .config / .table, or a Tables object).
 from __future__ import annotations
 
 import ctypes
+import struct
 
 from . import _lib
 from ._lib import RangeError, check, lib
@@ -28,15 +29,25 @@ MAX_WORKGROUPS_PER_DIMENSION = 0x7FFFFFFF
 ATTENTION_PATH = ("append", "encode_k", "dot", "compressed_dot", "softmax", "weighted")
 
 
-def _binding(b) -> _lib.Binding:
+# The C structs a submit passes, filled with struct: building a ctypes object per
+# binding (37 in a SmolLM2 layer's nine dispatches) cost as much host time as
+# the layer's kernels take.
+_DISPATCH = struct.Struct("=Q8IQQII")  # bgtq_model_dispatch
+assert _DISPATCH.size == ctypes.sizeof(_lib.ModelDispatch) and ctypes.sizeof(_lib.Binding) == 24
+_NAMES = {n: ctypes.create_string_buffer(n.encode()) for n in ATTENTION_PATH}
+
+
+def _binding(b) -> tuple[int, int, int]:
+    """bgtq_model_binding's words: device address, bytes, tables handle."""
     if b is None:
-        return _lib.Binding(None, 0, None)
-    handle = getattr(b, "handle", None)
-    if handle is not None and hasattr(b, "info"):  # calibration Tables
-        return _lib.Binding(None, 0, handle)
+        return 0, 0, 0
+    if not hasattr(type(b), "data_ptr"):
+        handle = getattr(b, "handle", None)
+        if handle is not None and hasattr(b, "info"):  # calibration Tables
+            return 0, 0, handle.value
     if not b.is_contiguous():
         raise RangeError("Model buffers must be contiguous")
-    return _lib.Binding(ctypes.c_void_p(b.data_ptr()), b.numel() * b.element_size(), None)
+    return b.data_ptr(), b.nbytes, 0
 
 
 class ModelOps:
@@ -60,21 +71,28 @@ class Commands:
         if x > MAX_WORKGROUPS_PER_DIMENSION or y > MAX_WORKGROUPS_PER_DIMENSION:
             raise RangeError("Model dispatch limit")
         params = [int(v) & 0xFFFFFFFF for v in list(parameters)[:8]]
-        self._dispatches.append((name, params + [0] * (8 - len(params)), list(buffers), int(x), int(y)))
+        if len(params) < 8:
+            params += [0] * (8 - len(params))
+        self._dispatches.append((name, params, list(buffers), int(x), int(y)))
 
     def submit(self) -> None:
         """Queue every recorded dispatch in order, then wait for the device.
         A dispatch that fails its checks raises before anything is queued."""
         n = len(self._dispatches)
+        words, keep = [], []
+        for _, _, buffers, _, _ in self._dispatches:
+            for b in buffers:
+                words += _binding(b)
+        binds = (ctypes.c_uint64 * max(1, len(words)))(*words)
+        at = ctypes.addressof(binds)
         arr = (_lib.ModelDispatch * max(1, n))()
-        keep = []
         for i, (name, params, buffers, x, y) in enumerate(self._dispatches):
-            binds = (_lib.Binding * max(1, len(buffers)))(*[_binding(b) for b in buffers])
-            keep.append(binds)
-            encoded = name.encode()
-            keep.append(encoded)
-            arr[i] = _lib.ModelDispatch(encoded, (ctypes.c_uint32 * 8)(*params),
-                                        ctypes.cast(binds, ctypes.POINTER(_lib.Binding)), len(buffers), x, y)
+            text = _NAMES.get(name)
+            if text is None:
+                text = ctypes.create_string_buffer(name.encode())
+                keep.append(text)
+            _DISPATCH.pack_into(arr, i * _DISPATCH.size, ctypes.addressof(text), *params, at, len(buffers), x, y)
+            at += 24 * len(buffers)
         self._dispatches = []
         check(lib().bgtq_model_submit(self.ops.device.handle, arr, n))
         self.ops.device.synchronize()
