@@ -1376,6 +1376,7 @@ static bgtq_status decode_impl(bgtq_context *ctx, const bgtq_decode_desc *d, con
 // ---------------------------------------------------------------- chunked prefill
 struct PrefillPlan {
   int tiles, tile_queries, ranges, range_blocks;
+  int64_t work;      // the most work of the launch, in the kernel's cost units
   size_t records;    // bytes of the workgroups' partial records
   size_t workspace;  // records, then the tile table (16 bytes per tile)
   size_t operands;   // bytes of the built K operands and their exponents after those, 0 = built per tile
@@ -1389,9 +1390,9 @@ struct PrefillPlan {
   size_t counters, part;  // rowwise: workspace offsets (the split counters first)
 };
 
-// Query tiles: four waves of one 16-query block each for small chunks (more
-// tiles to spread), of prefill_column_blocks(dim) blocks each for long ones
-// (the K operand rebuilt once per block serves more queries). Workgroups:
+// Query tiles: four waves of one 16-query block each for small launches (more
+// tiles to spread), of prefill_column_blocks(dim) blocks each for large ones
+// (a block's K operand serves more queries). Workgroups:
 // the flattened work (every KV head, sequence and tile's causal history in
 // 32-token blocks) is cut into equal ranges, about two workgroups per
 // compute unit, sized here for the most work (every chunk at the end of the
@@ -1460,16 +1461,21 @@ static bgtq_status plan_prefill(const bgtq_prefill_desc *d, PrefillPlan *plan, b
         kPrefillCounterBytes + sizeof(float) * (size_t)row_units * uc * (splits_plain + app_max) * (d->dim + 4);
     return BGTQ_OK;
   }
-  plan->tile_queries = nq >= 2048 ? 64 * prefill_column_blocks(d->dim) : 64;
-  plan->tiles = (int)((nq + plan->tile_queries - 1) / plan->tile_queries);
-  if ((int64_t)d->batch * plan->tiles > INT32_MAX / 2) return fail(BGTQ_ERR_UNSUPPORTED, "too many query tiles");
   // The most work (in the kernel's cost units: a segment's set-up plus 32-token blocks of every tile's
   // history) with each chunk at the end of the cache.
-  const int64_t start = (int64_t)d->max_length - d->rows, tq = plan->tile_queries;
-  int64_t w1 = 0;
-  for (int64_t t = 0; t < plan->tiles; ++t)
-    w1 += kPrefillSegmentCost + (start + (std::min(nq, (t + 1) * tq) - 1) / G + 1 + 31) / 32;
-  const int64_t w_max = w1 * d->batch * d->kv_heads;
+  const int64_t start = (int64_t)d->max_length - d->rows;
+  auto most_work = [&](int64_t tq) {
+    int64_t w = 0;
+    for (int64_t t = 0; t * tq < nq; ++t)
+      w += kPrefillSegmentCost + (start + (std::min(nq, (t + 1) * tq) - 1) / G + 1 + 31) / 32;
+    return w * d->batch * d->kv_heads;
+  };
+  const int64_t wide = 64 * prefill_column_blocks(d->dim);
+  plan->tile_queries = (int)(nq < 2048 || (d->dim == 64 && most_work(wide) < prefill_wide_tile_work(device_cus())) ? 64 : wide);
+  const int64_t tq = plan->tile_queries;
+  plan->tiles = (int)((nq + tq - 1) / tq);
+  if ((int64_t)d->batch * plan->tiles > INT32_MAX / 2) return fail(BGTQ_ERR_UNSUPPORTED, "too many query tiles");
+  const int64_t w_max = most_work(tq);
   if (w_max > INT32_MAX / 2) return fail(BGTQ_ERR_UNSUPPORTED, "prefill work above 2^30 blocks of 32 tokens");
   int64_t ranges, range_blocks = 0;
   if (d->split_tokens > 0) {
@@ -1483,12 +1489,13 @@ static bgtq_status plan_prefill(const bgtq_prefill_desc *d, PrefillPlan *plan, b
     ranges = std::min<int64_t>(2 * (int64_t)device_cus(), (w_max + kPrefillMinRange - 1) / kPrefillMinRange);
   }
   plan->ranges = (int)std::max<int64_t>(1, ranges);
+  plan->work = w_max;
   plan->range_blocks = (int)range_blocks;
   plan->records = plan->ranges > 1 ? sizeof(float) * (size_t)plan->ranges * 2 * tq * (d->dim + 2) : 0;
   const size_t info = plan->ranges > 1 ? 16 * (size_t)d->batch * d->kv_heads * plan->tiles : 0;
   plan->workspace = kPrefillCounterBytes + plan->records + info;
   if (d->key_format == BGTQ_KEYS_PACKED && plan->tiles > 1 &&
-      prefill_operands_once(d->dim, false, nq)) {
+      prefill_operands_once(d->dim, false, nq, plan->tile_queries, w_max, device_cus())) {
     plan->operand_blocks = (int)(((int64_t)d->max_length + 31) / 32);
     const size_t blocks = (size_t)d->batch * d->kv_heads * plan->operand_blocks;
     const size_t bytes = blocks * 32 * 4 * d->dim + (blocks * 4 + 15) / 16 * 16;
@@ -1654,7 +1661,7 @@ static bgtq_status prefill_impl(bgtq_context *ctx, const bgtq_prefill_desc *d, c
   p.out = d->out;
   // A workspace of the partials alone leaves the operands to each tile's own
   // build, as do books beyond the build's LDS.
-  bool once = prefill_operands_once(d->dim, nn >= 0, (int64_t)d->rows * dp.G);
+  bool once = prefill_operands_once(d->dim, nn >= 0, (int64_t)d->rows * dp.G, plan.tile_queries, plan.work, device_cus());
   for (int h = 0; h < d->kv_heads && d->key_format == BGTQ_KEYS_PACKED; ++h) {
     const DevTables *T = d->tables[h]->h();
     if (T->n_books * T->max_centroids * 4 > prefill_general_book_bytes(d->dim)) once = false;

@@ -244,14 +244,21 @@ constexpr int kPrefillSegmentCost = 4;    // cost units of a tile's set-up (a 32
 // A tiled chunk's K operands built once (prefill_operand_kernel, about 5 us) instead of by every query tile.
 // us per call, once / per tile (MI355X, same outputs bit for bit):
 //   any packed layout, d=128: 33 rows x 4 heads after 2000 tokens 26.5 / 29.2, 1001 rows x 4 after 3077 77 / 343: always;
-//   any packed layout, d=64: from the 256-query tiles on (1001 rows x 3 after 3077: 54.8 / 81.2; 300 rows x 7 after
-//   300: 27.2 / 24.6 structured); with 64-query tiles the build launch costs what it saves (771 queries 30.7 / 31.4,
-//   900 after 300 tokens 21.8 / 19.6);
+//   any packed layout, d=64: with 256-query tiles (1001 rows x 3 heads after 3077 tokens 54.8 / 81.2); with 64-query
+//   tiles from eight cost units per workgroup (SmolLM2 heads, 3 KV heads: 200 rows after 3896 32.9 / 33.7, 600 after 3496
+//   42.9 / 52.3; below it the build launch costs more than it saves, 600 after 0 22.9 / 21.6);
 //   structured layouts build cheaply per tile: d=128 2100 queries 37.9 / 36.5, 4200 73.2 / 76.8, 14336 79.1 / 87.6;
 //   d=64 28672 queries 109.4 / 110.1, 2100 27.2 / 24.6: never.
-__host__ __device__ constexpr bool prefill_operands_once(int dim, bool structured, int64_t queries) {
-  return dim == 128 ? !structured || queries >= 4096 : !structured && queries >= 2048;
+constexpr bool prefill_operands_once(int dim, bool structured, int64_t queries, int tile_queries, int64_t work, int cus) {
+  if (dim == 128) return !structured || queries >= 4096;
+  return !structured && (tile_queries > 64 || work >= 8 * 2 * (int64_t)cus);
 }
+// Cost units of a d=64 launch (256-query tiles) below which its tiles hold 64 queries: with at most 8.5 per workgroup
+// the short tiles' more even ranges, quicker set-up and four waves a SIMD outweigh K streamed four times as often.
+// us, 64- / 256-query tiles: SmolLM2 heads 700 rows after 0 22.8 / 29.4, 1500 after 0 33.3 / 40.0, 1001 after 3095 (4176
+// units) 53.0 / 54.7, 1500 after 2596 (5886) 66.2 / 63.4; layout B x 7 heads 300 after 3796 38.1 / 44.3, 642 after 3454
+// (4392) 58.5 / 55.3, 4096 after 0 149 / 114.
+constexpr int64_t prefill_wide_tile_work(int cus) { return 17 * (int64_t)cus; }
 constexpr size_t kPrefillOperandBytes = (size_t)1 << 30;  // workspace bytes of built operands at most
 constexpr int kPrefillMaxRanges = 2048;   // workgroups of one launch at most (bounds the records)
 // Chunks of at most this many rows run row-wise through the fused decode

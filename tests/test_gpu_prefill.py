@@ -355,8 +355,9 @@ def test_workspace_shared_across_paths(device, oracle):
 
 
 @pytest.mark.parametrize("layout,dim,hq,rows,starts", [
-    ("S", 64, 9, 683, [0, 300]),      # 2049 queries: just past the 256-query tiles' line, odd lengths
-    ("A", 64, 8, 512, [1, 33]),       # 2048 queries, a history one token into a block
+    ("S", 64, 9, 683, [0, 300]),      # 64-query tiles past 2048 queries, odd lengths
+    ("A", 64, 8, 129, [1, 3500]),     # few queries, a history long enough, one starting a token into a block
+    ("S", 64, 9, 1025, [0, 1801]),    # 256-query tiles
     ("A", 128, 2, 65, [0, 158]),      # two 64-query tiles, the smallest launch of this route
     ("A", 128, 8, 513, [31, 64]),
     ("B", 128, 16, 256, [0, 95]),     # a structured layout at its line (4096 queries)
