@@ -28,9 +28,9 @@
 // so the rotated queries are QK operands as they stand and the K operand is
 // gathered in the same order.
 //
-// Per 32-token block each wave rebuilds the K operand from LDS lookup tables
-// of fp16 (hi, lo) centroid splits once per 16-token x 32-dim step and reuses
-// it for its NCB column blocks: QK as 16x16x32 f16 MFMAs (hi*hi + lo*hi +
+// Per 32-token block the K operand (fp16 hi/lo centroid times scale) is built
+// once by the four waves in LDS, or arrives built (prefill_operand_kernel, long
+// chunks), and each wave reuses it for its NCB column blocks: QK as 16x16x32 f16 MFMAs (hi*hi + lo*hi +
 // hi*lo), per-token group scales, the causal mask, an online softmax in the
 // log2 domain and PV as MFMAs with V read transposed (ds_read_b64_tr_b16).
 // A tile inside one range writes its output directly; a tile shared by
