@@ -868,7 +868,9 @@ static int device_cus() {
 // rows 44.2 / 21.9. The thread-per-row encoder of the layouts the tile encoder
 // does not take starts later.
 constexpr int kEncodeTile = 3;  // encoder kind beside encode_bulk_kind's
-static int64_t encode_wave_max_rows(int dim, bool tile) { return !tile ? 16384 : dim == 64 ? 8192 : 4096; }
+// From this many rows a call's jobs go through the context's device table.
+constexpr int64_t kEncodeTableRows = 16384;
+static int64_t encode_wave_max_rows(int dim, bool tile) { return !tile ? kEncodeTableRows : dim == 64 ? 8192 : 4096; }
 // Layout B at d=64 from this many rows: the thread-per-row encoder with the
 // layout's structure at compile time (51 us for 368,640 rows, 57 with the tile
 // encoder; 44 against 41 for 262,144, 20 against 13 for 32,768).
@@ -891,10 +893,13 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
   }
   if (bgtq_status s = ctx->use()) return s;
   // Group jobs by dimension and encoder kind. Few rows in all (a decode
-  // step's appended tokens) go to the wave-per-row encoder, its jobs in kernel
-  // arguments (kEncodeJobsPerLaunch per launch); otherwise one tile or thread-per-row
-  // launch covers up to kEncodeJobTable jobs through the context's job table,
-  // so every job's rows share one grid and one round of workgroups.
+  // step's appended tokens) go to the wave-per-row encoder. Below
+  // kEncodeTableRows rows the jobs travel as kernel arguments
+  // (kEncodeJobsPerLaunch per launch, kTileJobsPerLaunch of the tile encoder),
+  // so such calls share no device memory with other calls on the context;
+  // from there one tile or thread-per-row launch covers up to
+  // kEncodeJobTable jobs through the context's job table, so every job's rows
+  // share one grid and one round of workgroups.
   std::map<std::pair<int, int>, std::vector<size_t>> by_kind;
   for (size_t i = 0; i < n_jobs; ++i)
     if (jobs[i].rows > 0) {
@@ -949,35 +954,64 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
       }
       continue;
     }
+    // A launch's extents: the longest job and the largest tables among its jobs.
+    struct Extents {
+      int64_t rows = 0;
+      int lut = 0, books = 0;
+      EncodeTileSizes tile{};
+      void add(const bgtq_encode_job &j) {
+        const bgtq_tables_info &t = j.tables->info;
+        rows = std::max(rows, j.rows);
+        lut = std::max(lut, t.n_codebooks * 256);
+        books = std::max(books, t.n_books * t.max_centroids);
+        tile.codebooks = std::max(tile.codebooks, t.n_codebooks);
+        tile.groups = std::max(tile.groups, t.groups);
+        tile.row_bytes = std::max(tile.row_bytes, t.row_bytes);
+      }
+      bool tile_fits(int dim) const {
+        return encode_tile_lds_bytes(dim, tile.codebooks, tile.groups, tile.row_bytes) <= 160 * 1024;
+      }
+    };
+    if (tile && total_rows < kEncodeTableRows) {
+      for (size_t b = 0; b < idx.size();) {
+        // Up to kTileJobsPerLaunch jobs whose tables fit the LDS together (any job's alone do).
+        EncodeTileLaunch L{};
+        Extents x;
+        for (; b < idx.size() && L.n_jobs < kTileJobsPerLaunch; ++b) {
+          const bgtq_encode_job &j = jobs[idx[b]];
+          const bgtq_tables_info &t = j.tables->info;
+          Extents with = x;
+          with.add(j);
+          if (!with.tile_fits(dim)) break;
+          x = with;
+          L.jobs[L.n_jobs++] = {j.tables->dev(), j.src, j.packed + j.dst_row0 * t.row_bytes,
+                                j.norms + j.dst_row0 * t.norm_stride, (int32_t)j.src_row_stride, (int32_t)j.rows};
+        }
+        HIP_TRY(launch_encode_tile_args(L, dim, src_f32, x.rows, device_cus(), x.tile, ctx->stream), "encode launch");
+      }
+      continue;
+    }
     EncodeJobDev *table = static_cast<EncodeJobDev *>(ctx->encode_jobs.ptr);
     std::lock_guard<std::mutex> lock(ctx->encode_mutex);
     for (size_t b = 0; b < idx.size(); b += kEncodeJobTable) {
       const size_t e = std::min(idx.size(), b + kEncodeJobTable);
-      int64_t max_rows = 0;
-      int lut_max = 0, books_max = 0, cb_max = 0, groups_max = 0, rb_max = 0;
+      Extents x;
       for (size_t c = b; c < e; c += kEncodeJobsPerLaunch) {
         EncodeLaunch L{};
         for (size_t k = c; k < std::min(e, c + kEncodeJobsPerLaunch); ++k) {
-          const bgtq_encode_job &j = jobs[idx[k]];
-          L.jobs[L.n_jobs++] = job_dev(j);
-          max_rows = std::max(max_rows, j.rows);
-          lut_max = std::max(lut_max, j.tables->info.n_codebooks * 256);
-          books_max = std::max(books_max, j.tables->info.n_books * j.tables->info.max_centroids);
-          cb_max = std::max(cb_max, j.tables->info.n_codebooks);
-          groups_max = std::max(groups_max, j.tables->info.groups);
-          rb_max = std::max(rb_max, j.tables->info.row_bytes);
+          L.jobs[L.n_jobs++] = job_dev(jobs[idx[k]]);
+          x.add(jobs[idx[k]]);
         }
         HIP_TRY(launch_encode_upload(L, table, (int)(c - b), ctx->stream), "encode job upload");
       }
       const int n = (int)(e - b);
-      if (tile && encode_tile_lds_bytes(dim, cb_max, groups_max, rb_max) <= 160 * 1024) {
-        HIP_TRY(launch_encode_tile(table, n, dim, src_f32, max_rows, device_cus(), cb_max, groups_max, rb_max, ctx->stream),
-                "encode launch");
-      } else if (kind == 1 && encode_bulk_lds_bytes(lut_max, books_max) <= 64 * 1024) {
+      if (tile && x.tile_fits(dim)) {
+        HIP_TRY(launch_encode_tile(table, n, dim, src_f32, x.rows, device_cus(), x.tile, ctx->stream), "encode launch");
+      } else if (kind == 1 && encode_bulk_lds_bytes(x.lut, x.books) <= 64 * 1024) {
         // Bulk encodes of layout-B-shaped tables: thread per row, structure at compile time.
-        HIP_TRY(launch_encode_bulk(table, n, src_f32, max_rows, lut_max, books_max, ctx->stream), "encode launch");
+        HIP_TRY(launch_encode_bulk(table, n, src_f32, x.rows, x.lut, x.books, ctx->stream), "encode launch");
       } else {
-        HIP_TRY(launch_encode(table, n, dim, src_f32, max_rows, ctx->stream), "encode launch");
+        HIP_TRY(launch_encode(table, n, dim, src_f32, x.rows, ctx->stream), "encode launch");
       }
     }
   }

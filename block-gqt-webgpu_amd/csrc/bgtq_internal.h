@@ -110,6 +110,28 @@ struct EncodeLaunch {
   int32_t n_jobs;
 };
 
+// The tile encoder's job (packed and norms at its first destination row), and
+// a launch's jobs as kernel arguments (under 4 KB).
+struct EncodeTileJob {
+  const DevTables *t;
+  const void *src;
+  uint8_t *packed;
+  uint16_t *norms;
+  int32_t src_stride;  // elements
+  int32_t rows;        // as a kernel argument (jobs in the device table keep 64 bits)
+};
+static_assert(sizeof(EncodeTileJob) == 40, "tile job layout");
+constexpr int kTileJobsPerLaunch = 100;
+struct EncodeTileLaunch {
+  EncodeTileJob jobs[kTileJobsPerLaunch];
+  int32_t n_jobs;
+};
+static_assert(sizeof(EncodeTileLaunch) + 16 <= 4096, "kernel arguments");
+// The largest codebook count, group count and row bytes among a launch's jobs.
+struct EncodeTileSizes {
+  int codebooks, groups, row_bytes;
+};
+
 // Pointers into global memory typed as such. The compiler knows the address
 // space of pointers it loads from kernel arguments, not of pointers it loads
 // from device memory (the encoders' job table): typed generic, wave-uniform
@@ -387,12 +409,15 @@ hipError_t launch_encode_bulk(const EncodeJobDev *jobs, int n_jobs, int src_f32,
 // cores): whether a table set's layout qualifies (ascending contiguous groups
 // with even boundaries, one centroid book per codebook, its LDS within
 // bounds), the LDS of a launch's largest codebook count, group count and row
-// bytes, and its launcher. Source row strides up to kTileMaxStride elements.
+// bytes, and its launchers: jobs from the device table, or as kernel
+// arguments. Source row strides up to kTileMaxStride elements.
 constexpr int64_t kTileMaxStride = 1 << 24;
 bool encode_tile_layout(const DevTables *T);
 int encode_tile_lds_bytes(int dim, int n_codebooks, int groups, int row_bytes);
 hipError_t launch_encode_tile(const EncodeJobDev *jobs, int n_jobs, int dim, int src_f32, int64_t max_rows, int cus,
-                              int max_codebooks, int max_groups, int max_row_bytes, hipStream_t stream);
+                              const EncodeTileSizes &z, hipStream_t stream);
+hipError_t launch_encode_tile_args(const EncodeTileLaunch &launch, int dim, int src_f32, int64_t max_rows, int cus,
+                                   const EncodeTileSizes &z, hipStream_t stream);
 hipError_t launch_rotate_q(const DecodeParams &p, const float *q, float *qr, hipStream_t stream);
 // Device address of this device's bgtq_decode_noalloc scratch (decode_scratch.hip).
 hipError_t decode_scratch_setup(int device, hipStream_t stream, uint8_t **out);

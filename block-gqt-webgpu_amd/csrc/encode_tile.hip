@@ -98,20 +98,19 @@ __host__ __device__ inline TileLds tile_lds(int n_codebooks, int groups, int row
   return L;
 }
 
+// Waves per SIMD that the register budget leaves room for.
+constexpr int tile_waves_per_simd(int D, bool src_f32) { return D != 64 ? 2 : src_f32 ? 3 : 4; }
+
+// One job: its packed and norms already point at its first destination row.
 template <int D, bool SRC_F32>
-__global__ __launch_bounds__(64 * tile_waves(D), D != 64 ? 2 : SRC_F32 ? 3 : 4) void encode_tile_kernel(
-    const EncodeJobDev *__restrict__ jobs, int max_codebooks, int max_groups, int max_row_bytes) {
+__device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const int64_t rows, int max_codebooks,
+                                                 int max_groups, int max_row_bytes) {
   using S = Tile<D>;
   constexpr int KS = S::KS, NT = S::NT, NV = S::NV, W = tile_waves(D), TH = 64 * W;
   constexpr int kSelRow = NT + (NT == 4 ? 0 : 4);
   extern __shared__ __align__(16) uint8_t smem[];
   const TileLds L = tile_lds<D>(max_codebooks, max_groups, max_row_bytes);
-  struct JobWords {
-    u32x4 w[4];
-  };
-  const BGTQ_CONST u32x4 *jw = to_const<u32x4>(jobs + blockIdx.y);
-  const EncodeJobDev job = __builtin_bit_cast(EncodeJobDev, (JobWords{{jw[0], jw[1], jw[2], jw[3]}}));
-  const int64_t n_blocks = (job.rows + kTileRows - 1) / kTileRows;
+  const int64_t n_blocks = (rows + kTileRows - 1) / kTileRows;
   if ((int64_t)blockIdx.x * W >= n_blocks) return;  // uniform for the workgroup
   const BGTQ_CONST DevTables *T = to_const<DevTables>(job.t);
   const int tid = threadIdx.x, lane = tid & 63, gq = lane >> 4, col = lane & 15;
@@ -123,7 +122,7 @@ __global__ __launch_bounds__(64 * tile_waves(D), D != 64 ? 2 : SRC_F32 ? 3 : 4) 
   uint8_t *const wv = smem + L.wave + wave * L.stride;
   // The image of a block's packed rows starts at the destination's byte in
   // its word (the same for every block: 16 rows are whole words).
-  const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(job.packed) + (uint64_t)job.dst_row0 * (uint64_t)RB) & 3u;
+  const uint32_t mis = (uint32_t)reinterpret_cast<uintptr_t>(job.packed) & 3u;
 
   // A quarter of row col of block b per lane, in 16-byte pieces where the
   // source allows, through a buffer range that ends with the job's last row
@@ -133,7 +132,7 @@ __global__ __launch_bounds__(64 * tile_waves(D), D != 64 ? 2 : SRC_F32 ? 3 : 4) 
   const bool vec = reinterpret_cast<uintptr_t>(job.src) % 16 == 0 && (job.src_stride * kElem) % 16 == 0;  // uniform
   u32x4 raw[NP];
   auto load_rows = [&](int64_t b, int gq, int col) {
-    const int nr = (int)min((int64_t)kTileRows, job.rows - b * kTileRows);
+    const int nr = (int)min((int64_t)kTileRows, rows - b * kTileRows);
     const uint8_t *base = static_cast<const uint8_t *>(job.src) + b * kTileRows * (int64_t)job.src_stride * kElem;
     const __amdgpu_buffer_rsrc_t r =
         rsrc(nr > 0 ? base : job.src, nr > 0 ? (uint32_t)((nr - 1) * job.src_stride + D) * kElem : 0u);
@@ -400,8 +399,8 @@ __global__ __launch_bounds__(64 * tile_waves(D), D != 64 ? 2 : SRC_F32 ? 3 : 4) 
     }
     // production_math.py:20-23: corrected_g = raw_g / max(sqrt(sum c^2), 1e-10).
     const int64_t row0 = b * kTileRows;
-    const int nr = (int)min((int64_t)kTileRows, job.rows - row0);
-    BGTQ_GLOBAL uint16_t *nrow = to_global(job.norms) + (job.dst_row0 + row0 + col) * NS;
+    const int nr = (int)min((int64_t)kTileRows, rows - row0);
+    BGTQ_GLOBAL uint16_t *nrow = to_global(job.norms) + (row0 + col) * NS;
     for (int h = 0; h < ngb; ++h) {
       const int g = gq + 4 * h;
       const float c = fmaxf(__builtin_sqrtf(tree_sum(h, [&](int s) { return c2[s]; })), 1e-10f);
@@ -413,7 +412,7 @@ __global__ __launch_bounds__(64 * tile_waves(D), D != 64 ? 2 : SRC_F32 ? 3 : 4) 
     wave_sync();
     // The image to the destination: whole words, then the bytes of the first
     // and last word when they are not whole.
-    uint8_t *dst = job.packed + (job.dst_row0 + row0) * RB - mis;
+    uint8_t *dst = job.packed + row0 * RB - mis;
     const int e1 = (int)mis + nr * RB, w0 = mis ? 1 : 0, w1 = e1 / 4;
     for (int w = w0 + lane; w < w1; w += 64)
       *reinterpret_cast<BGTQ_GLOBAL uint32_t *>(to_global(dst) + 4 * w) = reinterpret_cast<const uint32_t *>(wv)[w];
@@ -425,27 +424,68 @@ __global__ __launch_bounds__(64 * tile_waves(D), D != 64 ? 2 : SRC_F32 ? 3 : 4) 
   }
 }
 
-template <int D>
-hipError_t launch_d(const EncodeJobDev *jobs, int n_jobs, int src_f32, int wgs, int max_codebooks, int max_groups,
-                    int max_row_bytes, hipStream_t stream) {
-  const int lds = tile_lds<D>(max_codebooks, max_groups, max_row_bytes).total;
-  const dim3 grid((unsigned)wgs, (unsigned)n_jobs), wg(64 * tile_waves(D));
-  hipError_t e;
-  if (src_f32) {
-    static const hipError_t ok = hipFuncSetAttribute((const void *)encode_tile_kernel<D, true>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
-    if ((e = ok) == hipSuccess)
-      hipLaunchKernelGGL((encode_tile_kernel<D, true>), grid, wg, lds, stream, jobs, max_codebooks, max_groups,
-                         max_row_bytes);
-  } else {
-    static const hipError_t ok = hipFuncSetAttribute((const void *)encode_tile_kernel<D, false>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
-    if ((e = ok) == hipSuccess)
-      hipLaunchKernelGGL((encode_tile_kernel<D, false>), grid, wg, lds, stream, jobs, max_codebooks, max_groups,
-                         max_row_bytes);
+// Jobs from the context's device table, one per grid y.
+template <int D, bool SRC_F32>
+__global__ __launch_bounds__(64 * tile_waves(D), tile_waves_per_simd(D, SRC_F32)) void encode_tile_kernel(
+    const EncodeJobDev *__restrict__ jobs, int max_codebooks, int max_groups, int max_row_bytes) {
+  struct JobWords {
+    u32x4 w[4];
+  };
+  const BGTQ_CONST u32x4 *jw = to_const<u32x4>(jobs + blockIdx.y);
+  const EncodeJobDev j = __builtin_bit_cast(EncodeJobDev, (JobWords{{jw[0], jw[1], jw[2], jw[3]}}));
+  const BGTQ_CONST DevTables *T = to_const<DevTables>(j.t);
+  const EncodeTileJob job{j.t, j.src, j.packed + j.dst_row0 * T->row_bytes, j.norms + j.dst_row0 * T->norm_stride,
+                          j.src_stride, 0};
+  encode_tile_body<D, SRC_F32>(job, j.rows, max_codebooks, max_groups, max_row_bytes);
+}
+
+// Jobs from the kernel's arguments: small calls share no device memory with
+// other calls on the context, and take no upload launch.
+template <int D, bool SRC_F32>
+__global__ __launch_bounds__(64 * tile_waves(D), tile_waves_per_simd(D, SRC_F32)) void encode_tile_args_kernel(
+    EncodeTileLaunch launch, int max_codebooks, int max_groups, int max_row_bytes) {
+  const EncodeTileJob job = launch.jobs[blockIdx.y];
+  encode_tile_body<D, SRC_F32>(job, job.rows, max_codebooks, max_groups, max_row_bytes);
+}
+
+template <typename K, typename J>
+hipError_t launch_k(K kernel, const hipError_t allowed, const dim3 grid, int threads, int lds, hipStream_t stream,
+                    const J &jobs, const EncodeTileSizes &z) {
+  if (allowed != hipSuccess) {
+    (void)hipGetLastError();
+    return allowed;
   }
-  const hipError_t last = hipGetLastError();
-  return e != hipSuccess ? e : last;
+  hipLaunchKernelGGL(kernel, grid, dim3((unsigned)threads), lds, stream, jobs, z.codebooks, z.groups, z.row_bytes);
+  return hipGetLastError();
+}
+
+template <int D, bool SRC_F32>
+hipError_t launch_d(const EncodeJobDev *table, const EncodeTileLaunch *args, const dim3 grid, const EncodeTileSizes &z,
+                    hipStream_t stream) {
+  const int lds = tile_lds<D>(z.codebooks, z.groups, z.row_bytes).total, threads = 64 * tile_waves(D);
+  if (table) {
+    static const hipError_t ok = hipFuncSetAttribute((const void *)encode_tile_kernel<D, SRC_F32>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
+    return launch_k(encode_tile_kernel<D, SRC_F32>, ok, grid, threads, lds, stream, table, z);
+  }
+  static const hipError_t ok = hipFuncSetAttribute((const void *)encode_tile_args_kernel<D, SRC_F32>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kLdsLimit);
+  return launch_k(encode_tile_args_kernel<D, SRC_F32>, ok, grid, threads, lds, stream, *args, z);
+}
+
+// One round of workgroups (as many waves per SIMD as their registers allow, as far as the LDS holds
+// them) shared by the jobs, rounded down: a few more than fit take a second
+// round as long as the first. A wave walks its job's blocks with that stride.
+hipError_t launch_any(const EncodeJobDev *table, const EncodeTileLaunch *args, int n_jobs, int dim, int src_f32,
+                      int64_t max_rows, int cus, const EncodeTileSizes &z, hipStream_t stream) {
+  const int waves = tile_waves(dim), lds = encode_tile_lds_bytes(dim, z.codebooks, z.groups, z.row_bytes);
+  const int fit = std::min(4 * tile_waves_per_simd(dim, src_f32) / waves, kLdsLimit / lds);
+  const int64_t resident = (int64_t)cus * std::max(1, fit);
+  const int64_t blocks = (max_rows + kTileRows - 1) / kTileRows, most = (blocks + waves - 1) / waves;
+  const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(most, resident / n_jobs)), (unsigned)n_jobs);
+  if (dim == 64)
+    return src_f32 ? launch_d<64, true>(table, args, grid, z, stream) : launch_d<64, false>(table, args, grid, z, stream);
+  return src_f32 ? launch_d<128, true>(table, args, grid, z, stream) : launch_d<128, false>(table, args, grid, z, stream);
 }
 
 }  // namespace
@@ -471,17 +511,13 @@ int encode_tile_lds_bytes(int dim, int n_codebooks, int groups, int row_bytes) {
 }
 
 hipError_t launch_encode_tile(const EncodeJobDev *jobs, int n_jobs, int dim, int src_f32, int64_t max_rows, int cus,
-                              int max_codebooks, int max_groups, int max_row_bytes, hipStream_t stream) {
-  // One round of workgroups (as many waves per SIMD as their registers allow, as far as the LDS holds
-  // them) shared by the jobs, rounded down: a few more than fit take a second
-  // round as long as the first. A wave walks its job's blocks with that stride.
-  const int waves = tile_waves(dim), lds = encode_tile_lds_bytes(dim, max_codebooks, max_groups, max_row_bytes);
-  const int64_t resident = (int64_t)cus * std::max(1, std::min((dim != 64 ? 8 : src_f32 ? 12 : 16) / waves, kLdsLimit / lds));
-  const int64_t blocks = (max_rows + kTileRows - 1) / kTileRows, most = (blocks + waves - 1) / waves;
-  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(most, resident / n_jobs));
-  if (dim == 64)
-    return launch_d<64>(jobs, n_jobs, src_f32, (int)wgs, max_codebooks, max_groups, max_row_bytes, stream);
-  return launch_d<128>(jobs, n_jobs, src_f32, (int)wgs, max_codebooks, max_groups, max_row_bytes, stream);
+                              const EncodeTileSizes &z, hipStream_t stream) {
+  return launch_any(jobs, nullptr, n_jobs, dim, src_f32, max_rows, cus, z, stream);
+}
+
+hipError_t launch_encode_tile_args(const EncodeTileLaunch &launch, int dim, int src_f32, int64_t max_rows, int cus,
+                                   const EncodeTileSizes &z, hipStream_t stream) {
+  return launch_any(nullptr, &launch, launch.n_jobs, dim, src_f32, max_rows, cus, z, stream);
 }
 
 }  // namespace bgtq

@@ -433,6 +433,58 @@ def test_job_table_batches_and_stream_switch(device, oracle):
         tables.destroy()
 
 
+@pytest.mark.parametrize("dim,rows,heads", [(64, 3333, 3), (64, 100, 130), (128, 2048, 5)])
+def test_small_encode_shares_no_table(device, oracle, dim, rows, heads):
+    """A call below 16384 rows carries its jobs in kernel arguments (more jobs than one launch holds,
+    several launches): its captured graph replays on another stream while the same context encodes
+    eagerly through the device job table, and both keep giving the oracle's bytes."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    rng = np.random.default_rng(11)
+    p = calibrate.layout_a(dim)
+    small, large = heads * rows, 17000
+    assert small < 16384
+    k, kl = _random_half_rows(rng, small, dim), _random_half_rows(rng, large, dim)
+    tables = bgtq.Tables(device, p)
+    side, main = torch.cuda.Stream(), torch.cuda.Stream()
+    try:
+        def buffers(x):
+            return (torch.from_numpy(x.view(np.int16)).cuda(),
+                    torch.zeros((len(x), p.rowBytes), dtype=torch.uint8, device="cuda"),
+                    torch.zeros((len(x), p.normStride), dtype=torch.int16, device="cuda"))
+
+        def jobs(b, n, r):
+            return [dict(tables=tables, src=b[0][i * r:], src_row_stride=dim, rows=r, packed=b[1][i * r:],
+                         norms=b[2][i * r:]) for i in range(n)]
+
+        bs, bl = buffers(k), buffers(kl)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            device.set_stream(torch.cuda.current_stream().cuda_stream)
+            batched.encode(device, jobs(bs, heads, rows), "f16")
+        device.set_stream(main.cuda_stream)
+        ref = [oracle.encode_pack(_olayout(oracle, p), x) for x in (k, kl)]
+        for trial in range(6):
+            print("replay", dim, heads, trial, flush=True)
+            for t in (*bs[1:], *bl[1:]):
+                t.zero_()
+            torch.cuda.synchronize()
+            for _ in range(4):
+                with torch.cuda.stream(side):
+                    graph.replay()
+                batched.encode(device, jobs(bl, 17, large // 17), "f16")
+            torch.cuda.synchronize()
+            for (rp, rn), b in zip(ref, (bs, bl)):
+                assert np.array_equal(b[1].cpu().numpy(), rp)
+                assert np.array_equal(b[2].cpu().numpy().view(np.uint16), rn)
+    finally:
+        torch.cuda.synchronize()
+        device.set_stream(None)
+        tables.destroy()
+
+
 def test_concurrent_appends_near_capacity(device, oracle):
     """Two threads append at once near the end of a store's capacity (the Node addon runs appends off
     the JS thread). The store is claimed before the capacity check, as the reference refuses a second
