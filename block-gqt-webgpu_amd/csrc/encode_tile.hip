@@ -101,8 +101,29 @@ __host__ __device__ inline TileLds tile_lds(int n_codebooks, int groups, int row
 // Waves per SIMD that the register budget leaves room for.
 constexpr int tile_waves_per_simd(int D, bool src_f32) { return D != 64 ? 2 : src_f32 ? 3 : 4; }
 
+// Whether positions [lo, hi) of a row's position mask hold any set bit.
+template <int D>
+__device__ __forceinline__ bool any_in(const uint64_t (&m)[D / 64], int lo, int hi) {
+  bool any = false;
+#pragma unroll
+  for (int w = 0; w < D / 64; ++w) {
+    const int a = max(lo - 64 * w, 0), b = min(hi - 64 * w, 64);
+    if (a < b) any |= (m[w] >> a << (64 - (b - a))) != 0;
+  }
+  return any;
+}
+
 // One job: its packed and norms already point at its first destination row.
-template <int D, bool SRC_F32>
+//
+// Rows with infinities or NaNs come out as the other encoders give them. The
+// products with 0/1 masks above would spread such a value over every group
+// (0 inf = NaN); a block of rows that holds one (wave-uniform test) zeroes
+// it and keeps per row and group: raw_g (an infinity, or NaN), and whether
+// the group's y are NaN (bin 0), which they are when the FMA chain meets a
+// non-finite input. The chain runs over the 8-wide blocks that touch the
+// group (encode.hip; whole groups in encode_bulk.hip), or with WHOLE_ROWS
+// over the row (the wave encoder, which takes the smaller calls).
+template <int D, bool SRC_F32, bool WHOLE_ROWS>
 __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const int64_t rows, int max_codebooks,
                                                  int max_groups, int max_row_bytes) {
   using S = Tile<D>;
@@ -286,6 +307,7 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
 
     // The rows to LDS in natural order, the next block's loads, then this
     // lane's positions.
+    uint32_t nonfinite = 0;  // bits 15, 31: an exponent of all ones carried out
 #pragma unroll
     for (int k = 0; k < KS / 4; ++k) {
       u32x2 v;
@@ -300,7 +322,10 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
         v = u32x2{raw[k / 2][2 * (k % 2)], raw[k / 2][2 * (k % 2) + 1]};
       }
       *reinterpret_cast<u32x2 *>(wv + col * S::XROW + 2 * KS * gq + 8 * k) = v;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) nonfinite |= (v[h] & 0x7c007c00u) + 0x04000400u;
     }
+    const bool odd_rows = __builtin_amdgcn_ballot_w64((nonfinite & 0x80008000u) != 0) != 0;
     load_rows(b + (int64_t)gridDim.x * W, gq, col);  // in flight meanwhile
     wave_sync();
     const u32x4 *so = reinterpret_cast<const u32x4 *>(smem + L.src + gq * S::MROW * 4);
@@ -308,6 +333,27 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       x[s] = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(wv + col * S::XROW + (so[s / 4][s % 4] & 0xffffu)));
+    // Per group g of the row: bit g an infinity, 8 + g a NaN among its inputs, 16 + g its y are NaN.
+    uint32_t odd = 0;
+    if (odd_rows) {
+      uint64_t inf[D / 64] = {}, nan[D / 64] = {};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        auto row_bits = [&](bool c) {  // position 4 s + q of row col is lane 16 q + col's
+          const uint64_t b = __builtin_amdgcn_ballot_w64(c) >> col;
+          return ((b & 1) | (b >> 15 & 2) | (b >> 30 & 4) | (b >> 45 & 8)) << (4 * (s % 16));
+        };
+        inf[s / 16] |= row_bits(__builtin_fabsf(x[s]) == INFINITY);
+        nan[s / 16] |= row_bits(x[s] != x[s]);
+        x[s] = __builtin_fabsf(x[s]) < INFINITY ? x[s] : 0.0f;
+      }
+      for (int g = 0; g < ng; ++g) {
+        const int g0 = T->gstart[g], g1 = T->gend[g];
+        const int c0 = WHOLE_ROWS ? 0 : g0 & ~7, c1 = WHOLE_ROWS ? D : (g1 + 7) & ~7;
+        odd |= (uint32_t)any_in<D>(inf, g0, g1) << g | (uint32_t)any_in<D>(nan, g0, g1) << (8 + g) |
+               (uint32_t)(any_in<D>(inf, c0, c1) || any_in<D>(nan, c0, c1)) << (16 + g);
+      }
+    }
     // production_math.py:12-15 for the row's groups gq and gq + 4: n_g,
     // raw_g = sum(n_g over the group)/|g|; then every position's divisor and
     // its reciprocal.
@@ -343,6 +389,7 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
         }
         rg = t / (float)T->gsize[g];
       }
+      if (odd_rows) rg = odd >> (8 + g) & 1 ? __builtin_nanf("") : odd >> g & 1 ? INFINITY : rg;
       raw_g[0] = h == 0 ? rg : raw_g[0];
       raw_g[1] = h == 0 ? raw_g[1] : rg;
       const float dg = n > 1e-10f ? n : 1.0f, rd = 1.0f / dg;
@@ -367,6 +414,11 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       f32x4 y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (odd_rows) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (odd >> (16 + Tg[offsetof(DevTables, group_of) + 16 * t + 4 * r + gq]) & 1) y[r] = __builtin_nanf("");
+      }
 #pragma unroll
       for (int q = 0; q < NT; ++q) {
         if (q < qlo[t] || q > qhi[t]) continue;  // uniform
@@ -436,7 +488,7 @@ __global__ __launch_bounds__(64 * tile_waves(D), tile_waves_per_simd(D, SRC_F32)
   const BGTQ_CONST DevTables *T = to_const<DevTables>(j.t);
   const EncodeTileJob job{j.t, j.src, j.packed + j.dst_row0 * T->row_bytes, j.norms + j.dst_row0 * T->norm_stride,
                           j.src_stride, 0};
-  encode_tile_body<D, SRC_F32>(job, j.rows, max_codebooks, max_groups, max_row_bytes);
+  encode_tile_body<D, SRC_F32, false>(job, j.rows, max_codebooks, max_groups, max_row_bytes);
 }
 
 // Jobs from the kernel's arguments: small calls share no device memory with
@@ -445,7 +497,7 @@ template <int D, bool SRC_F32>
 __global__ __launch_bounds__(64 * tile_waves(D), tile_waves_per_simd(D, SRC_F32)) void encode_tile_args_kernel(
     EncodeTileLaunch launch, int max_codebooks, int max_groups, int max_row_bytes) {
   const EncodeTileJob job = launch.jobs[blockIdx.y];
-  encode_tile_body<D, SRC_F32>(job, job.rows, max_codebooks, max_groups, max_row_bytes);
+  encode_tile_body<D, SRC_F32, true>(job, job.rows, max_codebooks, max_groups, max_row_bytes);
 }
 
 template <typename K, typename J>

@@ -324,6 +324,91 @@ def test_tile_encoder_bit_exact(device, oracle, dim, layouts, src_kind):
             t.destroy()
 
 
+def _tree_sum(v):
+    """ATen's FP32 inner sum of one row (d 64 or 128): 8 lanes of four interleaved accumulators."""
+    total = np.float32(0)
+    for lane in range(8):
+        a = [np.float32(0)] * 4
+        for i, x in enumerate(v[lane::8]):
+            a[i % 4] = np.float32(a[i % 4] + x)
+        part = np.float32(np.float32(np.float32(a[0] + a[1]) + a[2]) + a[3])
+        total = np.float32(total + part)
+    return total
+
+
+def _encode_nonfinite(oracle, p, k, whole_rows):
+    """Packed rows and scales of FP16 rows that may hold infinities and NaNs. A group that holds one has
+    the scale inf or NaN over its centroids, and a group whose FMA chain (the 8-wide blocks it touches,
+    or the whole row) meets one has every code at bin 0; all else is as with zeros in their place."""
+    x = k.view(np.float16)
+    clean = np.where(np.isfinite(x), x, np.float16(0))
+    ref_p, ref_n = oracle.encode_pack(_olayout(oracle, p), np.ascontiguousarray(clean).view(np.uint16))
+    ref_p, ref_n = ref_p.copy(), ref_n.copy()
+    perm, group_of = np.asarray(p.permutation), np.asarray(p.groupOf)
+    bin0 = np.asarray(p.codeLut).reshape(-1, 256)[np.asarray(p.positionToCodebook), 0]
+    cent = np.asarray(p.centroids, np.float32).reshape(p.dim, -1)
+    for r in np.nonzero(~np.isfinite(x).all(axis=1))[0]:
+        v, z = x[r, perm].astype(np.float32), clean[r, perm].astype(np.float32)
+        bad = ~np.isfinite(v)
+        nib = p.nibbleDims
+        codes = np.r_[np.stack([ref_p[r, :nib // 2] & 15, ref_p[r, :nib // 2] >> 4], 1).ravel(),
+                      ref_p[r, nib // 2:nib // 2 + p.dim - nib]]
+        for g in range(p.groups):
+            at = np.nonzero(group_of == g)[0]
+            span = slice(None) if whole_rows else slice(at[0] // 8 * 8, (at[-1] + 8) // 8 * 8)
+            if bad[span].any():
+                codes[at] = bin0[at]
+        for g in range(p.groups):
+            own = group_of == g
+            n = np.sqrt(np.float32(_tree_sum(np.where(own, z * z, np.float32(0))) + np.float32(1e-30)))
+            raw = np.float32(_tree_sum(np.where(own, n, np.float32(0))) / np.float32(own.sum())) if p.groups > 1 else n
+            if bad[own].any():
+                raw = np.float32(np.nan if np.isnan(v[own]).any() else np.inf)
+            c = cent[np.arange(p.dim), codes]
+            s = np.sqrt(_tree_sum(np.where(own, c * c, np.float32(0))))
+            ref_n[r, g] = np.float16(raw / max(s, np.float32(1e-10))).view(np.uint16)
+        ref_p[r, :nib // 2] = codes[0:nib:2] | codes[1:nib:2] << 4
+        ref_p[r, nib // 2:nib // 2 + p.dim - nib] = codes[nib:]
+    return ref_p, ref_n
+
+
+@pytest.mark.parametrize("dim,name", [(64, "B"), (64, "A"), (64, "mixed_d64"), (64, "smollm2_h0"), (64, "smollm2_h17"),
+                                      (128, "B"), (128, "A"), (128, "mixed_d128")])
+def test_nonfinite_rows_keep_to_their_groups(device, oracle, dim, name):
+    """Infinities (an FP32 value above 65504 is one) and NaNs among the rows of a tile-encoder call: the
+    other rows and the row's other groups are as without them, in calls below and from 16384 rows."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    p = dict(_layouts(oracle), B=calibrate.layout_b(dim), A=calibrate.layout_a(dim))[name]
+    rng = np.random.default_rng(dim)
+    tables = bgtq.Tables(device, p)
+    try:
+        for rows in (9001, 16400):
+            k = _random_half_rows(rng, rows, dim)
+            f = k.view(np.float16)
+            for r in rng.choice(rows, 60, replace=False):
+                for c in rng.choice(dim, rng.choice([1, 1, 2, dim // 3]), replace=False):
+                    f[r, c] = rng.choice(np.array([np.inf, -np.inf, np.nan], np.float16))
+            f[37, :] = np.inf
+            ref_p, ref_n = _encode_nonfinite(oracle, p, k, rows < 16384)
+            for src_kind in ("f16", "f32"):
+                x = f.astype(np.float32)
+                x = np.where(np.isinf(x), np.copysign(np.float32(70000), x), x)
+                src = torch.from_numpy(f if src_kind == "f16" else x).cuda()
+                packed = torch.zeros((rows, p.rowBytes), dtype=torch.uint8, device="cuda")
+                norms = torch.zeros((rows, p.normStride), dtype=torch.int16, device="cuda")
+                batched.encode(device, [dict(tables=tables, src=src, src_row_stride=dim, rows=rows, packed=packed,
+                                             norms=norms)], src_kind)
+                device.synchronize()
+                got_p, got_n = packed.cpu().numpy(), norms.cpu().numpy().view(np.uint16)
+                same = (got_n == ref_n) | (np.isnan(got_n.view(np.float16)) & np.isnan(ref_n.view(np.float16)))
+                bad = np.nonzero(np.any(got_p != ref_p, axis=1) | ~same.all(axis=1))[0]
+                assert bad.size == 0, f"{rows} rows {src_kind}: {bad.size} differ, first {bad[:5]}"
+    finally:
+        tables.destroy()
+
+
 def test_bulk_layout_b_largest_calls(device, oracle):
     """Layout B at d=64 from 300,000 rows a call: the thread-per-row encoder with the layout's structure
     compiled in, FP16 and FP32 sources, a partial last workgroup."""
