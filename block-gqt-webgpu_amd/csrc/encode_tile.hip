@@ -101,28 +101,15 @@ __host__ __device__ inline TileLds tile_lds(int n_codebooks, int groups, int row
 // Waves per SIMD that the register budget leaves room for.
 constexpr int tile_waves_per_simd(int D, bool src_f32) { return D != 64 ? 2 : src_f32 ? 3 : 4; }
 
-// Whether positions [lo, hi) of a row's position mask hold any set bit.
-template <int D>
-__device__ __forceinline__ bool any_in(const uint64_t (&m)[D / 64], int lo, int hi) {
-  bool any = false;
-#pragma unroll
-  for (int w = 0; w < D / 64; ++w) {
-    const int a = max(lo - 64 * w, 0), b = min(hi - 64 * w, 64);
-    if (a < b) any |= (m[w] >> a << (64 - (b - a))) != 0;
-  }
-  return any;
-}
-
 // One job: its packed and norms already point at its first destination row.
 //
-// Rows with infinities or NaNs come out as the other encoders give them. The
-// products with 0/1 masks above would spread such a value over every group
-// (0 inf = NaN); a block of rows that holds one (wave-uniform test) zeroes
-// it and keeps per row and group: raw_g (an infinity, or NaN), and whether
-// the group's y are NaN (bin 0), which they are when the FMA chain meets a
-// non-finite input. The chain runs over the 8-wide blocks that touch the
-// group (encode.hip; whole groups in encode_bulk.hip), or with WHOLE_ROWS
-// over the row (the wave encoder, which takes the smaller calls).
+// The products with 0/1 masks below spread an infinity or a NaN over every
+// group of its row (0 inf = NaN). A wave that met one encodes those of its
+// blocks again after its loop, with selects, as the other encoders do: a
+// group's norm takes its own inputs, and its y are NaN (bin 0) when their FMA
+// chain meets a non-finite input. The chain runs over the 8-wide blocks that
+// touch the group (encode.hip; whole groups in encode_bulk.hip), or with
+// WHOLE_ROWS over the row (the wave encoder, for smaller calls).
 template <int D, bool SRC_F32, bool WHOLE_ROWS>
 __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const int64_t rows, int max_codebooks,
                                                  int max_groups, int max_row_bytes) {
@@ -174,8 +161,32 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
       }
     }
   };
-  int64_t b = (int64_t)blockIdx.x * W + wave;
-  load_rows(b, gq, col);
+  // The loaded rows to LDS as FP16, in natural order; the lanes whose part
+  // holds an infinity or a NaN (FP16 squares sum to at most 3e11).
+  auto stage_rows = [&](int gq, int col) {
+    float squares = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KS / 4; ++k) {
+      uint32_t v[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int c = 4 * k + 2 * h;
+        if (SRC_F32)
+          v[h] = (uint32_t)f32_to_f16_bits(__uint_as_float(raw[c / 4][c % 4])) |
+                 (uint32_t)f32_to_f16_bits(__uint_as_float(raw[c / 4][c % 4 + 1])) << 16;
+        else
+          v[h] = raw[k / 2][2 * (k % 2) + h];
+        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+        const half2_t x = __builtin_bit_cast(half2_t, v[h]);
+        squares = __builtin_amdgcn_fdot2(x, x, squares, false);
+      }
+      *reinterpret_cast<u32x2 *>(wv + col * S::XROW + 2 * KS * gq + 8 * k) = u32x2{v[0], v[1]};
+    }
+    return __builtin_amdgcn_ballot_w64(!(squares < INFINITY));
+  };
+  uint64_t odd_seen = 0;
+  const int64_t b_first = (int64_t)blockIdx.x * W + wave;
+  load_rows(b_first, gq, col);
 
   // ---- the workgroup's tables ----
   const uint8_t *Tg = reinterpret_cast<const uint8_t *>(job.t);
@@ -264,7 +275,7 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
     sw16(0, 1);
     sw16(2, 3);
   };
-  for (; b < n_blocks; b += (int64_t)gridDim.x * W) {
+  for (int64_t b = b_first; b < n_blocks; b += (int64_t)gridDim.x * W) {
     // The lane index through an opaque copy: offsets derived from it are
     // recomputed where they are used instead of being held in registers
     // across the loop (which spilled: 45 registers at four waves per SIMD).
@@ -307,25 +318,7 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
 
     // The rows to LDS in natural order, the next block's loads, then this
     // lane's positions.
-    uint32_t nonfinite = 0;  // bits 15, 31: an exponent of all ones carried out
-#pragma unroll
-    for (int k = 0; k < KS / 4; ++k) {
-      u32x2 v;
-      if (SRC_F32) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int c = 4 * k + 2 * h;
-          v[h] = (uint32_t)f32_to_f16_bits(__uint_as_float(raw[c / 4][c % 4])) |
-                 (uint32_t)f32_to_f16_bits(__uint_as_float(raw[c / 4][c % 4 + 1])) << 16;
-        }
-      } else {
-        v = u32x2{raw[k / 2][2 * (k % 2)], raw[k / 2][2 * (k % 2) + 1]};
-      }
-      *reinterpret_cast<u32x2 *>(wv + col * S::XROW + 2 * KS * gq + 8 * k) = v;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) nonfinite |= (v[h] & 0x7c007c00u) + 0x04000400u;
-    }
-    const bool odd_rows = __builtin_amdgcn_ballot_w64((nonfinite & 0x80008000u) != 0) != 0;
+    odd_seen |= stage_rows(gq, col);
     load_rows(b + (int64_t)gridDim.x * W, gq, col);  // in flight meanwhile
     wave_sync();
     const u32x4 *so = reinterpret_cast<const u32x4 *>(smem + L.src + gq * S::MROW * 4);
@@ -333,27 +326,6 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       x[s] = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(wv + col * S::XROW + (so[s / 4][s % 4] & 0xffffu)));
-    // Per group g of the row: bit g an infinity, 8 + g a NaN among its inputs, 16 + g its y are NaN.
-    uint32_t odd = 0;
-    if (odd_rows) {
-      uint64_t inf[D / 64] = {}, nan[D / 64] = {};
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        auto row_bits = [&](bool c) {  // position 4 s + q of row col is lane 16 q + col's
-          const uint64_t b = __builtin_amdgcn_ballot_w64(c) >> col;
-          return ((b & 1) | (b >> 15 & 2) | (b >> 30 & 4) | (b >> 45 & 8)) << (4 * (s % 16));
-        };
-        inf[s / 16] |= row_bits(__builtin_fabsf(x[s]) == INFINITY);
-        nan[s / 16] |= row_bits(x[s] != x[s]);
-        x[s] = __builtin_fabsf(x[s]) < INFINITY ? x[s] : 0.0f;
-      }
-      for (int g = 0; g < ng; ++g) {
-        const int g0 = T->gstart[g], g1 = T->gend[g];
-        const int c0 = WHOLE_ROWS ? 0 : g0 & ~7, c1 = WHOLE_ROWS ? D : (g1 + 7) & ~7;
-        odd |= (uint32_t)any_in<D>(inf, g0, g1) << g | (uint32_t)any_in<D>(nan, g0, g1) << (8 + g) |
-               (uint32_t)(any_in<D>(inf, c0, c1) || any_in<D>(nan, c0, c1)) << (16 + g);
-      }
-    }
     // production_math.py:12-15 for the row's groups gq and gq + 4: n_g,
     // raw_g = sum(n_g over the group)/|g|; then every position's divisor and
     // its reciprocal.
@@ -389,7 +361,6 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
         }
         rg = t / (float)T->gsize[g];
       }
-      if (odd_rows) rg = odd >> (8 + g) & 1 ? __builtin_nanf("") : odd >> g & 1 ? INFINITY : rg;
       raw_g[0] = h == 0 ? rg : raw_g[0];
       raw_g[1] = h == 0 ? raw_g[1] : rg;
       const float dg = n > 1e-10f ? n : 1.0f, rd = 1.0f / dg;
@@ -414,11 +385,6 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       f32x4 y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (odd_rows) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (odd >> (16 + Tg[offsetof(DevTables, group_of) + 16 * t + 4 * r + gq]) & 1) y[r] = __builtin_nanf("");
-      }
 #pragma unroll
       for (int q = 0; q < NT; ++q) {
         if (q < qlo[t] || q > qhi[t]) continue;  // uniform
@@ -473,6 +439,89 @@ __device__ __forceinline__ void encode_tile_body(const EncodeTileJob &job, const
       if (lane < 4 ? mis && o >= (int)mis && o < e1 : lane < 8 && o < e1 && (w1 > 0 || !mis)) to_global(dst)[o] = wv[o];
     }
     wave_sync();  // the rows' LDS is rewritten by the next block
+  }
+  if (odd_seen == 0) return;
+
+  // The blocks that hold infinities or NaNs once more, from their staged
+  // rows: lane (gq, col) takes positions 4 s + gq of row col as above, so
+  // columns gq and 4 + gq of the sum tree. Rolled loops: it is rare.
+  wait_vm<0>();  // the stores below come after the loop's
+  int odd_lane = lane_id();
+  asm volatile("" : "+v"(odd_lane));  // (not held across the loop above)
+  for (int64_t b = b_first; b < n_blocks; b += (int64_t)gridDim.x * W) {
+    const int gq = odd_lane >> 4, col = odd_lane & 15;
+    load_rows(b, gq, col);
+    const uint64_t odd = stage_rows(gq, col);
+    wave_sync();
+    auto input = [&](int p) {
+      return f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(wv + col * S::XROW + 2 * (int)T->perm[p]));
+    };
+    // The tree's sum of leaf(p) over the positions p of [g0, g1).
+    auto tree = [&](int g0, int g1, auto leaf) {
+      float part[2];
+#pragma clang loop unroll(disable)
+      for (int h = 0; h < 2; ++h) {
+        float t = 0.0f;
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < 4; ++k) {
+          float a = 0.0f;
+#pragma clang loop unroll(disable)
+          for (int v = k; v < NV; v += 4) {
+            const int p = 8 * v + 4 * h + gq;
+            const bool in = p >= g0 && p < g1;
+            if (__builtin_amdgcn_ballot_w64(in) == 0) continue;
+            const float x = leaf(p, in);
+            a += in ? x : 0.0f;
+          }
+          t = k == 0 ? a : t + a;
+        }
+        part[0] = h == 0 ? t : part[0];
+        part[1] = t;
+      }
+      float total = 0.0f;
+      for (int l = 0; l < 8; ++l) {
+        const float x = __shfl(l < 4 ? part[0] : part[1], 16 * (l & 3) + col, 64);
+        total = l == 0 ? x : total + x;
+      }
+      return total;
+    };
+    const int64_t row = b * kTileRows + col;
+    const bool stored = odd != 0 && row < rows;
+    const float *R = reinterpret_cast<const float *>(Tg + T->off_rot);
+    BGTQ_GLOBAL uint8_t *prow = to_global(job.packed) + row * RB;
+    BGTQ_GLOBAL uint16_t *nrow = to_global(job.norms) + row * NS;
+#pragma clang loop unroll(disable)
+    for (int g = 0; g < (odd ? ng : 0); ++g) {
+      const int g0 = T->gstart[g], g1 = T->gend[g];
+      const int c0 = WHOLE_ROWS ? 0 : g0 & ~7, c1 = WHOLE_ROWS ? D : (g1 + 7) & ~7;
+      const float n = __builtin_sqrtf(tree(g0, g1, [&](int p, bool) { return input(p) * input(p); }) + 1e-30f);
+      const float rg = ng > 1 ? tree(g0, g1, [&](int, bool) { return n; }) / (float)T->gsize[g] : n;
+      const float dg = n > 1e-10f ? n : 1.0f;
+      const float s = tree(g0, g1, [&](int p, bool in) {
+        float y = 0.0f;
+#pragma clang loop unroll(disable)
+        for (int i = c0; i < c1; ++i) {
+          // An input of another group meets a zero of R: only one that is not finite counts.
+          const float x = input(i);
+          const float xn = i >= g0 && i < g1 ? x / dg : __builtin_fabsf(x) < INFINITY ? 0.0f : __builtin_nanf("");
+          y = __builtin_fmaf(xn, R[p * D + i], y);
+        }
+        const float *f = reinterpret_cast<const float *>(smem + L.pos) + gq * S::PROW + 2 * (p >> 2);
+        const uint32_t cb = reinterpret_cast<const uint32_t *>(smem + L.src)[gq * S::MROW + (p >> 2)] >> 16;
+        const float u = fminf(fmaxf((y - f[0]) * f[1], 0.0f), 255.0f);
+        const u32x2 e = *reinterpret_cast<const u32x2 *>(smem + L.tab + (cb * 2048u + 8u * (uint32_t)(int)u));
+        // A nibble pair's lanes (gq even, odd) lie in one group; the even one stores the byte.
+        const uint32_t other = (uint32_t)__shfl_xor((int)e[1], 16, 64);
+        if (in && stored) {
+          if (p >= ns) prow[(ns >> 1) + p - ns] = (uint8_t)e[1];
+          else if (!(p & 1)) prow[p >> 1] = (uint8_t)(e[1] | other << 4);
+        }
+        return __uint_as_float(e[0]);
+      });
+      const uint16_t sc = f32_to_f16_bits(rg / fmaxf(__builtin_sqrtf(s), 1e-10f));
+      if (gq == 0 && stored) nrow[g] = sc;
+    }
+    wave_sync();
   }
 }
 
