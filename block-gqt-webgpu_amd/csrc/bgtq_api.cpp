@@ -876,6 +876,76 @@ static int64_t encode_wave_max_rows(int dim, bool tile) { return !tile ? kEncode
 // encoder; 44 against 41 for 262,144, 20 against 13 for 32,768).
 constexpr int64_t kEncodeBulkMinRows = 300000;
 
+}  // extern "C"
+
+namespace {
+
+// Rows row0 .. row0 + rows of a job, encoded as a job of their own.
+struct EncodePart {
+  const bgtq_encode_job *job;
+  int64_t row0, rows;
+  int64_t dst_row() const { return job->dst_row0 + row0; }
+  const void *src(bool f32) const {
+    return static_cast<const uint8_t *>(job->src) + row0 * job->src_row_stride * (f32 ? 4 : 2);
+  }
+};
+
+// A launch's extents: the longest part and the largest tables among its jobs.
+struct EncodeExtents {
+  int64_t rows = 0;
+  int lut = 0, books = 0;
+  EncodeTileSizes tile{};
+  void add(const EncodePart &p) {
+    const bgtq_tables_info &t = p.job->tables->info;
+    rows = std::max(rows, p.rows);
+    lut = std::max(lut, t.n_codebooks * 256);
+    books = std::max(books, t.n_books * t.max_centroids);
+    tile.codebooks = std::max(tile.codebooks, t.n_codebooks);
+    tile.groups = std::max(tile.groups, t.groups);
+    tile.row_bytes = std::max(tile.row_bytes, t.row_bytes);
+  }
+  bool tile_fits(int dim) const {
+    return encode_tile_lds_bytes(dim, tile.codebooks, tile.groups, tile.row_bytes) <= 160 * 1024;
+  }
+};
+
+// The tile encoder shares the chip equally among a launch's jobs, so a job
+// much longer than the others would be walked by few workgroups while theirs
+// have left: long jobs are cut into parts, as short as lets all parts go with
+// one more upload or launch at most, where that shortens the longest walk
+// (jobs of one length stay whole). us per call without / with the cut: SmolLM2
+// heads 8000 + 50 x 20 rows 39.7 / 18.0, 90 jobs of 10 to 4096 rows 56.0 / 43.8,
+// 32768 + 1023 x 1 1935 / 73; d=128 layout A 16384 + 511 x 1 1589 / 64.
+void cut_long_jobs(std::vector<EncodePart> &parts, int64_t total_rows, int64_t wg_rows, int64_t resident,
+                   size_t per_launch) {
+  auto walk = [&](int64_t rows, size_t n) {  // passes of the workgroups of the longest part
+    const int64_t wgs = std::max<int64_t>(1, resident / (int64_t)n);
+    return (rows + wgs * wg_rows - 1) / (wgs * wg_rows);
+  };
+  int64_t longest = 0;
+  for (const EncodePart &p : parts) longest = std::max(longest, p.rows);
+  const int64_t now = walk(longest, parts.size());
+  if (now <= 1 || now <= (total_rows + wg_rows * resident - 1) / (wg_rows * resident)) return;
+  const size_t budget = (parts.size() + per_launch / 2 + per_launch - 1) / per_launch * per_launch;
+  for (int64_t k = 1; k * wg_rows < longest; k += std::max<int64_t>(1, k / 4)) {
+    const int64_t piece = k * wg_rows;
+    size_t n = 0;
+    for (const EncodePart &p : parts) n += (size_t)((p.rows + piece - 1) / piece);
+    if (n > budget) continue;
+    if (walk(piece, n) >= now) return;
+    std::vector<EncodePart> cut;
+    cut.reserve(n);
+    for (const EncodePart &p : parts)
+      for (int64_t r = 0; r < p.rows; r += piece) cut.push_back({p.job, r, std::min(piece, p.rows - r)});
+    parts.swap(cut);
+    return;
+  }
+}
+
+}  // namespace
+
+extern "C" {
+
 // ---------------------------------------------------------------- batched entry points
 bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq_encode_job *jobs, size_t n_jobs) {
   if (!ctx) return fail(BGTQ_ERR_RANGE, "null context");
@@ -909,15 +979,16 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
       by_kind[{t->info.dim, bulk ? bulk : tile ? kEncodeTile : 0}].push_back(i);
     }
   const bool src_f32 = src_dtype == BGTQ_DTYPE_F32;
-  auto job_dev = [&](const bgtq_encode_job &j) {
+  auto job_dev = [&](const EncodePart &p) {
+    const bgtq_encode_job &j = *p.job;
     EncodeJobDev J{};
     J.t = j.tables->dev();
-    J.src = j.src;
+    J.src = p.src(src_f32);
     J.src_stride = (int32_t)j.src_row_stride;
-    J.rows = j.rows;
+    J.rows = p.rows;
     J.packed = j.packed;
     J.norms = j.norms;
-    J.dst_row0 = j.dst_row0;
+    J.dst_row0 = p.dst_row();
     J.dst_step = 1;
     J.enc_bytes = (int32_t)j.tables->h()->off_rot;
     J.off_rot_t = (int32_t)j.tables->h()->off_rot_t;
@@ -940,7 +1011,7 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
         EncodeLaunch L{};
         int64_t max_rows = 0, rows = 0;
         for (size_t k = b; k < std::min(idx.size(), b + kEncodeJobsPerLaunch); ++k) {
-          L.jobs[L.n_jobs++] = job_dev(jobs[idx[k]]);
+          L.jobs[L.n_jobs++] = job_dev({&jobs[idx[k]], 0, jobs[idx[k]].rows});
           max_rows = std::max(max_rows, jobs[idx[k]].rows);
           rows += jobs[idx[k]].rows;
         }
@@ -954,38 +1025,32 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
       }
       continue;
     }
-    // A launch's extents: the longest job and the largest tables among its jobs.
-    struct Extents {
-      int64_t rows = 0;
-      int lut = 0, books = 0;
-      EncodeTileSizes tile{};
-      void add(const bgtq_encode_job &j) {
-        const bgtq_tables_info &t = j.tables->info;
-        rows = std::max(rows, j.rows);
-        lut = std::max(lut, t.n_codebooks * 256);
-        books = std::max(books, t.n_books * t.max_centroids);
-        tile.codebooks = std::max(tile.codebooks, t.n_codebooks);
-        tile.groups = std::max(tile.groups, t.groups);
-        tile.row_bytes = std::max(tile.row_bytes, t.row_bytes);
-      }
-      bool tile_fits(int dim) const {
-        return encode_tile_lds_bytes(dim, tile.codebooks, tile.groups, tile.row_bytes) <= 160 * 1024;
-      }
-    };
-    if (tile && total_rows < kEncodeTableRows) {
-      for (size_t b = 0; b < idx.size();) {
-        // Up to kTileJobsPerLaunch jobs whose tables fit the LDS together (any job's alone do).
+    std::vector<EncodePart> parts;
+    EncodeExtents all;
+    for (size_t i : idx) {
+      parts.push_back({&jobs[i], 0, jobs[i].rows});
+      all.add(parts.back());
+    }
+    const bool in_args = tile && total_rows < kEncodeTableRows;
+    if (tile && all.tile_fits(dim))
+      cut_long_jobs(parts, total_rows, encode_tile_wg_rows(dim),
+                    encode_tile_resident(dim, src_f32, device_cus(), all.tile),
+                    in_args ? kTileJobsPerLaunch : kEncodeJobsPerLaunch);
+    if (in_args) {
+      for (size_t b = 0; b < parts.size();) {
+        // Up to kTileJobsPerLaunch parts whose tables fit the LDS together (any job's alone do).
         EncodeTileLaunch L{};
-        Extents x;
-        for (; b < idx.size() && L.n_jobs < kTileJobsPerLaunch; ++b) {
-          const bgtq_encode_job &j = jobs[idx[b]];
-          const bgtq_tables_info &t = j.tables->info;
-          Extents with = x;
-          with.add(j);
+        EncodeExtents x;
+        for (; b < parts.size() && L.n_jobs < kTileJobsPerLaunch; ++b) {
+          const EncodePart &p = parts[b];
+          const bgtq_encode_job &j = *p.job;
+          EncodeExtents with = x;
+          with.add(p);
           if (!with.tile_fits(dim)) break;
           x = with;
-          L.jobs[L.n_jobs++] = {j.tables->dev(), j.src, j.packed + j.dst_row0 * t.row_bytes,
-                                j.norms + j.dst_row0 * t.norm_stride, (int32_t)j.src_row_stride, (int32_t)j.rows};
+          L.jobs[L.n_jobs++] = {j.tables->dev(), p.src(src_f32), j.packed + p.dst_row() * j.tables->info.row_bytes,
+                                j.norms + p.dst_row() * j.tables->info.norm_stride, (int32_t)j.src_row_stride,
+                                (int32_t)p.rows};
         }
         HIP_TRY(launch_encode_tile_args(L, dim, src_f32, x.rows, device_cus(), x.tile, ctx->stream), "encode launch");
       }
@@ -993,14 +1058,14 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
     }
     EncodeJobDev *table = static_cast<EncodeJobDev *>(ctx->encode_jobs.ptr);
     std::lock_guard<std::mutex> lock(ctx->encode_mutex);
-    for (size_t b = 0; b < idx.size(); b += kEncodeJobTable) {
-      const size_t e = std::min(idx.size(), b + kEncodeJobTable);
-      Extents x;
+    for (size_t b = 0; b < parts.size(); b += kEncodeJobTable) {
+      const size_t e = std::min(parts.size(), b + kEncodeJobTable);
+      EncodeExtents x;
       for (size_t c = b; c < e; c += kEncodeJobsPerLaunch) {
         EncodeLaunch L{};
         for (size_t k = c; k < std::min(e, c + kEncodeJobsPerLaunch); ++k) {
-          L.jobs[L.n_jobs++] = job_dev(jobs[idx[k]]);
-          x.add(jobs[idx[k]]);
+          L.jobs[L.n_jobs++] = job_dev(parts[k]);
+          x.add(parts[k]);
         }
         HIP_TRY(launch_encode_upload(L, table, (int)(c - b), ctx->stream), "encode job upload");
       }

@@ -414,6 +414,9 @@ hipError_t launch_encode_bulk(const EncodeJobDev *jobs, int n_jobs, int src_f32,
 constexpr int64_t kTileMaxStride = 1 << 24;
 bool encode_tile_layout(const DevTables *T);
 int encode_tile_lds_bytes(int dim, int n_codebooks, int groups, int row_bytes);
+int encode_tile_wg_rows(int dim);  // rows of a workgroup's pass
+// Workgroups the chip holds at once; a launch shares them equally among its jobs.
+int64_t encode_tile_resident(int dim, int src_f32, int cus, const EncodeTileSizes &z);
 hipError_t launch_encode_tile(const EncodeJobDev *jobs, int n_jobs, int dim, int src_f32, int64_t max_rows, int cus,
                               const EncodeTileSizes &z, hipStream_t stream);
 hipError_t launch_encode_tile_args(const EncodeTileLaunch &launch, int dim, int src_f32, int64_t max_rows, int cus,

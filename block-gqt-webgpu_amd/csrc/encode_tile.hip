@@ -574,15 +574,10 @@ hipError_t launch_d(const EncodeJobDev *table, const EncodeTileLaunch *args, con
   return launch_k(encode_tile_args_kernel<D, SRC_F32>, ok, grid, threads, lds, stream, *args, z);
 }
 
-// One round of workgroups (as many waves per SIMD as their registers allow, as far as the LDS holds
-// them) shared by the jobs, rounded down: a few more than fit take a second
-// round as long as the first. A wave walks its job's blocks with that stride.
 hipError_t launch_any(const EncodeJobDev *table, const EncodeTileLaunch *args, int n_jobs, int dim, int src_f32,
                       int64_t max_rows, int cus, const EncodeTileSizes &z, hipStream_t stream) {
-  const int waves = tile_waves(dim), lds = encode_tile_lds_bytes(dim, z.codebooks, z.groups, z.row_bytes);
-  const int fit = std::min(4 * tile_waves_per_simd(dim, src_f32) / waves, kLdsLimit / lds);
-  const int64_t resident = (int64_t)cus * std::max(1, fit);
-  const int64_t blocks = (max_rows + kTileRows - 1) / kTileRows, most = (blocks + waves - 1) / waves;
+  const int64_t wg_rows = encode_tile_wg_rows(dim), most = (max_rows + wg_rows - 1) / wg_rows;
+  const int64_t resident = encode_tile_resident(dim, src_f32, cus, z);
   const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(most, resident / n_jobs)), (unsigned)n_jobs);
   if (dim == 64)
     return src_f32 ? launch_d<64, true>(table, args, grid, z, stream) : launch_d<64, false>(table, args, grid, z, stream);
@@ -609,6 +604,16 @@ bool encode_tile_layout(const DevTables *T) {
 int encode_tile_lds_bytes(int dim, int n_codebooks, int groups, int row_bytes) {
   return dim == 64 ? tile_lds<64>(n_codebooks, groups, row_bytes).total
                    : tile_lds<128>(n_codebooks, groups, row_bytes).total;
+}
+
+int encode_tile_wg_rows(int dim) { return kTileRows * tile_waves(dim); }
+
+// One round of workgroups (as many waves per SIMD as their registers allow, as far as the LDS holds
+// them) shared by the jobs, rounded down: a few more than fit take a second
+// round as long as the first. A wave walks its job's blocks with that stride.
+int64_t encode_tile_resident(int dim, int src_f32, int cus, const EncodeTileSizes &z) {
+  const int lds = encode_tile_lds_bytes(dim, z.codebooks, z.groups, z.row_bytes);
+  return (int64_t)cus * std::max(1, std::min(4 * tile_waves_per_simd(dim, src_f32) / tile_waves(dim), kLdsLimit / lds));
 }
 
 hipError_t launch_encode_tile(const EncodeJobDev *jobs, int n_jobs, int dim, int src_f32, int64_t max_rows, int cus,

@@ -570,6 +570,46 @@ def test_small_encode_shares_no_table(device, oracle, dim, rows, heads):
         tables.destroy()
 
 
+@pytest.mark.parametrize("dim,lengths", [(64, [8001] + [1] * 40), (64, [20011] + [3] * 75 + [700]), (64, [9000] + [1] * 130),
+                                         (128, [5003] + [17] * 9), (128, [16385] + [2] * 61)])
+def test_one_long_job_among_short_ones(device, oracle, dim, lengths):
+    """A long job beside many short ones is cut into parts (calls below and from 16384 rows): odd strides,
+    odd destination rows, guard rows on both sides."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    rng = np.random.default_rng(len(lengths))
+    names = ("smollm2_h0", "smollm2_h17", "mixed_d64") if dim == 64 else ("A", "mixed_d128")
+    known = dict(_layouts(oracle), A=calibrate.layout_a(dim))
+    tabs = [bgtq.Tables(device, known[n]) for n in names]
+    try:
+        for src_kind in ("f16", "f32"):
+            jobs, checks = [], []
+            for i, rows in enumerate(lengths):
+                p, row0, stride = known[names[i % len(names)]], i % 4, dim + (1, 8, 0)[i % 3]
+                k = _random_half_rows(rng, rows, dim)
+                flat = np.zeros((rows, stride), np.float16)
+                flat[:, :dim] = k.view(np.float16)
+                src = torch.from_numpy(flat if src_kind == "f16" else flat.astype(np.float32)).cuda()
+                packed = torch.full((row0 + rows + 2, p.rowBytes), 0xA5, dtype=torch.uint8, device="cuda")
+                norms = torch.full((row0 + rows + 2, p.normStride), 0x5A5A, dtype=torch.int16, device="cuda")
+                jobs.append(dict(tables=tabs[i % len(names)], src=src, src_row_stride=stride, rows=rows, packed=packed,
+                                 norms=norms, dst_row0=row0))
+                checks.append((p, row0, k, packed, norms))
+            batched.encode(device, jobs, src_kind)
+            device.synchronize()
+            for i, (p, row0, k, packed, norms) in enumerate(checks):
+                ref_p, ref_n = oracle.encode_pack(_olayout(oracle, p), k)
+                got_p, got_n = packed.cpu().numpy(), norms.cpu().numpy().view(np.uint16)
+                own = slice(row0, row0 + len(k))
+                assert np.array_equal(got_p[own], ref_p) and np.array_equal(got_n[own], ref_n), f"job {i} {src_kind}"
+                outside = np.r_[0:row0, row0 + len(k):len(got_p)]
+                assert np.all(got_p[outside] == 0xA5) and np.all(got_n[outside] == 0x5A5A), f"job {i}: guard rows"
+    finally:
+        for t in tabs:
+            t.destroy()
+
+
 def test_concurrent_appends_near_capacity(device, oracle):
     """Two threads append at once near the end of a store's capacity (the Node addon runs appends off
     the JS thread). The store is claimed before the capacity check, as the reference refuses a second
