@@ -475,12 +475,14 @@ __global__ __launch_bounds__(64 * kWeightedWaves) void model_weighted_kernel(Mod
           }
         }
       } else {
-        // A block past the last has V rows of zeros (and the last block's,
-        // finite or its row's own, probabilities).
+        // (a block past the last would multiply the last one's probabilities,
+        // perhaps infinite ones of the caller's, by zeros)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+          if (b + u * kWeightedWaves >= n_blocks) break;  // wave-uniform
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc = mfma_f32(pr[u][i], h2f(v[u][i]), acc);
+        }
       }
 #pragma unroll
       for (int u = 0; u < U; ++u)

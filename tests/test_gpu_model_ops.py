@@ -293,3 +293,32 @@ def test_model_dispatch_weighted_causal_ends(device, kvh, gqa, rows, start):
     inf[odd:, (kvh - 1) * gqa:, 7] = True
     assert torch.isposinf(attn[inf]).all()
     torch.testing.assert_close(attn.double()[~inf], out[~inf], rtol=0, atol=2 * tokens * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("gqa,rows,tokens", [(3, 1, 70), (3, 2, 16), (3, 2, 100), (2, 5, 530), (1, 9, 2300)])
+def test_model_dispatch_weighted_infinite_probabilities(device, gqa, rows, tokens):
+    """weighted over a caller's own probabilities with an infinity in the last token of one row: that row's
+    outputs are infinities of V's signs, the others finite, for token counts around whole rounds of the
+    kernel's blocks."""
+    import torch
+    import bgtq
+    ops = bgtq.ModelOps.create(device)
+    kvh, d, start = 2, 64, tokens - 1
+    qh = kvh * gqa
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    probs = torch.rand((rows, qh, tokens), generator=g, device="cuda")
+    v = torch.rand((kvh, tokens, d), generator=g, device="cuda").half() + 1
+    v[:, :, 1::2] *= -1
+    probs[0, 1, tokens - 1] = float("inf")
+    attn = torch.full((rows, qh, d), float("nan"), device="cuda")
+    cmd = ops.commands()
+    cmd.dispatch("weighted", [rows, tokens, tokens, start, qh, kvh, gqa, d],
+                 [None, None, v.view(torch.int16), None, probs, attn], rows * qh * d)
+    cmd.submit()
+    attn = attn.cpu().double()
+    assert torch.isposinf(attn[0, 1, 0::2]).all() and torch.isneginf(attn[0, 1, 1::2]).all()
+    attn[0, 1] = probs[0, 1, tokens - 1] = 0
+    ref = torch.einsum("rkgt,ktd->rkgd", probs.cpu().double().view(rows, kvh, gqa, tokens), v.cpu().double())
+    ref = ref.reshape(rows, qh, d)
+    ref[0, 1] = 0
+    torch.testing.assert_close(attn, ref, rtol=tokens * 2.0 ** -24, atol=0)
