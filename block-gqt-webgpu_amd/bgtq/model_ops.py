@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes
 import struct
+import sys
 
 from . import _lib
 from ._lib import RangeError, check, lib
@@ -41,13 +42,14 @@ def _binding(b) -> tuple[int, int, int]:
     """bgtq_model_binding's words: device address, bytes, tables handle."""
     if b is None:
         return 0, 0, 0
-    if not hasattr(type(b), "data_ptr"):
+    torch = sys.modules.get("torch")
+    if torch is None or not isinstance(b, torch.Tensor):  # (a tensor's missing attribute is slow to look up)
         handle = getattr(b, "handle", None)
         if handle is not None and hasattr(b, "info"):  # calibration Tables
-            return 0, 0, handle.value
+            return 0, 0, getattr(handle, "value", handle) or 0
     if not b.is_contiguous():
         raise RangeError("Model buffers must be contiguous")
-    return b.data_ptr(), b.nbytes, 0
+    return b.data_ptr(), b.numel() * b.element_size(), 0
 
 
 class ModelOps:
@@ -91,7 +93,8 @@ class Commands:
             if text is None:
                 text = ctypes.create_string_buffer(name.encode())
                 keep.append(text)
-            _DISPATCH.pack_into(arr, i * _DISPATCH.size, ctypes.addressof(text), *params, at, len(buffers), x, y)
+            _DISPATCH.pack_into(arr, i * _DISPATCH.size, ctypes.addressof(text), *params, at, len(buffers), x & 0xFFFFFFFF,
+                                y & 0xFFFFFFFF)
             at += 24 * len(buffers)
         self._dispatches = []
         check(lib().bgtq_model_submit(self.ops.device.handle, arr, n))

@@ -505,3 +505,50 @@ def test_encoder_division_by_reciprocal(tmp_path):
     r = subprocess.run([str(exe), "600"], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout
     assert r.stdout.strip().endswith("mismatches 0"), r.stdout
+
+
+def test_model_commands_take_what_they_took(monkeypatch):
+    """Commands.submit packs its C structs itself: counts outside 32 bits wrap as C's, table handles may be
+    plain integers or null (the library's own check answers), buffers need data_ptr, numel, element_size
+    and is_contiguous only."""
+    import types
+    import torch
+    from bgtq import _lib, model_ops
+
+    got = []
+
+    class Lib:
+        def bgtq_model_submit(self, handle, arr, n):
+            for d in arr[:n]:
+                b = d.bindings[0]
+                got.append((d.name, list(d.params), (b.ptr, b.bytes, b.tables), d.n_bindings, d.x, d.y))
+            return 0
+
+    class Buffer:
+        def __init__(self, t):
+            self.data_ptr, self.numel, self.element_size = t.data_ptr, t.numel, t.element_size
+            self.is_contiguous = t.is_contiguous
+
+    monkeypatch.setattr(model_ops, "lib", lambda: Lib())
+    device = types.SimpleNamespace(handle=None, synchronize=lambda: None)
+    x = torch.zeros(6)
+    fields = [f for f, _ in _lib.Binding._fields_]
+    assert len(fields) == 3
+
+    def submit(buffer, x=1, y=1, params=(7,)):
+        got.clear()
+        cmd = model_ops.Commands(types.SimpleNamespace(device=device))
+        cmd.dispatch("append", params, [buffer, None], x, y)
+        cmd.submit()
+        return got[0]
+
+    def tables(handle):
+        return types.SimpleNamespace(handle=handle, info={})
+
+    assert submit(x) == (b"append", [7] + [0] * 7, (x.data_ptr(), 24, None), 2, 1, 1)
+    assert submit(x, -1, -2)[4:] == (2 ** 32 - 1, 2 ** 32 - 2)
+    assert submit(Buffer(x))[2] == (x.data_ptr(), 24, None)
+    assert submit(torch.nn.Parameter(x))[2] == (x.data_ptr(), 24, None)
+    assert submit(tables(ctypes.c_void_p(4096)))[2] == (None, 0, 4096)
+    assert submit(tables(4096))[2] == (None, 0, 4096)
+    assert submit(tables(ctypes.c_void_p(0)))[2] == (None, 0, None)
