@@ -1215,6 +1215,16 @@ static bool fused_v(const DecodeParams &p) {
          (p.v_head_stride * vb) % 16 == 0;
 }
 
+// KV head h's lookup tables and rotation as the fused kernel reads them: FP32
+// for FP32 V, else f16 hi/lo operands.
+static void fused_tables(const DecodeParams &p, const DevTables *T, const uint8_t *base, int h, FastLayout *fl) {
+  const bool f32 = p.v_dtype == BGTQ_DTYPE_F32;
+  fl->mfma[h] = base + (f32 ? T->off_books : T->off_mfma);
+  fl->rot_q[h] = base + (f32 ? T->off_rot : T->off_rot_q);
+  fl->cent_exp[h] = f32 ? 0 : T->cent_exp;
+  fl->gmc[h] = T->max_centroids;
+}
+
 // Whether the fused matrix-core kernel handles this launch (FastLayout in
 // bgtq_internal.h); on success fills the K-step books, nn and sg.
 static bool fast_layout(const DecodeParams &p, const bgtq_tables *const *tables, FastLayout *fl, int *nn, int *sg) {
@@ -1248,11 +1258,9 @@ static bool fast_layout(const DecodeParams &p, const bgtq_tables *const *tables,
       else if (fl->book[s] != bk) return false;
     }
     const uint8_t *base = reinterpret_cast<const uint8_t *>(tables[h]->dev());
-    fl->mfma[h] = base + T->off_mfma;
-    fl->rot_q[h] = base + T->off_rot_q;
+    fused_tables(p, T, base, h, fl);
     fl->rot_t[h] = reinterpret_cast<const float *>(base + T->off_rot_t);
     fl->enc_bytes[h] = (int32_t)T->off_rot;  // header, LUT, books
-    fl->cent_exp[h] = T->cent_exp;
     const int sgv = T->groups == 1 ? ks : g0;
     if (h == 0) {
       *nn = n;
@@ -1290,7 +1298,7 @@ static bool general_layout(const DecodeParams &p, const bgtq_tables *const *tabl
     for (int j = 0; j < p.dim; ++j) (j < T->nibble_dims ? nib_books : byte_books) |= 1u << T->pos_book[j];
     if (nib_books & byte_books) return false;
     const uint8_t *base = reinterpret_cast<const uint8_t *>(tables[h]->dev());
-    fl->rot_q[h] = base + T->off_rot_q;
+    fused_tables(p, T, base, h, fl);
     fl->rot_t[h] = reinterpret_cast<const float *>(base + T->off_rot_t);
     // The append's encoder reads an LDS copy of the header, LUT and books
     // when they fit a ring slot, else of the LUT and books (the header in
@@ -1304,8 +1312,6 @@ static bool general_layout(const DecodeParams &p, const bgtq_tables *const *tabl
       fl->enc_from[h] = (int32_t)T->off_lut;
       fl->enc_bytes[h] = (int32_t)(T->off_rot - T->off_lut);
     }
-    fl->cent_exp[h] = T->cent_exp;
-    fl->mfma[h] = base + T->off_mfma;
     fl->gdesc[h] = reinterpret_cast<const uint32_t *>(base + T->off_gdesc);
     fl->glane[h] = reinterpret_cast<const uint32_t *>(base + T->off_glane);
     fl->grb[h] = (int16_t)T->row_bytes;

@@ -353,10 +353,12 @@ struct FastLayout {
   int32_t book[4];  // centroid book of each K-step
   // Per KV head, resolved on the host so the kernel's first loads need no
   // dependent read of the tables' header: the MFMA lookup tables, the
-  // permuted rotation's MFMA operands and cent_exp.
+  // permuted rotation's MFMA operands and cent_exp; for FP32 V the books'
+  // FP32 centroids (max_centroids a row, gmc), the rotation as it is, and 0.
   const uint8_t *mfma[kMaxKvHeads];
   const uint8_t *rot_q[kMaxKvHeads];
   int32_t cent_exp[kMaxKvHeads];
+  int32_t gmc[kMaxKvHeads];
   // The decode-step append's encoder: transposed rotation, and the bytes of
   // the table set's header, code LUT and books (contiguous from its start).
   const float *rot_t[kMaxKvHeads];

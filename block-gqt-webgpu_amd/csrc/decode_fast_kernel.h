@@ -154,7 +154,16 @@ struct MergeRows {
   }
 };
 
-template <int D, int SMAX, int NW>
+// Weight of a logit, or of a state's maximum, d above the merged maximum (d <=
+// 0). The logits are in the log2 domain; with FP32 V in natural units (NAT),
+// so that the difference of two large ones is exact (scaled to the log2 domain
+// only then; expf itself measured no closer to 64 bits and 4% slower).
+template <bool NAT>
+__device__ __forceinline__ float exp_of(float d) {
+  return __builtin_amdgcn_exp2f(NAT ? d * kLog2e : d);
+}
+
+template <int D, int SMAX, int NW, bool NAT>
 __device__ __forceinline__ void merge_one_round(float *part, float *out, float *stats, int64_t head0, int G, int S,
                                              int wave, int lane) {
   constexpr int kWaves = NW;
@@ -194,7 +203,7 @@ __device__ __forceinline__ void merge_one_round(float *part, float *out, float *
       if (g >= G) continue;
       const int64_t head = head0 + g;
       const float M = col_max(row_max(ms[h]));
-      const float w = ms[h] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms[h] - M);
+      const float w = ms[h] == -INFINITY ? 0.0f : exp_of<NAT>(ms[h] - M);
       float lw = ls[h] * w;
       lw += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(lw), 0x128, 0xf, 0xf, false));
       lw += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(lw), 0x124, 0xf, 0xf, false));
@@ -215,7 +224,7 @@ __device__ __forceinline__ void merge_one_round(float *part, float *out, float *
 #pragma unroll
       for (int dl = 0; dl < DL; ++dl) out[head * D + DL * lane + dl] = acc[dl] / Lsum;
       if (lane == 0 && stats) {
-        stats[head * 2] = M * kLn2;
+        stats[head * 2] = NAT ? M : M * kLn2;
         stats[head * 2 + 1] = Lsum;
       }
     }
@@ -334,7 +343,14 @@ __device__ __forceinline__ void merge_rows(float *part, float *out, const MergeR
 // only as many of its splits as its history needs (p.split_floor tokens per
 // split at least); the others exit before their first chunk.
 // VF: V rows of FP32 values (1; decode without an appended token) or FP16
-// (0). FP32 V takes its PV products on the FP32 matrix cores.
+// (0). FP32 V: the whole pass in FP32, as the general kernel computes it:
+// rotation, QK with the FP32 centroids and PV on the FP32 matrix cores,
+// logits in natural units (FP16 V: f16 matrix cores with hi/lo operands; so
+// also QK of FP16 K, whose values one f16 operand holds exactly). Error of the
+// output against 64 bits with |logits| up to about 60, general kernel / hi/lo
+// operands / this: layout A 6.6e-7 / 8.4e-7 / 5.7e-7, SmolLM2 heads 1.13e-6 /
+// 0.92e-6 / 0.72e-6, FP16 K 1.29e-6 / 0.74e-6 / the same; 8 sequences x 14
+// heads x 4096 tokens 57.7 / 18.1 / 20.3 us.
 // NW: waves per workgroup (4; row-wise prefill at d=64, 8: a unit's splits
 // then cover twice the tokens each and half as many partials are merged).
 // Every kernel argument the set-up reads, loaded at once (one asm statement,
@@ -372,6 +388,9 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   static_assert(KF == 0 || row_enc::scratch_bytes(D) <= Sl::BYTES, "append scratch fits a ring slot");
   constexpr int KS = Gm::KS, DT = Gm::DT, PR = Gm::PR, VI = Sl::VI, KRI = Gm::KRI;
   constexpr int VB = VF ? 4 : 2;  // bytes per V value
+  constexpr bool NAT = VF != 0;                // logits in natural units, else log2 domain
+  constexpr bool F32 = VF && KF >= 1;          // rotation and QK in FP32
+  constexpr float kLogit = NAT ? 1.0f : kLn2;  // a logit's natural value
   // P is carried times 2^15 where it is split into FP16 parts; unscaled for FP32 V.
   constexpr float kPShift = VF ? 0.0f : 15.0f, kPFactor = VF ? 1.0f : kPScale;
   constexpr int RB = Sl::RB, KI = Sl::KI, L = Sl::L, AHEAD = Sl::AHEAD;
@@ -473,7 +492,18 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   // col, dims 32 s + 8 gq + 0..7) and, for packed K, the MFMA operands of its
   // tiles of the permuted rotation. The first AHEAD chunks are issued behind
   // these loads and stay in flight through the prologue.
-  if (KF == 1 && wave == 0) {
+  // FP32 V: the books' FP32 centroids (fl.mfma: the first book, rows of
+  // max_centroids), in the places of the code tables.
+  const int mc4 = F32 ? 4 * fl.gmc[kv] : 0;
+  if (F32 && KF == 1 && wave == 0) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const __amdgpu_buffer_rsrc_t rt = rsrc(fl.mfma[kv] + fl.book[s] * mc4, (uint32_t)min(mc4, 1024));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dma4(rt, tabs + s * 2048 + k * 256, k * 256 + lane * 4, 0);
+    }
+  }
+  if (!F32 && KF == 1 && wave == 0) {
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const uint8_t *src = fl.mfma[kv] + fl.book[s] * kMfmaTableBytes + (s < NN ? 0 : 2048);
@@ -493,7 +523,9 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
 #pragma unroll
       for (int pc = 0; pc < 4; ++pc) {
         if (bk < nb && pc < pieces) {
-          const __amdgpu_buffer_rsrc_t rt = rsrc(fl.mfma[kv] + bk * kMfmaTableBytes + 2048 + pc * 256, 256);
+          const __amdgpu_buffer_rsrc_t rt =
+              F32 ? rsrc(fl.mfma[kv] + bk * mc4 + pc * 256, (uint32_t)max(0, min(mc4 - pc * 256, 256)))
+                  : rsrc(fl.mfma[kv] + bk * kMfmaTableBytes + 2048 + pc * 256, 256);
           dma4(rt, tabs + bk * span + ((nibble_books >> bk) & 1u ? 4 : 8) + pc * 256, lane * 4, 0);
         }
       }
@@ -532,9 +564,25 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) qload[s][hh] = src[8 * s + 2 * gq + hh];
   }
-  u32x4 rq[NT][KS][2];
+  u32x4 rq[F32 ? 1 : NT][F32 ? 1 : KS][2];
+  // FP32 V: the rotation's rows 16 n + col of this wave's tiles n (fl.rot_q:
+  // R), columns 16 m + 4 gq + 0..3, and the natural positions of those columns.
+  f32x4 rf[F32 ? NT : 1][F32 ? DT : 1];
+  uint32_t pw[F32 ? DT : 1];
+  if constexpr (F32) {
+    if (rotate) {
+      const float *R = reinterpret_cast<const float *>(fl.rot_q[kv]);
+#pragma unroll
+      for (int m = 0; m < DT; ++m) pw[m] = *reinterpret_cast<const uint32_t *>(p.tables[kv]->perm + 16 * m + 4 * gq);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < DT; ++m)
+          rf[t][m] = *reinterpret_cast<const f32x4 *>(R + (16 * (rot_wave ? wave * NT + t : 0) + col) * D + 16 * m + 4 * gq);
+    }
+  }
   // (wave-uniform: waves past the tiles load none)
-  if (rotate && rot_wave) {
+  if (!F32 && rotate && rot_wave) {
     const u32x4 *op = reinterpret_cast<const u32x4 *>(fl.rot_q[kv]);  // [tile][K-step][lane][hi, lo]
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -886,30 +934,60 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
     // K-step, off-group entries exact zeros). Tile n leaves rows
     // j = 16 n + 4 gq + 0..3 of head col in this lane; they go through LDS
     // (the last ring slot, rows padded to D + 4 floats) to the QK layout.
-    float qmax = 0.0f;
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int jv = 0; jv < 8; ++jv) qmax = fmaxf(qmax, fabsf(qv[s][jv]));
-    const int e0 = split_exp(col_max(qmax));
-    half8 bh[KS], bl[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) split_scaled(qv[s], __builtin_ldexpf(1.0f, e0), bh[s], bl[s]);
+    // F32: in FP32, the query permuted through LDS instead.
     // (row-wise prefill: its staging area after the ring)
     float *qs = reinterpret_cast<float *>(PF ? ring + Sl::DYN : ring + ((Sl::RING - 1) * kWaves + stage_w) * Sl::BYTES);
-    const float unscale = __builtin_ldexpf(1.0f, -e0);
+    if constexpr (F32) {
+      // The queries in natural order in the next wave's last ring slot (free until the loop).
+      float *qn = reinterpret_cast<float *>(ring + ((Sl::RING - 1) * kWaves + 1) * Sl::BYTES);
+      if (wave == 0) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (!rot_wave) break;  // wave-uniform: waves past the tiles only read the result
-      f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s = 0; s < KS; ++s)
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const half8 ah = __builtin_bit_cast(half8, rq[t][s][0]), al = __builtin_bit_cast(half8, rq[t][s][1]);
-        acc = mfma(ah, bh[s], acc);
-        acc = mfma(al, bh[s], acc);
-        acc = mfma(ah, bl[s], acc);
+          for (int hh = 0; hh < 2; ++hh)
+            *reinterpret_cast<f32x4 *>(qn + col * (D + 4) + 32 * s + 8 * gq + 4 * hh) =
+                f32x4{qv[s][4 * hh], qv[s][4 * hh + 1], qv[s][4 * hh + 2], qv[s][4 * hh + 3]};
       }
-      *reinterpret_cast<f32x4 *>(qs + col * (D + 4) + 16 * (wave * NT + t) + 4 * gq) = acc * unscale;
+      lds_barrier();
+      float x[DT][4];
+#pragma unroll
+      for (int m = 0; m < DT; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[m][i] = qn[col * (D + 4) + (int)((pw[m] >> (8 * i)) & 255u)];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (!rot_wave) break;
+        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int m = 0; m < DT; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rf[t][m][i], x[m][i], acc, 0, 0, 0);
+        *reinterpret_cast<f32x4 *>(qs + col * (D + 4) + 16 * (wave * NT + t) + 4 * gq) = acc;
+      }
+    } else {
+      float qmax = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int jv = 0; jv < 8; ++jv) qmax = fmaxf(qmax, fabsf(qv[s][jv]));
+      const int e0 = split_exp(col_max(qmax));
+      half8 bh[KS], bl[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) split_scaled(qv[s], __builtin_ldexpf(1.0f, e0), bh[s], bl[s]);
+      const float unscale = __builtin_ldexpf(1.0f, -e0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (!rot_wave) break;  // wave-uniform: waves past the tiles only read the result
+        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const half8 ah = __builtin_bit_cast(half8, rq[t][s][0]), al = __builtin_bit_cast(half8, rq[t][s][1]);
+          acc = mfma(ah, bh[s], acc);
+          acc = mfma(al, bh[s], acc);
+          acc = mfma(ah, bl[s], acc);
+        }
+        *reinterpret_cast<f32x4 *>(qs + col * (D + 4) + 16 * (wave * NT + t) + 4 * gq) = acc * unscale;
+      }
     }
     if (app_wg) wait_vm<0>();  // the table DMAs (append workgroups issue no chunks)
     else wait_vm<AHEAD * L>();  // the table DMAs, which precede the chunks
@@ -929,9 +1007,16 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   }
   // B operand of QK: lane holds qr[head = col][32 s + 8 gq + 0..7], split hi/lo
   // after scaling the head's row so its largest entry is near 2^14.
+  // F32: the FP32 values themselves.
   half8 qhi[KS], qlo[KS];
-  float kq;  // log2-domain logit = (sum_g s_g acc_g) * kq
-  {
+  float qf[F32 ? KS : 1][8];
+  float kq = 1.0f;  // logit = (sum_g s_g acc_g) * kq
+  if constexpr (F32) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int jv = 0; jv < 8; ++jv) qf[s][jv] = head_ok ? qv[s][jv] * p.inv_sqrt_d : 0.0f;
+  } else {
     float qmax = 0.0f;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
@@ -952,7 +1037,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
         qhi[s][jv] = (_Float16)x;
         qlo[s][jv] = (_Float16)(x - (float)qhi[s][jv]);
       }
-    kq = __builtin_ldexpf(kLog2e, -(eq + ec));
+    kq = __builtin_ldexpf(NAT ? 1.0f : kLog2e, -(eq + ec));
   }
   // The q staging (a ring slot's, whose chunk comes later) is dead; row-wise
   // prefill's own staging area is never written again, so it needs no
@@ -988,6 +1073,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   int glo[KS2], nsl[KS2], koff[KS2], hib[KS2], nmf[KS2];
   uint32_t ext[KS2][8], tbo[KS2][8];
   half8 qbh[KS2][kSlots], qbl[KS2][kSlots];  // masked (packed) query operands of MFMA m
+  float qbf[F32 ? KS2 : 1][kSlots][8];       // the same in FP32
   const int GP = KF == 2 ? (ncol <= 4 ? 4 : ncol <= 8 ? 2 : 1) : 1;  // group slots per MFMA
   const int HW = 16 / GP, cg = col / HW;
   constexpr int NSV = KF == 2 ? 2 * Sl::NSC : 1;  // scale entries a lane moves
@@ -1009,13 +1095,19 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       nmf[s] = (nsl[s] + GP - 1) / GP;
       // Head hc's operands come from lane (gq, hc); slot cg + m * GP's mask
       // keeps that group's positions (slots past the K-step's groups: none).
-      const u32x4 h = __builtin_bit_cast(u32x4, qhi[s]), l = __builtin_bit_cast(u32x4, qlo[s]);
       const int src = 16 * gq + (col & (HW - 1));
       u32x4 hs, ls;
+      float fs[8];
+      if constexpr (F32) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        hs[k] = (uint32_t)__shfl((int)h[k], src, 64);
-        ls[k] = (uint32_t)__shfl((int)l[k], src, 64);
+        for (int k = 0; k < 8; ++k) fs[k] = __shfl(qf[s][k], src, 64);
+      } else {
+        const u32x4 h = __builtin_bit_cast(u32x4, qhi[s]), l = __builtin_bit_cast(u32x4, qlo[s]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          hs[k] = (uint32_t)__shfl((int)h[k], src, 64);
+          ls[k] = (uint32_t)__shfl((int)l[k], src, 64);
+        }
       }
 #pragma unroll
       for (int m = 0; m < kSlots; ++m) {
@@ -1024,8 +1116,13 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
 #pragma unroll
         for (int i = 0; i < kSlots; ++i)
           if (slot == i) mk = grec[s][5 + i];
-        qbh[s][m] = __builtin_bit_cast(half8, hs & mk);
-        qbl[s][m] = __builtin_bit_cast(half8, ls & mk);
+        if constexpr (F32) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) qbf[s][m][k] = mk[k >> 1] >> (16 * (k & 1)) & 1u ? fs[k] : 0.0f;
+        } else {
+          qbh[s][m] = __builtin_bit_cast(half8, hs & mk);
+          qbl[s][m] = __builtin_bit_cast(half8, ls & mk);
+        }
       }
     }
     // The chunk's scale rows [token][ns] become [group][32 tokens] in place
@@ -1205,10 +1302,19 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
           }
       }
       half8 ah[KS2][2], al[KS2][2];
+      float af[F32 ? KS2 : 1][2][8];
 #pragma unroll
       for (int s = 0; s < KS2; ++s)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
+          if constexpr (F32) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const uint32_t code = __builtin_amdgcn_ubfe(k < 4 ? w0[s][u] : wh[s][u], ext[s][k], tbo[s][k]);
+              af[s][u][k] = *reinterpret_cast<const float *>(tabs + tbo[s][k] + 4 * code);
+            }
+            continue;
+          }
           u32x4 hi, lo;
           if (s < PK) {
             // Pair K-step: the lane's 8 nibble codes are the 4 bytes of w0;
@@ -1249,9 +1355,14 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            a = mfma(ah[s][u], qbh[s][m], a);
-            a = mfma(al[s][u], qbh[s][m], a);
-            a = mfma(ah[s][u], qbl[s][m], a);
+            if constexpr (F32) {
+#pragma unroll
+              for (int k = 0; k < 8; ++k) a = __builtin_amdgcn_mfma_f32_16x16x4f32(af[s][u][k], qbf[s][m][k], a, 0, 0, 0);
+            } else {
+              a = mfma(ah[s][u], qbh[s][m], a);
+              a = mfma(al[s][u], qbh[s][m], a);
+              a = mfma(ah[s][u], qbl[s][m], a);
+            }
             const u32x2 w = *reinterpret_cast<const u32x2 *>(sb + Sl::NOFF + 2 * (g * 32 + 16 * u + 4 * gq));
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -1297,10 +1408,18 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
           else wb[u][s] = *reinterpret_cast<const u32x2 *>(row + 16 * NN + 32 * (s - NN) + 8 * gq);
         }
       u32x4 hi[2][KS], lo[2][KS];
+      float af[2][F32 ? KS : 1][8];
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
+          if constexpr (F32) {
+            const float *tf = reinterpret_cast<const float *>(tn + s * 512);  // [code]
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              af[u][s][k] = tf[s < NN ? wn[u][s] >> (4 * k) & 15u : wb[u][s][k >> 2] >> (8 * (k & 3)) & 255u];
+            continue;
+          }
           if (s < NN) {
             const u32x2 *t64 = reinterpret_cast<const u32x2 *>(tn + s * 512);  // [byte]: hi pair, lo pair
 #pragma unroll
@@ -1325,6 +1444,12 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
           const int g = s < SG ? 0 : 1;
+          if constexpr (F32) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              acc[u][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[u][s][k], qf[s][k], acc[u][g], 0, 0, 0);
+            continue;
+          }
           const half8 ah = __builtin_bit_cast(half8, hi[u][s]), al = __builtin_bit_cast(half8, lo[u][s]);
           acc[u][g] = mfma(ah, qhi[s], acc[u][g]);
           acc[u][g] = mfma(al, qhi[s], acc[u][g]);
@@ -1388,10 +1513,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       // B operand of its probability j = 0..7 (row reads; the four lane
       // groups hit different banks through swz32). The 16x16x4 FP32 product
       // takes P and V as they are, so it serves any FP32 value and spends no
-      // vector instructions on splitting (each value into three FP16 parts
-      // served |V| < 65504 only, and batched calls, whose values the library
-      // does not see, took the general kernels: 8 sequences x 14 heads x 4096
-      // tokens 65 us against 17.7).
+      // vector instructions on splitting.
       const uint8_t *vl = sb + 16 * gq * D + 4 * col;
       float v[8][DT];
 #pragma unroll
@@ -1516,18 +1638,18 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int tok = c0 + 16 * (j >> 2) + 4 * gq + (j & 3);
-          if (head_ok && tok < t_logit) p.logits[((int64_t)qrow * Hq + hq0 + col) * p.logit_stride + tok] = x[j] * kLn2;
+          if (head_ok && tok < t_logit) p.logits[((int64_t)qrow * Hq + hq0 + col) * p.logit_stride + tok] = x[j] * kLogit;
         }
       }
-      // online softmax (log2 domain) for head col
+      // online softmax (log2 domain; FP32 V: natural units) for head col
       float mloc = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
       const float m_new = fmaxf(m_run, col_max(mloc));
-      const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+      const float alpha = m_new == -INFINITY ? 1.0f : exp_of<NAT>(m_run - m_new);
       const float mb = (m_new == -INFINITY ? 0.0f : m_new) - kPShift;
       float pr[8], psum = 0.0f;
   #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        pr[j] = __builtin_amdgcn_exp2f(x[j] - mb);
+        pr[j] = exp_of<NAT>(x[j] - mb);
         psum += pr[j];
       }
       l_run = __builtin_fmaf(l_run, alpha, psum);
@@ -1609,7 +1731,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) {
         const bool live = mw[w] != -INFINITY;
-        const float wt = __builtin_amdgcn_exp2f(mw[w] - M);
+        const float wt = exp_of<NAT>(mw[w] - M);
         Lsum = live ? __builtin_fmaf(lw[w], wt, Lsum) : Lsum;
         Ov = live ? __builtin_fmaf(ow[w], wt, Ov) : Ov;
       }
@@ -1618,7 +1740,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
       if (S == 1) {
         p.out[head * D + dm] = Ov / Lsum;
         if (dm == 0 && p.stats) {
-          p.stats[head * 2] = M * kLn2;
+          p.stats[head * 2] = M * kLogit;
           p.stats[head * 2 + 1] = Lsum;
         }
       } else {
@@ -1720,10 +1842,10 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
     return;
   }
   if (S <= kMergeOneRound) {
-    if (S <= 8) merge_one_round<D, 8, NW>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
-    else if (S <= 16) merge_one_round<D, 16, NW>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
-    else if (S <= 24) merge_one_round<D, 24, NW>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
-    else merge_one_round<D, kMergeOneRound, NW>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
+    if (S <= 8) merge_one_round<D, 8, NW, NAT>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
+    else if (S <= 16) merge_one_round<D, 16, NW, NAT>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
+    else if (S <= 24) merge_one_round<D, 24, NW, NAT>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
+    else merge_one_round<D, kMergeOneRound, NW, NAT>(p.part, p.out, p.stats, (int64_t)qrow * Hq + hq0, G, S, wave, lane);
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
@@ -1745,14 +1867,14 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
     float Lsum = 0.0f;
     for (int s = 0; s < S; ++s) {
       const float m = mrow[tid * S + s];
-      const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
+      const float w = m == -INFINITY ? 0.0f : exp_of<NAT>(m - M);
       Lsum = __builtin_fmaf(wgt[tid * S + s], w, Lsum);
       mrow[tid * S + s] = w;
     }
     for (int s = 0; s < S; ++s) wgt[tid * S + s] = mrow[tid * S + s] / Lsum;
     if (p.stats) {
       const int64_t head = out_row(tid);
-      p.stats[head * 2] = M * kLn2;
+      p.stats[head * 2] = M * kLogit;
       p.stats[head * 2 + 1] = Lsum;
     }
   }
@@ -1833,8 +1955,8 @@ hipError_t launch_one(const DecodeParams &p, const FastLayout &fl, hipStream_t s
   if (p.v_dtype == BGTQ_DTYPE_F32) {
     if constexpr ((KINDS & kKindDecode) != 0)
       if (kind == kKindDecode)
-        return p.logits ? launch_mode<D, KF, NN, SG, PK, 0, 1, kWaves, 2>(p, fl, stream)
-                        : launch_mode<D, KF, NN, SG, PK, 0, 1, kWaves, 0>(p, fl, stream);
+        return p.logits ? launch_mode<D, KF, NN, SG, 0, 0, 1, kWaves, 2>(p, fl, stream)  // (FP32 centroids: no pairs)
+                        : launch_mode<D, KF, NN, SG, 0, 0, 1, kWaves, 0>(p, fl, stream);
     return hipErrorInvalidValue;
   }
   if constexpr ((KINDS & kKindDecode) != 0)

@@ -411,6 +411,68 @@ def test_fp32_values_batched(device, oracle, key_format, layout, dim, hq, hkv, l
             t.destroy()
 
 
+@pytest.mark.parametrize("layout,dim,hq,hkv", [("A", 64, 9, 3), ("A", 64, 2, 1), ("B", 64, 14, 2), ("A", 128, 4, 2),
+                                              ("B", 128, 8, 2)])
+def test_fp32_values_keep_fp32_logits(device, oracle, layout, dim, hq, hkv):
+    """bgtq_decode over FP32 V with logits of up to about 80 (the output's error then is the logits'): about
+    as far from 64 bits as the same attention in plain FP32 on the CPU (query rotation, QK with the
+    centroids, scales, softmax and PV). The bound is 1.35 times that error: the sums here are chains, the
+    CPU's are blocked (FP32 chains measured 0.9 to 1.3 times it, 22-bit operands up to 1.9 times)."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    batched.bind_torch_stream(device)
+    p = calibrate.layout_b(dim) if layout == "B" else calibrate.layout_a(dim)
+    g = torch.Generator().manual_seed(dim + hq)
+    B, T, G = 24, 1500, hq // hkv
+    k = torch.randn((B, hkv, T, dim), generator=g).half()
+    v = torch.randn((B, hkv, T, dim), generator=g).cuda()
+    q = (torch.randn((B, hq, dim), generator=g) * 15).cuda()
+    tables = bgtq.Tables(device, p)
+    try:
+        packed = torch.zeros((B, hkv, (T * p.rowBytes + 79) // 16 * 16), dtype=torch.uint8, device="cuda")
+        norms = torch.zeros((B, hkv, (T * p.normStride + 39) // 8 * 8), dtype=torch.int16, device="cuda")
+        kd = k.cuda()
+        batched.encode(device, [dict(tables=tables, src=kd[b, h], src_row_stride=dim, rows=T, packed=packed[b, h],
+                                     norms=norms[b, h]) for b in range(B) for h in range(hkv)], "f16")
+        out = torch.empty((B, hq, dim), device="cuda")
+        args = dict(batch=B, q_heads=hq, kv_heads=hkv, dim=dim, q=q, out=out, max_length=T, v=v, v_dtype="f32",
+                    lengths=torch.full((B,), T, dtype=torch.int32, device="cuda"), v_seq_stride=v.stride(0),
+                    v_head_stride=v.stride(1), tables=[tables] * hkv, packed=packed,
+                    packed_seq_stride=packed.stride(0), packed_head_stride=packed.stride(1), norms=norms,
+                    norms_seq_stride=norms.stride(0), norms_head_stride=norms.stride(1))
+        ws = torch.zeros(batched.workspace_bytes(batched.decode_desc(**args)), dtype=torch.uint8, device="cuda")
+        batched.decode(device, batched.decode_desc(workspace=ws, **args))
+        torch.cuda.synchronize()
+    finally:
+        tables.destroy()
+    perm, group_of = torch.tensor(np.asarray(p.permutation).astype(np.int64)), np.asarray(p.groupOf)
+    cent = torch.tensor(np.asarray(p.centroids, np.float32).reshape(dim, -1))
+    rot = torch.tensor(np.asarray(p.rotation, np.float32).reshape(dim, dim))
+    refs = {torch.float32: [], torch.float64: []}
+    largest = 0.0
+    for b in range(B):
+        for h in range(hkv):
+            pk = packed[b, h, :T * p.rowBytes].cpu().numpy().reshape(T, p.rowBytes)
+            codes = torch.tensor(oracle.unpack(pk, dim, p.nibbleDims).astype(np.int64))
+            c32 = cent[torch.arange(dim)[None], codes]
+            s32 = norms[b, h, :T * p.normStride].cpu().view(torch.float16).view(T, p.normStride)
+            for dt, got in refs.items():
+                qr = (q[b, h * G:(h + 1) * G].cpu().to(dt)[:, perm] @ rot.to(dt).t()) * torch.tensor(dim ** -0.5, dtype=dt)
+                lg = torch.zeros((G, T), dtype=dt)
+                for i in range(p.groups):
+                    own = torch.tensor(np.nonzero(group_of == i)[0])
+                    lg += (qr[:, own] @ c32.to(dt)[:, own].t()) * s32[:, i].to(dt)
+                largest = max(largest, lg.abs().max().item())
+                got.append(torch.softmax(lg, 1) @ v[b, h].cpu().to(dt))
+    assert 40 < largest < 150
+    ref = torch.cat(refs[torch.float64]).view(B, hq, dim)
+    plain = (torch.cat(refs[torch.float32]).view(B, hq, dim).double() - ref).norm() / ref.norm()
+    err = (out.cpu().double() - ref).norm() / ref.norm()
+    print(f"fp32 logits {layout} d{dim}: error {err:.2e}, plain FP32 {plain:.2e}, logits to {largest:.0f}", flush=True)
+    assert err <= 1.35 * plain, (err, plain)
+
+
 @pytest.mark.parametrize("batch,hkv,ctx,fewer", [
     (150, 2, 3000, 2),  # 300 units: three splits where the rounded-up count is two
     (150, 2, 3000, 0),
