@@ -1102,32 +1102,53 @@ static int choose_splits(int64_t units, uint32_t max_length, int32_t requested) 
 // round of their own. Cost in tokens of one workgroup: every round has a set-up
 // and merge worth 512 tokens (6 us), a full round its share of the sequence,
 // a last round filled to f 0.6 + 0.4 f of that (HBM feeds the fewer workgroups
-// faster). Fewest splits win ties within 1%. us per call, rounded up / this rule:
+// faster). us per call, rounded up / this rule, equal lengths:
 // 63 units x 8191 tokens (SmolLM2 heads) 35.7 (9) / 25.0 (8), 42 x 8191 22.4 (13) /
-// 17.5 (12), 200 x 8191 68.1 (3) / 53.4 (2), 120 x 2000 24.6 (5) / 18.1 (4), d=128
-// 40 x 5000 25.9 (13) / 23.4 (12); above half the slots 270 x 8000 102.8 (2) / 84.4
-// (3), 300 x 1000 19.8 (2) / 16.6 (1), 320 x 4000 53.6 (2) / 43.7 (3). More units
-// than slots keep one split (640 sequences of 250 to 2000 tokens 32.6 us, two
-// splits 37.0: the short ones' workgroups already make room). Lengths spread
-// over max/8 .. max gain less or lose a little, the host does not know them: 63
-// units 25.8 / 24.4, 120 x 2000 22.5 / 17.6, but 33 x 20000 28.6 / 29.1 and 380 x
-// 4000 38.7 / 40.2. extra: more
-// workgroups per unit beside the splits (an appended token's).
+// 17.5 (12), 200 x 8000 68.9 (3) / 56.1 (5), 120 x 2000 24.6 (5) / 18.1 (4), d=128
+// 40 x 5000 25.9 (13) / 23.4 (12), 300 x 1000 19.8 (2) / 16.6 (1), 320 x 4000 53.6 (2) /
+// 43.7 (3). More units than slots keep one split (640 sequences of 250 to 2000
+// tokens 32.6 us, two splits 37.0: the short ones' workgroups already make room).
+//
+// The host does not know the lengths. Where they spread over max/8 .. max, a
+// launch that leaves slots idle loses, so more splits within 8% of the cost
+// win if they fill the rounds better (5% of the slots): 198 x 5000 equal 44.2 (2:
+// 44.3), spread 37.8 (2: 42.0, rounded up 3: 37.9), 200 x 8000 spread 41.0 (2: 44.2,
+// 3: 43.1), 280 x 2500 32.9 (1: 32.3), spread 26.4 (28.5, 2: 27.1). And two or three
+// splits that overflow the slots by 2% at most are kept from 3000 tokens: only
+// equal lengths pay for the second round. 171 x 9000 (3) spread 48.2 (8: 55.8, 2:
+// 64.0), equal 78.3 (67.9, 69.6); 258 x 4000 (2) spread 35.5 (3: 42.8), equal 60.4 (52.6).
+// The rule still loses up to 11% to rounding up for spread lengths on the SmolLM2
+// heads at 360 to 378 units x 4000 (1: 57.1, 2: 53.8; equal 62.8 and 63.0, layout B
+// 42.3 and 41.6, equal 52.5 and 60.0).
+//
+// extra: workgroups per unit beside the splits (an appended token's one, which
+// holds its slot about as long as a history split's, encoding). There fewer
+// splits win ties within 3%: 63 x 8191 36.9 (9) / 29.4 (7), 128 x 1000 16.0 (4) / 12.9 (3),
+// 129 x 8192 64.0 (4) / 56.5 (6), 128 x 32768 172 (4) / 137 (7), 512 x 8192 171 (1) / 156 (3),
+// 450 x 4096 86.8 (2) with 103 (3) 2% cheaper by this count.
 static int fused_decode_splits(int64_t units, uint32_t max_length, int extra) {
   const int64_t max_splits = std::min<int64_t>(256, std::max<int64_t>(1, (max_length + 127) / 128));
   const int64_t slots = 2 * (int64_t)device_cus();
   const int64_t first = std::min(max_splits, std::max<int64_t>(1, slots / units - extra));
   const int64_t last = units > slots ? 1 : std::min(max_splits, std::max<int64_t>(first, 3 * slots / units));
-  int64_t best = first;
-  double best_cost = 0;
-  for (int64_t s = first; s <= last; ++s) {
+  auto cost = [&](int64_t s) {
     const int64_t wgs = units * (s + extra), full = wgs / slots, rest = wgs % slots;
     const double part = rest ? 0.6 + 0.4 * (double)rest / (double)slots : 0.0;
-    const double cost = ((double)full + part) * max_length / (double)s + 512.0 * (double)(full + (rest ? 1 : 0));
-    if (s == first || cost < 0.99 * best_cost) {
-      best = s;
-      best_cost = cost;
-    }
+    return ((double)full + part) * max_length / (double)s + 512.0 * (double)(full + (rest ? 1 : 0));
+  };
+  auto fill = [&](int64_t s) {
+    const int64_t wgs = units * s, rounds = (wgs + slots - 1) / slots;
+    return (double)wgs / (double)(rounds * slots);
+  };
+  const int64_t up = choose_splits(units, max_length, 0), over = units * up - slots;
+  if (!extra && (up == 2 || up == 3) && over > 0 && over <= slots / 50 && max_length >= 3000) return (int)up;
+  int64_t best = first;
+  for (int64_t s = first + 1; s <= last; ++s)
+    if (cost(s) < (extra ? 0.97 : 0.99) * cost(best)) best = s;
+  if (!extra) {
+    const int64_t cheapest = best;
+    for (int64_t s = cheapest + 1; s <= last; ++s)
+      if (cost(s) <= 1.08 * cost(cheapest) && fill(s) > fill(best) + 0.05) best = s;
   }
   return (int)best;
 }
@@ -1200,7 +1221,9 @@ bgtq_status bgtq_decode_workspace_size(const bgtq_decode_desc *d, size_t *bytes)
   if (bgtq_status s = validate_decode(d, &splits)) return s;
   if (!bytes) return fail(BGTQ_ERR_RANGE, "null output");
   const int64_t units = (int64_t)d->batch * d->kv_heads;
-  if (d->splits <= 0) splits = std::max(splits, fused_decode_splits(units, d->max_length, 0));
+  // For either entry point, so that a call's split does not depend on which one the workspace was sized for.
+  for (int extra = 0; extra < 2 && d->splits <= 0; ++extra)
+    splits = std::max(splits, fused_decode_splits(units, d->max_length, extra));
   *bytes = decode_ws(units, (int64_t)d->batch * d->q_heads, d->dim, splits).total;
   return BGTQ_OK;
 }

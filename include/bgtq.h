@@ -285,7 +285,7 @@ bgtq_status bgtq_decode_append(bgtq_context *ctx, const bgtq_decode_desc *d, con
  * the decode's workspace is a library-owned device array of
  * BGTQ_DECODE_SCRATCH_BYTES per device, held until the process ends and
  * resolved and cleared by bgtq_context_create (once per device). A launch
- * whose bgtq_decode_workspace_size exceeds it, or with more than
+ * whose partial results exceed it, or with more than
  * BGTQ_DECODE_COUNTER_UNITS (sequence, KV head) pairs, fails with
  * BGTQ_ERR_RANGE and queues nothing. Same kernels and results as
  * bgtq_decode. Every call on one
