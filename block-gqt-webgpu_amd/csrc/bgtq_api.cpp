@@ -1507,10 +1507,9 @@ static bgtq_status decode_impl(bgtq_context *ctx, const bgtq_decode_desc *d, con
 // ---------------------------------------------------------------- chunked prefill
 struct PrefillPlan {
   int tiles, tile_queries, ranges, range_blocks;
-  int64_t work;      // the most work of the launch, in the kernel's cost units
   size_t records;    // bytes of the workgroups' partial records
   size_t workspace;  // records, then the tile table (16 bytes per tile)
-  size_t operands;   // bytes of the built K operands and their exponents after those, 0 = built per tile
+  size_t operands;   // bytes of the built K operands and their exponents after those, 0 = the route is not taken
   int operand_blocks;
   bool rowwise;      // the fused decode kernel, units of 16 (row, head) query columns
   int qgroups;       // rowwise: units per (sequence, KV head)
@@ -1530,6 +1529,7 @@ struct PrefillPlan {
 // cache: the starts are device values) and by the kernel for the actual one;
 // split_tokens > 0 fixes the range length instead.
 // append: the chunk's rows are appended in the same launch (bgtq_prefill_append).
+static bool structured_layout(const bgtq_prefill_desc *d);
 static bgtq_status plan_prefill(const bgtq_prefill_desc *d, PrefillPlan *plan, bool append = false) {
   if (!d) return fail(BGTQ_ERR_RANGE, "null descriptor");
   if (d->batch < 1 || d->rows < 1 || d->kv_heads < 1 || d->kv_heads > kMaxKvHeads || d->q_heads < d->kv_heads ||
@@ -1620,22 +1620,41 @@ static bgtq_status plan_prefill(const bgtq_prefill_desc *d, PrefillPlan *plan, b
     ranges = std::min<int64_t>(2 * (int64_t)device_cus(), (w_max + kPrefillMinRange - 1) / kPrefillMinRange);
   }
   plan->ranges = (int)std::max<int64_t>(1, ranges);
-  plan->work = w_max;
   plan->range_blocks = (int)range_blocks;
   plan->records = plan->ranges > 1 ? sizeof(float) * (size_t)plan->ranges * 2 * tq * (d->dim + 2) : 0;
   const size_t info = plan->ranges > 1 ? 16 * (size_t)d->batch * d->kv_heads * plan->tiles : 0;
   plan->workspace = kPrefillCounterBytes + plan->records + info;
-  if (d->key_format == BGTQ_KEYS_PACKED && plan->tiles > 1 &&
-      prefill_operands_once(d->dim, false, nq, plan->tile_queries, w_max, device_cus())) {
-    plan->operand_blocks = (int)(((int64_t)d->max_length + 31) / 32);
-    const size_t blocks = (size_t)d->batch * d->kv_heads * plan->operand_blocks;
+  if (d->key_format == BGTQ_KEYS_PACKED && plan->tiles > 1) {
+    // Operands built once, where the layout and the books' LDS take that route.
+    bool once = prefill_operands_once(d->dim, structured_layout(d), nq, plan->tile_queries, w_max, device_cus());
+    for (int h = 0; h < d->kv_heads; ++h) {
+      const DevTables *T = d->tables[h]->h();
+      if (T->n_books * T->max_centroids * 4 > prefill_general_book_bytes(d->dim)) once = false;
+    }
+    const int64_t operand_blocks = ((int64_t)d->max_length + 31) / 32;
+    const size_t blocks = (size_t)(d->batch * operand_blocks) * d->kv_heads;
     const size_t bytes = blocks * 32 * 4 * d->dim + (blocks * 4 + 15) / 16 * 16;
-    if (bytes <= kPrefillOperandBytes) {
+    if (once && bytes <= kPrefillOperandBytes) {
       plan->workspace = (plan->workspace + 15) / 16 * 16;
+      plan->operand_blocks = (int)operand_blocks;
       plan->operands = bytes;
     }
   }
   return BGTQ_OK;
+}
+
+// Whether the packed layout is one whose structure the kernels have compiled
+// in (fast_layout without the buffers: a misaligned one takes no other route).
+static bool structured_layout(const bgtq_prefill_desc *d) {
+  DecodeParams p{};
+  p.kv_heads = d->kv_heads;
+  p.dim = d->dim;
+  p.G = d->q_heads / d->kv_heads;
+  p.key_format = 1;
+  p.v_dtype = BGTQ_DTYPE_F16;
+  FastLayout fl{};
+  int nn = 0, sg = 0;
+  return fast_layout(p, d->tables, &fl, &nn, &sg);
 }
 
 bgtq_status bgtq_prefill_workspace_size(const bgtq_prefill_desc *d, size_t *bytes) {
@@ -1790,14 +1809,8 @@ static bgtq_status prefill_impl(bgtq_context *ctx, const bgtq_prefill_desc *d, c
   p.part = reinterpret_cast<float *>(static_cast<uint8_t *>(d->workspace) + kPrefillCounterBytes);
   p.tile_info = reinterpret_cast<int32_t *>(static_cast<uint8_t *>(d->workspace) + kPrefillCounterBytes + plan.records);
   p.out = d->out;
-  // A workspace of the partials alone leaves the operands to each tile's own
-  // build, as do books beyond the build's LDS.
-  bool once = prefill_operands_once(d->dim, nn >= 0, (int64_t)d->rows * dp.G, plan.tile_queries, plan.work, device_cus());
-  for (int h = 0; h < d->kv_heads && d->key_format == BGTQ_KEYS_PACKED; ++h) {
-    const DevTables *T = d->tables[h]->h();
-    if (T->n_books * T->max_centroids * 4 > prefill_general_book_bytes(d->dim)) once = false;
-  }
-  if (plan.operands && d->workspace_bytes >= plan.workspace + plan.operands && once) {
+  // A workspace of the partials alone leaves the operands to each tile's own build.
+  if (plan.operands && d->workspace_bytes >= plan.workspace + plan.operands) {
     p.operand_blocks = plan.operand_blocks;
     p.operands = static_cast<uint8_t *>(d->workspace) + plan.workspace;
     p.operand_exp = reinterpret_cast<int32_t *>(

@@ -402,3 +402,27 @@ def test_operands_built_once_match_per_tile_build(device, oracle, layout, dim, h
             _check(got[b, sel][:, (hkv - 1) * G:], ref.astype(np.float64), f"b{b}")
     finally:
         cache.destroy()
+
+
+@pytest.mark.parametrize("layout,dim,hq,hkv,rows,max_length,built", [
+    ("B", 64, 14, 2, 4096, 32768, False), ("B", 64, 8, 8, 700, 32768, False),  # never at d=64
+    ("B", 128, 16, 1, 255, 131072, False), ("B", 128, 16, 1, 256, 131072, True),  # from 4096 queries
+    ("A", 64, 8, 2, 4096, 8192, True), ("A", 128, 8, 2, 64, 8192, True),
+])
+def test_operand_space_only_where_it_is_used(device, layout, dim, hq, hkv, rows, max_length, built):
+    """The workspace size holds room for the built K operands (4 dim bytes per token and KV head) exactly
+    where the launch builds them: layouts of compiled-in structure rarely do."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    tables = bgtq.Tables(device, (calibrate.layout_a if layout == "A" else calibrate.layout_b)(dim))
+    try:
+        t = torch.zeros(16, dtype=torch.uint8, device="cuda")  # addresses only: nothing is launched
+        need = batched.prefill_workspace_bytes(batched.prefill_desc(
+            batch=3, rows=rows, q_heads=hq, kv_heads=hkv, dim=dim, q=t, out=t, starts=t, max_length=max_length, v=t,
+            v_seq_stride=0, v_head_stride=0, tables=[tables] * hkv, packed=t, norms=t))
+        partials = 4 * 512 * 2 * 256 * (dim + 2) + 2 ** 20  # 512 workgroups' two records of 256 queries, counters, tiles
+        operands = 3 * hkv * max_length * 4 * dim
+        assert operands <= need <= operands + partials if built else need <= partials
+    finally:
+        tables.destroy()
