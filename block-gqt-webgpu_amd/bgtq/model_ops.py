@@ -38,17 +38,25 @@ assert _DISPATCH.size == ctypes.sizeof(_lib.ModelDispatch) and ctypes.sizeof(_li
 _NAMES = {n: ctypes.create_string_buffer(n.encode()) for n in ATTENTION_PATH}
 
 
+_TENSORS: set = set()  # torch's own tensor types, once met: no attributes to look for
+
+
 def _binding(b) -> tuple[int, int, int]:
     """bgtq_model_binding's words: device address, bytes, tables handle."""
+    if type(b) in _TENSORS:
+        if not b.is_contiguous():
+            raise RangeError("Model buffers must be contiguous")
+        return b.data_ptr(), b.nbytes, 0
     if b is None:
         return 0, 0, 0
-    torch = sys.modules.get("torch")
-    if torch is None or not isinstance(b, torch.Tensor):  # (a tensor's missing attribute is slow to look up)
-        handle = getattr(b, "handle", None)
-        if handle is not None and hasattr(b, "info"):  # calibration Tables
-            return 0, 0, getattr(handle, "value", handle) or 0
+    handle = getattr(b, "handle", None)
+    if handle is not None and hasattr(b, "info"):  # calibration Tables
+        return 0, 0, getattr(handle, "value", handle) or 0
     if not b.is_contiguous():
         raise RangeError("Model buffers must be contiguous")
+    torch = sys.modules.get("torch")
+    if torch is not None and type(b) in (torch.Tensor, torch.nn.Parameter):
+        _TENSORS.add(type(b))
     return b.data_ptr(), b.numel() * b.element_size(), 0
 
 
