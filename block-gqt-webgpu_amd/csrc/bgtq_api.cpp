@@ -1831,11 +1831,14 @@ bgtq_status bgtq_attention_create(bgtq_keys *k, bgtq_values *v, uint32_t max_que
   a->values = v;
   a->max_queries = max_queries;
   a->materialize = materialize ? 1 : 0;
-  // Splits of one 32-token chunk per wave of the fused kernel (4096 tokens, d=128,
-  // FP32 V, 3 queries: 20.6 us with two chunks per wave, 17.7 with one);
-  // the general kernel keeps 256 tokens.
-  const int64_t floor_tok = k->kind != BGTQ_KEYS_COMPRESSED && (k->dim == 64 || k->dim == 128) ? 128 : 256;
-  a->max_splits = (uint32_t)std::min<int64_t>(256, std::max<int64_t>(1, ((int64_t)k->capacity + floor_tok - 1) / floor_tok));
+  // Splits of one 32-token chunk per wave of the fused kernel, as long as one
+  // round of loads merges them all; past that, and for the general kernel, of
+  // two. us of GPU time per attend, 3 queries over FP32 V, two chunks / one:
+  // d=64 600 tokens 14.6 / 13.5, 4096 15.0 / 14.3; 8000 15.8 / 20.7, 16,000
+  // 24.1 / 31.0; d=128 600 21.5 / 20.2, 10,000 23.6 / 32.9.
+  const bool fused = k->kind != BGTQ_KEYS_COMPRESSED && (k->dim == 64 || k->dim == 128);
+  const int64_t one = ((int64_t)k->capacity + 127) / 128, two = ((int64_t)k->capacity + 255) / 256;
+  a->max_splits = (uint32_t)std::min<int64_t>(256, std::max<int64_t>(1, fused && one <= kDecodeMergeOneRound ? one : two));
   const size_t d = k->dim, Q = max_queries;
   bgtq_status s = k->ctx->use();
   struct Item {

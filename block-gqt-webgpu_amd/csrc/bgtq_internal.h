@@ -67,6 +67,7 @@ struct DevTables {
   //             two codes per packed byte.
 };
 constexpr int kMfmaTableBytes = 3072;
+constexpr int kDecodeMergeOneRound = 40;  // split counts the fused decode merges with a single round of loads
 constexpr int kPairSlots = 4;         // pair tables (2 KB each) the fused decode keeps in LDS
 constexpr int kLaneRecordWords = 44;
 constexpr int kCounterStride = 16;   // words between the decode's split counters (one per 64-byte line)  // words of one per-lane code-lookup record

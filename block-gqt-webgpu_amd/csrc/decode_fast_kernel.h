@@ -56,7 +56,7 @@ constexpr int kThreads = 64 * kWaves;
 constexpr int kChunk = 32;  // tokens per wave iteration: two 16-token MFMA tiles
 constexpr int kRing = 2;    // LDS chunk buffers per wave: compute one, the next in flight
 constexpr bool kInterleaved = true;
-constexpr int kMergeOneRound = 40;  // split counts merged with a single round of loads
+constexpr int kMergeOneRound = kDecodeMergeOneRound;
 
 // Kinds of launch of the fused kernel. Each kind's instances can sit in a
 // translation unit of their own, compiled with the scheduling options that

@@ -291,3 +291,29 @@ def test_record_with_timestamps(device, attention_cases):
         att.destroy()
         values.destroy()
         keys.destroy()
+
+
+@pytest.mark.parametrize("dim,tokens,splits", [(64, 1, 1), (64, 5120, 40), (64, 5121, 21), (128, 10000, 40)])
+def test_session_splits_stay_within_one_merge_round(device, oracle, dim, tokens, splits):
+    """A session's splits are as short as one 32-token chunk per wave only while a single round of loads
+    merges them (40); its partials' allocation says how many. Outputs against the oracle at both sides."""
+    import bgtq
+    rng = np.random.default_rng(tokens)
+    keys, values = bgtq.FP16Keys(device, dim, tokens), bgtq.Values(device, dim, tokens)
+    session = bgtq.AttentionEngine.create(device).session(keys, values, 3, False)
+    try:
+        part = [a["bytes"] for a in session.allocations if a["name"] == "split partials"]
+        assert part == [3 * splits * (dim + 2) * 4], session.allocations
+        k = (rng.standard_normal((tokens, dim)) * 0.7).astype(np.float16)
+        v = rng.standard_normal((tokens, dim)).astype(np.float32)
+        keys.append(k.view(np.uint16))
+        values.append(v)
+        q = rng.standard_normal((3, dim)).astype(np.float32)
+        pos = np.array([0, tokens // 2, tokens - 1], np.uint32)
+        out = session.attend(q, pos, True)
+        _, _, ref = oracle.attention(q, k.astype(np.float32), v, pos, True)
+        _close(out, ref, ATOL, RTOL, f"{tokens} tokens")
+    finally:
+        session.destroy()
+        values.destroy()
+        keys.destroy()
