@@ -186,6 +186,9 @@ struct bgtq_values {
   uint32_t dim = 0, capacity = 0, length = 0;
   int32_t dtype = BGTQ_DTYPE_F32;
   DeviceBuffer buf;
+  // FP32 V: some |v| >= 65504. Attention then computes QK in FP32 too (as the
+  // general kernel served such values), else with hi/lo operands.
+  bool large = false;
   Ledger ledger;
 };
 
@@ -825,6 +828,9 @@ bgtq_status bgtq_values_append(bgtq_values *v, const float *values, size_t n) {
     HIP_TRY(hipMemcpy(static_cast<float *>(v->buf.ptr) + (size_t)v->length * v->dim, values, n * 4,
                       hipMemcpyHostToDevice),
             "V upload");
+    bool large = false;  // (no branch in the loop: vector compares)
+    for (size_t i = 0; i < n; ++i) large |= std::fabs(values[i]) >= 65504.0f;
+    v->large |= large;
   } else {
     std::vector<uint16_t> h(n);
     for (size_t i = 0; i < n; ++i) h[i] = f32_to_f16(values[i]);
@@ -1239,9 +1245,9 @@ static bool fused_v(const DecodeParams &p) {
 }
 
 // KV head h's lookup tables and rotation as the fused kernel reads them: FP32
-// for FP32 V, else f16 hi/lo operands.
+// with qk_f32, else f16 hi/lo operands.
 static void fused_tables(const DecodeParams &p, const DevTables *T, const uint8_t *base, int h, FastLayout *fl) {
-  const bool f32 = p.v_dtype == BGTQ_DTYPE_F32;
+  const bool f32 = p.v_dtype == BGTQ_DTYPE_F32 && p.qk_f32;
   fl->mfma[h] = base + (f32 ? T->off_books : T->off_mfma);
   fl->rot_q[h] = base + (f32 ? T->off_rot : T->off_rot_q);
   fl->cent_exp[h] = f32 ? 0 : T->cent_exp;
@@ -1468,6 +1474,7 @@ static bgtq_status decode_impl(bgtq_context *ctx, const bgtq_decode_desc *d, con
   p.splits = splits;
   p.splits_forced = d->splits > 0;
   p.fused_splits = fused_splits;
+  p.qk_f32 = 1;
   p.split_tokens = (int)((d->max_length + p.splits - 1) / p.splits);
   p.split_tokens = ((p.split_tokens + 127) / 128) * 128;
   p.inv_sqrt_d = (float)(1.0 / std::sqrt((double)d->dim));
@@ -1946,6 +1953,7 @@ static bgtq_status attention_record(bgtq_attention *a, bgtq_timestamps *ts, uint
   }
   p.v = v->buf.ptr;
   p.v_dtype = v->dtype;
+  p.qk_f32 = v->large;
   p.qr = static_cast<float *>(a->qr.ptr);
   p.lengths = static_cast<const uint32_t *>(a->small.ptr);
   p.max_length = (int32_t)T;

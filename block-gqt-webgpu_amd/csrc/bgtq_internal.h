@@ -178,6 +178,7 @@ struct DecodeParams {
   int32_t v_dtype;  // 0 = FP32, 1 = FP16
   int32_t waves;          // decode workgroup waves of the fused kernel: 8 (d=64, few units), else 4
   int32_t splits_forced;  // the caller fixed the split count
+  int32_t qk_f32;           // FP32 V: the fused kernel rotates and multiplies packed K in FP32
   int32_t fused_splits;     // the fused kernel's splits, 0 = splits (bgtq_decode's general kernel always takes splits)
   int64_t v_seq_stride, v_head_stride;  // elements
   const float *q;         // [B*Hq*dim] queries
@@ -354,7 +355,7 @@ struct FastLayout {
   int32_t book[4];  // centroid book of each K-step
   // Per KV head, resolved on the host so the kernel's first loads need no
   // dependent read of the tables' header: the MFMA lookup tables, the
-  // permuted rotation's MFMA operands and cent_exp; for FP32 V the books'
+  // permuted rotation's MFMA operands and cent_exp; with qk_f32 the books'
   // FP32 centroids (max_centroids a row, gmc), the rotation as it is, and 0.
   const uint8_t *mfma[kMaxKvHeads];
   const uint8_t *rot_q[kMaxKvHeads];

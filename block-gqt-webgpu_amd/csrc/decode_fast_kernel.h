@@ -98,7 +98,7 @@ __host__ __device__ constexpr int swz32(int row) { return ((row >> 2) & 3) << 2;
 // to be read, and an append workgroup's slots keep its encoders' data.
 __host__ __device__ constexpr int prefill_stage_bytes(int D) { return 16 * (D + 4) * 4; }
 
-// VF: the V rows' format, 0 = FP16 (2 bytes per value), 1 = FP32 (4 bytes;
+// VF: the V rows' format, 0 = FP16 (2 bytes per value), 1, 2 = FP32 (4 bytes;
 // a ring of one slot per wave where two do not fit). NW: waves per workgroup.
 template <int D, int KF, int NN, int VF = 0, int NW = kWaves>
 struct Slot {
@@ -342,15 +342,16 @@ __device__ __forceinline__ void merge_rows(float *part, float *out, const MergeR
 // the first min(starts[b], max_length - rows) + row + 1 tokens. A unit uses
 // only as many of its splits as its history needs (p.split_floor tokens per
 // split at least); the others exit before their first chunk.
-// VF: V rows of FP32 values (1; decode without an appended token) or FP16
-// (0). FP32 V: the whole pass in FP32, as the general kernel computes it:
-// rotation, QK with the FP32 centroids and PV on the FP32 matrix cores,
-// logits in natural units (FP16 V: f16 matrix cores with hi/lo operands; so
-// also QK of FP16 K, whose values one f16 operand holds exactly). Error of the
-// output against 64 bits with |logits| up to about 60, general kernel / hi/lo
-// operands / this: layout A 6.6e-7 / 8.4e-7 / 5.7e-7, SmolLM2 heads 1.13e-6 /
-// 0.92e-6 / 0.72e-6, FP16 K 1.29e-6 / 0.74e-6 / the same; 8 sequences x 14
-// heads x 4096 tokens 57.7 / 18.1 / 20.3 us.
+// VF: V rows of FP16 values (0) or FP32 (1, 2; decode without an appended
+// token), whose PV products then run on the FP32 matrix cores, with logits in
+// natural units. 1: the whole pass in FP32, as the general kernel computes it,
+// also rotation and QK with the FP32 centroids (batched calls, sessions with
+// large V); 2: rotation and QK with hi/lo operands as for FP16 V (sessions).
+// FP16 K: QK with hi/lo queries in both, its values being exact in one f16
+// operand. Error of the output against 64 bits with |logits| up to about 60,
+// general kernel / hi/lo operands / FP32: layout A 5.8e-7 / 7.9e-7 / 5.7e-7,
+// SmolLM2 heads 9.4e-7 / 8.0e-7 / 6.5e-7, FP16 K 1.24e-6 / 0.69e-6; 8 sequences
+// x 14 heads x 4096 tokens 57.7 / 18.1 / 20.3 us.
 // NW: waves per workgroup (4; row-wise prefill at d=64, 8: a unit's splits
 // then cover twice the tokens each and half as many partials are merged).
 // Every kernel argument the set-up reads, loaded at once (one asm statement,
@@ -389,7 +390,7 @@ __device__ __forceinline__ void decode_fast_body(const DecodeParams &p, const Fa
   constexpr int KS = Gm::KS, DT = Gm::DT, PR = Gm::PR, VI = Sl::VI, KRI = Gm::KRI;
   constexpr int VB = VF ? 4 : 2;  // bytes per V value
   constexpr bool NAT = VF != 0;                // logits in natural units, else log2 domain
-  constexpr bool F32 = VF && KF >= 1;          // rotation and QK in FP32
+  constexpr bool F32 = VF == 1 && KF >= 1;     // rotation and QK in FP32
   constexpr float kLogit = NAT ? 1.0f : kLn2;  // a logit's natural value
   // P is carried times 2^15 where it is split into FP16 parts; unscaled for FP32 V.
   constexpr float kPShift = VF ? 0.0f : 15.0f, kPFactor = VF ? 1.0f : kPScale;
@@ -1954,9 +1955,13 @@ hipError_t launch_one(const DecodeParams &p, const FastLayout &fl, hipStream_t s
   if (!(kind & KINDS)) return hipErrorInvalidValue;
   if (p.v_dtype == BGTQ_DTYPE_F32) {
     if constexpr ((KINDS & kKindDecode) != 0)
-      if (kind == kKindDecode)
-        return p.logits ? launch_mode<D, KF, NN, SG, 0, 0, 1, kWaves, 2>(p, fl, stream)  // (FP32 centroids: no pairs)
+      if (kind == kKindDecode && (KF == 0 || p.qk_f32))  // (FP32 centroids: no pairs)
+        return p.logits ? launch_mode<D, KF, NN, SG, 0, 0, 1, kWaves, 2>(p, fl, stream)
                         : launch_mode<D, KF, NN, SG, 0, 0, 1, kWaves, 0>(p, fl, stream);
+    if constexpr ((KINDS & kKindDecode) != 0 && KF >= 1)
+      if (kind == kKindDecode)
+        return p.logits ? launch_mode<D, KF, NN, SG, PK, 0, 2, kWaves, 2>(p, fl, stream)
+                        : launch_mode<D, KF, NN, SG, PK, 0, 2, kWaves, 0>(p, fl, stream);
     return hipErrorInvalidValue;
   }
   if constexpr ((KINDS & kKindDecode) != 0)

@@ -142,9 +142,10 @@ void bgtq_keys_destroy(bgtq_keys *k);
 /* ---- Values (src/runtime/values.ts:3-16) --------------------------------- *
  * dtype BGTQ_DTYPE_F32 stores FP32 V exactly (the synthetic path); F16 stores
  * RNE-rounded FP16 V (src/model/append.wgsl:6-10). append() is synchronous.
- * Attention over F32 V runs on the fused kernel, in FP32 throughout (packed K
- * from its FP32 centroids; FP16 K rows, exact in one FP16 operand, against
- * queries as pairs of FP16 values of 22 bits or more). */
+ * Attention over F32 V runs on the fused kernel, its PV products on the FP32
+ * matrix cores; packed K is multiplied in FP32 too once an appended |v| is
+ * 65504 or more, else by queries and centroids as pairs of FP16 values (22 bits
+ * or more). bgtq_decode over F32 V multiplies packed K in FP32 always. */
 typedef struct bgtq_values bgtq_values;
 bgtq_status bgtq_values_create(bgtq_context *ctx, uint32_t dim, uint32_t capacity, int32_t dtype,
                                bgtq_values **out);

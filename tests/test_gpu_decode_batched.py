@@ -473,6 +473,51 @@ def test_fp32_values_keep_fp32_logits(device, oracle, layout, dim, hq, hkv):
     assert err <= 1.35 * plain, (err, plain)
 
 
+def test_session_with_large_values_keeps_fp32_logits(device, oracle):
+    """A session whose V reaches 65504 multiplies packed K in FP32 too: the bound above, over sixteen
+    queries of three sessions, with logits of up to about 80."""
+    import torch
+    import bgtq
+    from bgtq import calibrate
+    p = calibrate.layout_a(64)
+    rng = np.random.default_rng(8)
+    T, errs, plains, norms2 = 1500, 0.0, 0.0, 0.0
+    tables = bgtq.Tables(device, p)
+    for _ in range(3):
+        keys, values = bgtq.PackedKeys(device, tables, T), bgtq.Values(device, 64, T)
+        session = bgtq.OptimizedAttention.create(device, keys, values, 16, materialize=False)
+        try:
+            keys.append(rng.standard_normal((T, 64)).astype(np.float16).view(np.uint16))
+            v = (rng.standard_normal((T, 64)) * 1e5).astype(np.float32)
+            values.append(v[:700])
+            values.append(v[700:])
+            q = (rng.standard_normal((16, 64)) * 15).astype(np.float32)
+            out = torch.tensor(session.attend(q, np.zeros(16, np.uint32), False)).double()
+            packed, norms = keys.read()
+        finally:
+            session.destroy()
+            values.destroy()
+            keys.destroy()
+        codes = torch.tensor(oracle.unpack(packed[:T * p.rowBytes].reshape(T, -1), 64, p.nibbleDims).astype(np.int64))
+        c = torch.tensor(np.asarray(p.centroids, np.float32).reshape(64, -1))[torch.arange(64)[None], codes]
+        scale = torch.tensor(norms[:T * p.normStride].reshape(T, -1).view(np.float16).astype(np.float32))
+        perm, rot = np.asarray(p.permutation), torch.tensor(np.asarray(p.rotation, np.float32).reshape(64, 64))
+        outs = []
+        for dt in (torch.float32, torch.float64):
+            qr = (torch.tensor(q[:, perm]).to(dt) @ rot.to(dt).t()) * 0.125
+            lg = torch.zeros((16, T), dtype=dt)
+            for i in range(p.groups):
+                own = torch.tensor(np.nonzero(np.asarray(p.groupOf) == i)[0])
+                lg += (qr[:, own] @ c.to(dt)[:, own].t()) * scale[:, i].to(dt)
+            outs.append((torch.softmax(lg, 1) @ torch.tensor(v).to(dt)).double())
+        errs += float(((out - outs[1]) ** 2).sum())
+        plains += float(((outs[0] - outs[1]) ** 2).sum())
+        norms2 += float((outs[1] ** 2).sum())
+    tables.destroy()
+    print(f"large V session: error {(errs / norms2) ** 0.5:.2e}, plain FP32 {(plains / norms2) ** 0.5:.2e}", flush=True)
+    assert errs <= 1.35 ** 2 * plains
+
+
 @pytest.mark.parametrize("batch,hkv,ctx,fewer", [
     (150, 2, 3000, 2),  # 300 units: three splits where the rounded-up count is two
     (150, 2, 3000, 0),
