@@ -269,13 +269,17 @@ constexpr int kPrefillSegmentCost = 4;    // cost units of a tile's set-up (a 32
 // us per call, once / per tile (MI355X, same outputs bit for bit):
 //   any packed layout, d=128: 33 rows x 4 heads after 2000 tokens 26.5 / 29.2, 1001 rows x 4 after 3077 77 / 343: always;
 //   any packed layout, d=64: with 256-query tiles (1001 rows x 3 heads after 3077 tokens 54.8 / 81.2); with 64-query
-//   tiles from eight cost units per workgroup (SmolLM2 heads, 3 KV heads: 200 rows after 3896 32.9 / 33.7, 600 after 3496
-//   42.9 / 52.3; below it the build launch costs more than it saves, 600 after 0 22.9 / 21.6);
+//   tiles, ten or more of them per KV head from eight cost units per workgroup (SmolLM2 heads, 3 KV heads: 200 rows
+//   after 3896 32.9 / 33.7, 600 after 3496 42.9 / 52.3; below eight the build launch costs more than it saves, 600
+//   after 0 22.9 / 21.6). Fewer tiles build K too few times: in a cache of 16384 tokens 64 rows (3 tiles) after 8160
+//   34.1 / 29.4, 150 rows (8) after 4058 30.6 / 29.2 and after 16234 49.2 / 54.5; 200 rows (10) after 4046 32.3 / 32.5, after
+//   8092 40.7 / 43.6, after 16184 56.4 / 66.1. The host knows the cache's length only: a chunk at its start pays
+//   1.1 us (340 rows after 0 17.0 / 15.9, after 8022 47.3 / 53.6);
 //   structured layouts build cheaply per tile: d=128 2100 queries 37.9 / 36.5, 4200 73.2 / 76.8, 14336 79.1 / 87.6;
 //   d=64 28672 queries 109.4 / 110.1, 2100 27.2 / 24.6: never.
 constexpr bool prefill_operands_once(int dim, bool structured, int64_t queries, int tile_queries, int64_t work, int cus) {
   if (dim == 128) return !structured || queries >= 4096;
-  return !structured && (tile_queries > 64 || work >= 8 * 2 * (int64_t)cus);
+  return !structured && (tile_queries > 64 || (queries > 9 * 64 && work >= 8 * 2 * (int64_t)cus));
 }
 // Cost units of a d=64 launch (256-query tiles) below which its tiles hold 64 queries: with at most 8.5 per workgroup
 // the short tiles' more even ranges, quicker set-up and four waves a SIMD outweigh K streamed four times as often.

@@ -356,7 +356,7 @@ def test_workspace_shared_across_paths(device, oracle):
 
 @pytest.mark.parametrize("layout,dim,hq,rows,starts", [
     ("S", 64, 9, 683, [0, 300]),      # 64-query tiles past 2048 queries, odd lengths
-    ("A", 64, 8, 129, [1, 3500]),     # few queries, a history long enough, one starting a token into a block
+    ("A", 64, 8, 145, [1, 3500]),     # ten 64-query tiles, a history long enough, one starting a token into a block
     ("S", 64, 9, 1025, [0, 1801]),    # 256-query tiles
     ("A", 128, 2, 65, [0, 158]),      # two 64-query tiles, the smallest launch of this route
     ("A", 128, 8, 513, [31, 64]),
@@ -408,6 +408,7 @@ def test_operands_built_once_match_per_tile_build(device, oracle, layout, dim, h
     ("B", 64, 14, 2, 4096, 32768, False), ("B", 64, 8, 8, 700, 32768, False),  # never at d=64
     ("B", 128, 16, 1, 255, 131072, False), ("B", 128, 16, 1, 256, 131072, True),  # from 4096 queries
     ("A", 64, 8, 2, 4096, 8192, True), ("A", 128, 8, 2, 64, 8192, True),
+    ("A", 64, 8, 8, 576, 32768, False), ("A", 64, 8, 8, 577, 32768, True),     # from ten 64-query tiles
 ])
 def test_operand_space_only_where_it_is_used(device, layout, dim, hq, hkv, rows, max_length, built):
     """The workspace size holds room for the built K operands (4 dim bytes per token and KV head) exactly
