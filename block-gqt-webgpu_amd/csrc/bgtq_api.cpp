@@ -877,10 +877,6 @@ constexpr int kEncodeTile = 3;  // encoder kind beside encode_bulk_kind's
 // From this many rows a call's jobs go through the context's device table.
 constexpr int64_t kEncodeTableRows = 16384;
 static int64_t encode_wave_max_rows(int dim, bool tile) { return !tile ? kEncodeTableRows : dim == 64 ? 8192 : 4096; }
-// Layout B at d=64 from this many rows: the thread-per-row encoder with the
-// layout's structure at compile time (51 us for 368,640 rows, 57 with the tile
-// encoder; 44 against 41 for 262,144, 20 against 13 for 32,768).
-constexpr int64_t kEncodeBulkMinRows = 300000;
 
 }  // extern "C"
 
@@ -915,37 +911,74 @@ struct EncodeExtents {
   }
 };
 
+// us of a tile encoder call of `walk` passes of the longest part's workgroups
+// and `load` passes of every resident workgroup on average. Measured, with
+// the upload of a table's jobs: layout B d=64 64 x 1000 rows (walk 1, load 1)
+// 19, 48 x 1500 (2, 1.1) 21, 24 x 8192 (4, 3) 37.5, 64 x 4096 (4, 4) 45;
+// layout A d=128 90 x 2048 (8, 5.6) 118.
+double tile_us(int dim, double walk, double load) {
+  return dim == 64 ? 9.8 + 2.2 * walk + 6.3 * load : 13.0 + 12.4 * std::max(walk, load);
+}
+
+// us of a bulk encoder call of `wgs` workgroups (256 rows each) on `slots` of them,
+// `idle` more that leave at once: a round's time hardly depends on its fill
+// (96,000 rows 24, 192,000 29, 200,000 43, 288,000 47; FP32 source 210,000 rows 51).
+double bulk_us(int64_t wgs, int64_t idle, int64_t slots, bool src_f32) {
+  const double us = 4.2 + 14.5 * (double)((wgs + slots - 1) / slots) + 8.0 * (double)wgs / (double)slots;
+  return (src_f32 ? 1.2 * us : us) + 0.0025 * (double)idle;
+}
+
+constexpr double kEncodeUploadUs = 1.7;  // one upload launch into the job table
+
 // The tile encoder shares the chip equally among a launch's jobs, so a job
 // much longer than the others would be walked by few workgroups while theirs
-// have left: long jobs are cut into parts, as short as lets all parts go with
-// one more upload or launch at most, where that shortens the longest walk
-// (jobs of one length stay whole). us per call without / with the cut: SmolLM2
-// heads 8000 + 50 x 20 rows 39.7 / 18.0, 90 jobs of 10 to 4096 rows 56.0 / 43.8,
-// 32768 + 1023 x 1 1935 / 73; d=128 layout A 16384 + 511 x 1 1589 / 64.
-void cut_long_jobs(std::vector<EncodePart> &parts, int64_t total_rows, int64_t wg_rows, int64_t resident,
-                   size_t per_launch) {
-  auto walk = [&](int64_t rows, size_t n) {  // passes of the workgroups of the longest part
-    const int64_t wgs = std::max<int64_t>(1, resident / (int64_t)n);
-    return (rows + wgs * wg_rows - 1) / (wgs * wg_rows);
+// have left: long jobs are cut into parts where the shorter walk is worth the
+// uploads or launches of more jobs. Jobs of up to twice the mean length stay
+// whole (90 x 2048 at d=128 118, cut 157). Returns the estimated us. us per call
+// without / with the cut: SmolLM2 heads 8000 + 50 x 20 rows 40 / 12.6, 90 jobs
+// of 10 to 4096 rows 56 / 38, 32768 + 1023 x 1 1914 / 55; d=128 layout A
+// 16384 + 511 x 1 1573 / 65.
+double cut_long_jobs(std::vector<EncodePart> &parts, int dim, int64_t resident, bool in_args) {
+  const int64_t wg_rows = encode_tile_wg_rows(dim);
+  const size_t per_launch = in_args ? kTileJobsPerLaunch : kEncodeJobsPerLaunch;
+  int64_t longest = 0, total = 0, passes = 0;
+  for (const EncodePart &p : parts) {
+    longest = std::max(longest, p.rows);
+    total += p.rows;
+    passes += (p.rows + wg_rows - 1) / wg_rows;
+  }
+  auto estimate = [&](int64_t rows, size_t n) {
+    const double launches = (double)((n + per_launch - 1) / per_launch);
+    const size_t together = in_args ? std::min(n, per_launch) : n;
+    const int64_t wgs = std::max<int64_t>(1, resident / (int64_t)together);
+    const double walk = (double)((rows + wgs * wg_rows - 1) / (wgs * wg_rows));
+    // (more jobs than workgroups fit: rounds of set-ups, each worth about a pass)
+    const double rounds = (double)together / (double)resident, load = (double)passes / (double)resident;
+    if (in_args) return launches * tile_us(dim, walk, load / launches);
+    return tile_us(dim, rounds > 1.0 ? std::max(walk, load + rounds) : walk, load) + launches * kEncodeUploadUs;
   };
-  int64_t longest = 0;
-  for (const EncodePart &p : parts) longest = std::max(longest, p.rows);
-  const int64_t now = walk(longest, parts.size());
-  if (now <= 1 || now <= (total_rows + wg_rows * resident - 1) / (wg_rows * resident)) return;
-  const size_t budget = (parts.size() + per_launch / 2 + per_launch - 1) / per_launch * per_launch;
+  double best = estimate(longest, parts.size());
+  if ((double)longest * (double)parts.size() <= 2.0 * (double)total) return best;
+  const double floor = tile_us(dim, (double)((passes + resident - 1) / resident), (double)passes / (double)resident);
+  if (best - floor < kEncodeUploadUs * (1.0 + (double)((parts.size() - 1) / per_launch))) return best;
+  int64_t piece = 0;
   for (int64_t k = 1; k * wg_rows < longest; k += std::max<int64_t>(1, k / 4)) {
-    const int64_t piece = k * wg_rows;
     size_t n = 0;
-    for (const EncodePart &p : parts) n += (size_t)((p.rows + piece - 1) / piece);
-    if (n > budget) continue;
-    if (walk(piece, n) >= now) return;
+    for (const EncodePart &p : parts) n += (size_t)((p.rows + k * wg_rows - 1) / (k * wg_rows));
+    if (n > kEncodeJobTable) continue;
+    const double t = estimate(k * wg_rows, n);
+    if (t < best - 1.0) {
+      best = t;
+      piece = k * wg_rows;
+    }
+  }
+  if (piece) {
     std::vector<EncodePart> cut;
-    cut.reserve(n);
     for (const EncodePart &p : parts)
       for (int64_t r = 0; r < p.rows; r += piece) cut.push_back({p.job, r, std::min(piece, p.rows - r)});
     parts.swap(cut);
-    return;
   }
+  return best;
 }
 
 }  // namespace
@@ -1011,7 +1044,6 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
       tile &= jobs[i].tables->tile_encode && jobs[i].src_row_stride <= kTileMaxStride;
       wave_lds = std::max(wave_lds, encode_wave_lds_bytes(dim, (int)jobs[i].tables->h()->off_rot));
     }
-    if (kind == 1 && total_rows >= kEncodeBulkMinRows) tile = false;
     if (wave_lds <= 160 * 1024 && total_rows < encode_wave_max_rows(dim, tile)) {
       for (size_t b = 0; b < idx.size(); b += kEncodeJobsPerLaunch) {
         EncodeLaunch L{};
@@ -1038,10 +1070,28 @@ bgtq_status bgtq_encode_batched(bgtq_context *ctx, int32_t src_dtype, const bgtq
       all.add(parts.back());
     }
     const bool in_args = tile && total_rows < kEncodeTableRows;
-    if (tile && all.tile_fits(dim))
-      cut_long_jobs(parts, total_rows, encode_tile_wg_rows(dim),
-                    encode_tile_resident(dim, src_f32, device_cus(), all.tile),
-                    in_args ? kTileJobsPerLaunch : kEncodeJobsPerLaunch);
+    const bool bulk = kind == 1 && !in_args && encode_bulk_lds_bytes(all.lut, all.books) <= 64 * 1024;
+    if (tile && all.tile_fits(dim)) {
+      const std::vector<EncodePart> whole = parts;
+      const double tile_time = cut_long_jobs(parts, dim, encode_tile_resident(dim, src_f32, device_cus(), all.tile), in_args);
+      if (bulk) {
+        // Layout B at d=64: the thread-per-row encoder with the layout's
+        // structure at compile time where its rounds fit the rows better. us,
+        // thread per row / tile: 48 x 1500 rows 23.0 / 20.7, 24 x 4096 23.9 /
+        // 25.3, 24 x 8192 28.8 / 37.5, 2 x 100,000 43.4 / 37.8, 64 x 4096 48 / 45.3,
+        // 24 x 12,000 47.1 / 49.3.
+        const int lds = encode_bulk_lds_bytes(all.lut, all.books);
+        int64_t wgs = 0;
+        for (const EncodePart &p : whole) wgs += (p.rows + 255) / 256;
+        const int64_t grid = (all.rows + 255) / 256 * (int64_t)whole.size();
+        const int64_t slots = (int64_t)device_cus() * std::max(1, std::min(3, 160 * 1024 / lds));
+        const double uploads = kEncodeUploadUs * (double)((whole.size() + kEncodeJobsPerLaunch - 1) / kEncodeJobsPerLaunch);
+        if (bulk_us(wgs, grid - wgs, slots, src_f32) + uploads < tile_time) {
+          tile = false;
+          parts = whole;
+        }
+      }
+    }
     if (in_args) {
       for (size_t b = 0; b < parts.size();) {
         // Up to kTileJobsPerLaunch parts whose tables fit the LDS together (any job's alone do).

@@ -35,9 +35,9 @@
 // and four groups), the LDS reads of their operands and of the code table,
 // and the vector instructions take about equal time. 368,640 rows of the 90
 // SmolLM2 calibration heads: 77 us, 331 with a thread per row (encode.hip);
-// 262,144 rows of layout B 41 us, 44 with its compile-time structure
-// (encode_bulk.hip, which is ahead again above 300,000 rows: 51 against 57 us
-// at 368,640); d=128 layouts 103-117 us for 184,320 rows, 137 and 624 before.
+// 262,144 rows of layout B 45 us, 48 with its compile-time structure
+// (encode_bulk.hip, ahead where its rounds of 196,608 rows are well filled: 29
+// against 37.5 us for 196,608, 51 against 57 for 368,640); d=128 layouts 103-117 us for 184,320 rows, 137 and 624 before.
 #include <hip/hip_fp16.h>
 
 #include "bgtq_internal.h"

@@ -248,31 +248,39 @@ def test_bulk_layout_b_encoder_bit_exact(device, oracle):
 
 
 def test_bulk_encoder_unaligned_source(device, oracle):
-    """The bulk encoder stages rows as 16-byte pieces when the source and its row stride allow it; a
-    source starting one element past a 16-byte boundary with an odd row stride takes its element-wise
-    staging, FP16 and FP32, over a partial last workgroup of rows."""
+    """The bulk encoder stages rows as 16-byte pieces when the source and its row stride allow it, else
+    element-wise: 190,004 rows of layout B (one round of its workgroups) in three jobs, one starting past
+    a 16-byte boundary with an odd stride, one with padded rows, one with only its start unaligned, FP16
+    and FP32, partial last workgroups, offset destinations with guard rows on both sides."""
     import torch
     import bgtq
     from bgtq import batched, calibrate
     rng = np.random.default_rng(321)
-    dim, rows = 64, 1000
-    stride = dim + 1
+    dim, guard = 64, 2
     p = calibrate.layout_b(dim)
-    k = _random_half_rows(rng, rows, dim)
+    shapes = ((90001, dim + 1, 1, 3), (60000, dim + 8, 0, 0), (40003, dim, 3, 1))  # rows, stride, lead, row0
+    ks = [_random_half_rows(rng, rows, dim) for rows, *_ in shapes]
+    refs = [oracle.encode_pack(_olayout(oracle, p), np.ascontiguousarray(k)) for k in ks]
     tables = bgtq.Tables(device, p)
     try:
-        ref_p, ref_n = oracle.encode_pack(_olayout(oracle, p), np.ascontiguousarray(k))
         for src_kind in ("f16", "f32"):
-            flat = np.zeros(1 + rows * stride, dtype=np.float16)
-            flat[1:].reshape(rows, stride)[:, :dim] = k.view(np.float16)
-            src = torch.from_numpy(flat.view(np.int16) if src_kind == "f16" else flat.astype(np.float32)).cuda()
-            packed = torch.zeros((rows, p.rowBytes), dtype=torch.uint8, device="cuda")
-            norms = torch.zeros((rows, p.normStride), dtype=torch.int16, device="cuda")
-            batched.encode(device, [dict(tables=tables, src=src[1:], src_row_stride=stride, rows=rows, packed=packed,
-                                         norms=norms, dst_row0=0)], src_kind)
+            jobs = []
+            for (rows, stride, lead, row0), k in zip(shapes, ks):
+                flat = np.zeros(lead + rows * stride, dtype=np.float16)
+                flat[lead:].reshape(rows, stride)[:, :dim] = k.view(np.float16)
+                src = torch.from_numpy(flat.view(np.int16) if src_kind == "f16" else flat.astype(np.float32)).cuda()
+                n = row0 + rows + guard
+                jobs.append(dict(tables=tables, src=src[lead:], src_row_stride=stride, rows=rows, dst_row0=row0,
+                                 packed=torch.full((n, p.rowBytes), 0xA5, dtype=torch.uint8, device="cuda"),
+                                 norms=torch.full((n, p.normStride), 0x5A5A, dtype=torch.int16, device="cuda")))
+            batched.encode(device, jobs, src_kind)
             device.synchronize()
-            assert np.array_equal(packed.cpu().numpy(), ref_p), src_kind
-            assert np.array_equal(norms.cpu().numpy().view(np.uint16), ref_n), src_kind
+            for j, (rows, _, _, row0), (ref_p, ref_n) in zip(jobs, shapes, refs):
+                got_p, got_n = j["packed"].cpu().numpy(), j["norms"].cpu().numpy().view(np.uint16)
+                outside = np.r_[0:row0, row0 + rows:len(got_p)]
+                assert np.all(got_p[outside] == 0xA5) and np.all(got_n[outside] == 0x5A5A), (src_kind, rows)
+                assert np.array_equal(got_p[row0:row0 + rows], ref_p), (src_kind, rows)
+                assert np.array_equal(got_n[row0:row0 + rows], ref_n), (src_kind, rows)
     finally:
         tables.destroy()
 
@@ -410,13 +418,13 @@ def test_nonfinite_rows_keep_to_their_groups(device, oracle, dim, name):
 
 
 def test_bulk_layout_b_largest_calls(device, oracle):
-    """Layout B at d=64 from 300,000 rows a call: the thread-per-row encoder with the layout's structure
-    compiled in, FP16 and FP32 sources, a partial last workgroup."""
+    """Layout B at d=64 where the thread-per-row encoder's second round of workgroups is well filled: FP16
+    and FP32 sources, a partial last workgroup."""
     import torch
     import bgtq
     from bgtq import batched, calibrate
     rng = np.random.default_rng(5)
-    p, rows = calibrate.layout_b(64), 300077
+    p, rows = calibrate.layout_b(64), 380077
     k = _random_half_rows(rng, rows, 64)
     ref_p, ref_n = oracle.encode_pack(_olayout(oracle, p), k)
     tables = bgtq.Tables(device, p)
