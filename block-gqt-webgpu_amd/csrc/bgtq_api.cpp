@@ -867,12 +867,13 @@ static int device_cus() {
   return cached[dev];
 }
 
-// Below a number of rows per launch the wave-per-row encoder (short latency
+// Below a number of rows per call the wave-per-row encoder (short latency
 // per row) runs, above it an encoder that takes more rows per instruction.
-// Measured in microseconds per call, wave against tile encoder: d=64, 6144
-// rows 9.4 / 11.4, 12,288 rows 13.3 / 11.1; d=128, 1000 rows 9.5 / 23.9, 8000
-// rows 44.2 / 21.9. The thread-per-row encoder of the layouts the tile encoder
-// does not take starts later.
+// Measured in us per call, wave against tile encoder, 1 to 24 jobs: d=64,
+// 4000 rows 7.8 / 8.7-10.8, 8000 rows 11.0 / 8.8-11.0 (90 jobs, two wave
+// launches, 15.4 / 8.9-11.2); d=128, 1000 rows 9.2-14.4 / 16.5-23.0, 4000 rows
+// 27.5 / 21.1-23.3. The line for the thread-per-row encoder of the layouts the
+// tile encoder does not take is kEncodeTableRows.
 constexpr int kEncodeTile = 3;  // encoder kind beside encode_bulk_kind's
 // From this many rows a call's jobs go through the context's device table.
 constexpr int64_t kEncodeTableRows = 16384;

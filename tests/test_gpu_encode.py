@@ -171,8 +171,8 @@ def test_append_contracts(device, attention_cases):
 
 
 def test_bulk_encode_bit_exact(device, oracle):
-    """A launch of at least 16384 rows takes the thread-per-row encoder (smaller
-    launches the wave-per-row one); both must give the oracle's bytes."""
+    """From 16384 rows a call leaves the wave-per-row encoder: d=16 takes the thread-per-row one, the d=64
+    and d=128 layouts here the tile encoder through the device job table."""
     import torch
     import bgtq
     from bgtq import batched
@@ -197,15 +197,15 @@ def test_bulk_encode_bit_exact(device, oracle):
 
 
 def test_bulk_layout_b_encoder_bit_exact(device, oracle):
-    """Layout B tables (two equal groups, nibbles first) take the bulk encoder with the layout's structure
-    compiled in: FP16 and FP32 sources, interleaved heads (row stride above dim), an offset destination,
-    a launch that also carries a job of another layout kind, and at d=64 a launch large enough for
-    the wide (256-row) workgroups."""
+    """Layout B tables (two equal groups, nibbles first), FP16 and FP32 sources, interleaved heads (row
+    stride above dim), an offset destination. d=64: 270,000 rows, where FP16 sources take the bulk encoder
+    with the layout's structure compiled in and FP32 sources the tile encoder, in a call that also carries
+    a job of another layout kind. d=128: the tile encoder."""
     import torch
     import bgtq
     from bgtq import batched, calibrate
     rng = np.random.default_rng(123)
-    other = _layouts(oracle)[2][1]  # mixed_d64: the generic encoder in the same call
+    other = _layouts(oracle)[2][1]  # mixed_d64: a launch of its own in the same call
     for dim in (64, 128):
         p = calibrate.layout_b(dim)
         print("bulk layout B", dim, flush=True)
@@ -245,6 +245,48 @@ def test_bulk_layout_b_encoder_bit_exact(device, oracle):
             tables.destroy()
             if t_other is not None:
                 t_other.destroy()
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_generic_encoder_bit_exact(device, oracle, dim):
+    """A group boundary at an odd position is for neither the tile encoder nor the one with layout B's
+    structure: from 16384 rows a call takes the generic thread-per-row encoder. Two jobs, one of them
+    unaligned with an odd stride, FP16 and FP32, offset destinations with guard rows on both sides."""
+    import torch
+    import bgtq
+    from bgtq import batched, calibrate
+    rng = np.random.default_rng(64 + dim)
+    p, cut = calibrate.layout_b(dim), dim // 2 - 1
+    assert np.array_equal(p.groupOf, np.arange(dim) >= dim // 2)
+    p.groupOf = (np.arange(dim) >= cut).astype(np.uint32)
+    rot = np.zeros((dim, dim), np.float32)
+    rot[:cut, :cut], rot[cut:, cut:] = calibrate.haar_rotation(cut, 1), calibrate.haar_rotation(dim - cut, 2)
+    p.rotation = rot.reshape(-1)
+    shapes = ((9001, dim + 1, 1, 3), (8000, dim, 0, 0))  # rows, stride, lead, row0
+    ks = [_random_half_rows(rng, rows, dim) for rows, *_ in shapes]
+    refs = [oracle.encode_pack(_olayout(oracle, p), k) for k in ks]
+    tables = bgtq.Tables(device, p)
+    try:
+        for src_kind in ("f16", "f32"):
+            jobs = []
+            for (rows, stride, lead, row0), k in zip(shapes, ks):
+                flat = np.zeros(lead + rows * stride, dtype=np.float16)
+                flat[lead:].reshape(rows, stride)[:, :dim] = k.view(np.float16)
+                src = torch.from_numpy(flat if src_kind == "f16" else flat.astype(np.float32)).cuda()
+                n = row0 + rows + 2
+                jobs.append(dict(tables=tables, src=src[lead:], src_row_stride=stride, rows=rows, dst_row0=row0,
+                                 packed=torch.full((n, p.rowBytes), 0xA5, dtype=torch.uint8, device="cuda"),
+                                 norms=torch.full((n, p.normStride), 0x5A5A, dtype=torch.int16, device="cuda")))
+            batched.encode(device, jobs, src_kind)
+            device.synchronize()
+            for j, (rows, _, _, row0), (ref_p, ref_n) in zip(jobs, shapes, refs):
+                got_p, got_n = j["packed"].cpu().numpy(), j["norms"].cpu().numpy().view(np.uint16)
+                outside = np.r_[0:row0, row0 + rows:len(got_p)]
+                assert np.all(got_p[outside] == 0xA5) and np.all(got_n[outside] == 0x5A5A), (src_kind, rows)
+                assert np.array_equal(got_p[row0:row0 + rows], ref_p), (src_kind, rows)
+                assert np.array_equal(got_n[row0:row0 + rows], ref_n), (src_kind, rows)
+    finally:
+        tables.destroy()
 
 
 def test_bulk_encoder_unaligned_source(device, oracle):
