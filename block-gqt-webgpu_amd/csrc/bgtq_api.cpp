@@ -1278,9 +1278,12 @@ bgtq_status bgtq_decode_workspace_size(const bgtq_decode_desc *d, size_t *bytes)
   if (bgtq_status s = validate_decode(d, &splits)) return s;
   if (!bytes) return fail(BGTQ_ERR_RANGE, "null output");
   const int64_t units = (int64_t)d->batch * d->kv_heads;
-  // For either entry point, so that a call's split does not depend on which one the workspace was sized for.
-  for (int extra = 0; extra < 2 && d->splits <= 0; ++extra)
-    splits = std::max(splits, fused_decode_splits(units, d->max_length, extra));
+  // Room for the splits an append takes beyond the decode's, so that no call's
+  // split depends on the workspace; whether the count is forced or the library's, so
+  // that a size asked with the library's count is the size asked with none.
+  const int own = std::max(choose_splits(units, d->max_length, 0), fused_decode_splits(units, d->max_length, 0));
+  if (d->splits <= 0) splits = own;
+  splits += std::max(0, fused_decode_splits(units, d->max_length, 1) - own);
   *bytes = decode_ws(units, (int64_t)d->batch * d->q_heads, d->dim, splits).total;
   return BGTQ_OK;
 }

@@ -554,21 +554,27 @@ def test_model_commands_take_what_they_took(monkeypatch):
     assert submit(tables(ctypes.c_void_p(0)))[2] == (None, 0, None)
 
 
-@pytest.mark.parametrize("batch,kv_heads,tokens,append_splits", [(64, 2, 32768, 7), (43, 3, 8192, 6), (256, 2, 8192, 3),
-                                                                 (150, 2, 8000, 4), (21, 3, 8191, 7)])
-def test_decode_workspace_serves_an_append(batch, kv_heads, tokens, append_splits):
+@pytest.mark.parametrize("batch,kv_heads,tokens,own_splits,append_splits",
+                         [(64, 2, 32768, 4, 7), (43, 3, 8192, 4, 6), (256, 2, 8192, 1, 3), (150, 2, 8000, 5, 4),
+                          (21, 3, 8191, 9, 7)])
+def test_decode_workspace_serves_an_append(batch, kv_heads, tokens, own_splits, append_splits):
     """The workspace bgtq_decode_workspace_size names holds the partials of the splits a decode with an
     appended token takes by itself (two workgroups on each of 256 compute units), so that a call's split
-    does not depend on whether a larger workspace was given."""
+    does not depend on whether a larger workspace was given; asked with the decode's own count it is the
+    same, with another count another."""
     import bgtq  # noqa: F401  (loads the library)
     from bgtq import _lib, batched
+    heads, dim = batch * kv_heads * 3, 64
 
     def size(splits):
         d = _lib.DecodeDesc()
-        d.batch, d.q_heads, d.kv_heads, d.dim = batch, kv_heads * 3, kv_heads, 64
+        d.batch, d.q_heads, d.kv_heads, d.dim = batch, kv_heads * 3, kv_heads, dim
         d.key_format, d.v_dtype, d.max_length, d.splits = _lib.KEYS_FP16, _lib.DTYPE_F16, tokens, splits
         for name in ("k_f16", "v", "q", "out", "lengths"):
             setattr(d, name, 4096)  # never read
         return batched.workspace_bytes(d)
 
-    assert size(0) >= size(append_splits)
+    # counters, rotated queries, statistics; then (m, l, o) of every split and of the appended token
+    fixed = 64 * max(batch * kv_heads, 1024) + 4 * heads * dim + 8 * heads
+    assert size(0) >= fixed + 4 * heads * (append_splits + 1) * (dim + 2)
+    assert size(own_splits) == size(0) != size(own_splits + 1)
