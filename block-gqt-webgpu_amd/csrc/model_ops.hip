@@ -306,7 +306,9 @@ __global__ __launch_bounds__(kRowThreads) void model_softmax_kernel(ModelAttnPar
 // Eight waves: the loads of nine tokens a thread in flight cover 4608 tokens
 // in one round trip, and the reductions at the end (a wave's worth of
 // instructions each) share a SIMD with one other wave (9 heads x 4097
-// tokens: 8.0 us, 8.9 with 16 waves of five tokens).
+// tokens: 8.0 us, 8.9 with 16 waves of five tokens); longer histories take
+// more rounds (a whole SmolLM2 layer's dispatches, us, general kernels / these: 1
+// row after 4096 tokens 290 / 62, 9000 420 / 70, 16,000 1112 / 91, 40,000 2970 / 143).
 constexpr int kFewItems = 4, kFewThreads = 512;
 
 template <bool ALIGNED>
@@ -388,8 +390,10 @@ __global__ __launch_bounds__(kFewThreads) void model_weighted_few_kernel(ModelAt
 // More items: 16 items by 16 dimensions a workgroup, in FP32 on the matrix
 // cores (16x16x4), its eight waves taking every eighth block of 16 tokens
 // and meeting in LDS; the items' probabilities come through LDS (kChunk
-// tokens at a time). Bound: the products and one memory round trip per four
-// blocks of V. Grid: (d / 16, tiles of 16 items, KV heads).
+// tokens at a time, within the LDS of one workgroup). Bound: the products and one memory round trip per four
+// blocks of V. A whole SmolLM2 layer's dispatches, us, general kernels / these: 32 rows
+// after 10 tokens 186 / 65, 2016 240 / 78, 4064 310 / 101, 8000 705 / 136; 200
+// rows after 4000 768 / 180. Grid: (d / 16, tiles of 16 items, KV heads).
 constexpr int kWeightedWaves = 8, kProbChunk = 2176, kProbRow = kProbChunk + 4;
 constexpr int kProbBytes = 16 * kProbRow * 4;
 

@@ -2,7 +2,7 @@
  *
  * A plain-C restatement of the reference's Python path (encode, pack, unpack,
  * reconstruct, attention, allocator). Only tests/, the smoke check
- * and bench.py's CPU-baseline leg may load it, and only as the checker. The
+ * and bench.py's CPU-baseline leg may load it, to compare with. The
  * product library (libbgtq.so) never links or calls anything declared here.
  */
 #ifndef BGTQ_ORACLE_H

@@ -233,9 +233,9 @@ def test_fp32_values_benchmark_shapes(device, attention_cases, oracle, T):
 
 
 def test_fp32_values_beyond_fp16_range(device, attention_cases, oracle):
-    """FP32 V with a value past FP16's range (|v| >= 65504) cannot be split
-    into FP16 parts: the session computes it on the general kernels, with the
-    same result bar, and an FP16 K session likewise."""
+    """FP32 V with a value past FP16's range (|v| >= 65504): the session takes
+    the instance with FP32 QK, with the same result bar, and an FP16 K session
+    likewise."""
     import bgtq
     name, m, a, lm, la = next(c for c in attention_cases if c[0] == "t256_d64")
     T, d = m["context_length"], m["dim"]

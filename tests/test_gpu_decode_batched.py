@@ -127,7 +127,8 @@ def test_forced_splits_long(device, oracle, splits):
 
 
 def test_non_fast_layouts_use_general_kernel(device, oracle):
-    """Layouts whose K-steps mix groups (a real SmolLM2 head; layout A) run the general kernel."""
+    """Layouts whose K-steps mix groups (real SmolLM2 heads; layout A) over caches whose strides are no
+    multiple of 16 bytes run the general kernel."""
     from bgtq import BlockGTQParameters, calibrate
     m, a = oracle.read_fixture(REF / "model" / "calibration.json")
     heads = [BlockGTQParameters.from_serialized(a[f"h{i}_config"], a[f"h{i}_table"]) for i in (3, 4, 5)]

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle before it is trusted as the checker.
+"""Pins the CPU oracle before anything is compared with it.
 
 Every oracle function is checked against the reference's committed goldens
 (tests/golden/reference, copied data), against torch itself where the

@@ -1,7 +1,7 @@
 """bgtq_decode_noalloc (the decode with the library's own device scratch, no allocation) against
 bgtq_decode with a caller workspace, through the C ABI: identical outputs on two calls in a row,
-the second with a smaller input, on the fused kernel (packed layout B, FP16 K) and the general
-kernel (FP32 V); launches whose workspace exceeds the scratch are refused before anything is
+the second with a smaller input, on the fused kernel (packed layout B with FP16 and FP32 V, FP16 K)
+and the general kernel (scale strides that are no multiple of 16 bytes); launches whose workspace exceeds the scratch are refused before anything is
 queued."""
 import ctypes
 
@@ -11,7 +11,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _case(device, *, batch, hkv, hq, dim, T, key_format, v_dtype, seed, splits=0):
+def _case(device, *, batch, hkv, hq, dim, T, key_format, v_dtype, seed, splits=0, general=False):
     import torch
     import bgtq
     from bgtq import batched, calibrate
@@ -27,7 +27,7 @@ def _case(device, *, batch, hkv, hq, dim, T, key_format, v_dtype, seed, splits=0
         p = calibrate.layout_b(dim)
         tabs = [bgtq.Tables(device, p) for _ in range(hkv)]
         packed = torch.zeros((batch, hkv, (T * p.rowBytes + 64 + 15) // 16 * 16), dtype=torch.uint8, device="cuda")
-        norms = torch.zeros((batch, hkv, (T * p.normStride + 32 + 7) // 8 * 8), dtype=torch.int16, device="cuda")
+        norms = torch.zeros((batch, hkv, (T * p.normStride + 32 + 7) // 8 * 8 + (2 if general else 0)), dtype=torch.int16, device="cuda")
         batched.encode(device, [dict(tables=tabs[h], src=k[b, h], src_row_stride=dim, rows=T, packed=packed[b, h],
                                      norms=norms[b, h]) for b in range(batch) for h in range(hkv)], "f16")
         kw = dict(tables=tabs, packed=packed, packed_seq_stride=packed.stride(0), packed_head_stride=packed.stride(1),
@@ -63,14 +63,14 @@ def _both(device, args):
     return outs
 
 
-@pytest.mark.parametrize("key_format,v_dtype,dim", [("packed", "f16", 64), ("fp16", "f16", 128),
-                                                    ("packed", "f32", 64)])
-def test_noalloc_matches_decode_twice_second_smaller(device, key_format, v_dtype, dim):
+@pytest.mark.parametrize("key_format,v_dtype,dim,general", [("packed", "f16", 64, False), ("fp16", "f16", 128, False),
+                                                            ("packed", "f32", 64, False), ("packed", "f32", 64, True)])
+def test_noalloc_matches_decode_twice_second_smaller(device, key_format, v_dtype, dim, general):
     first = dict(batch=4, hkv=2, hq=14, T=5000, seed=1)
     second = dict(batch=2, hkv=1, hq=7, T=900, seed=2, splits=5)
     for shape in (first, second):
         print("noalloc", key_format, v_dtype, dim, shape, flush=True)
-        args, keep, tabs = _case(device, dim=dim, key_format=key_format, v_dtype=v_dtype, **shape)
+        args, keep, tabs = _case(device, dim=dim, key_format=key_format, v_dtype=v_dtype, general=general, **shape)
         try:
             ref, got = _both(device, args)
             assert np.isfinite(ref).all()
@@ -152,11 +152,12 @@ def test_noalloc_allocates_nothing_and_captures(device, key_format, dim):
 
 def test_decode_workspace_shared_across_geometries(device):
     """One workspace, zeroed once, shared by bgtq_decode calls of changing geometries (a small
-    batch on the general kernels, larger ones on the fused kernel, twice round), and the library
+    batch on the general kernel, others on the fused kernel, twice round), and the library
     scratch of bgtq_decode_noalloc likewise: every output equals that of a fresh workspace."""
     import torch
     from bgtq import batched
-    shapes = [dict(batch=2, hkv=1, hq=7, T=900, seed=2, splits=5, key_format="packed", v_dtype="f32", dim=64),
+    shapes = [dict(batch=2, hkv=1, hq=7, T=900, seed=2, splits=5, key_format="packed", v_dtype="f32", dim=64, general=True),
+              dict(batch=2, hkv=2, hq=14, T=900, seed=3, key_format="packed", v_dtype="f32", dim=64),
               dict(batch=3, hkv=2, hq=14, T=3000, seed=5, key_format="packed", v_dtype="f16", dim=64),
               dict(batch=1, hkv=1, hq=7, T=500, seed=7, key_format="fp16", v_dtype="f16", dim=128),
               dict(batch=6, hkv=2, hq=14, T=2000, seed=9, key_format="packed", v_dtype="f16", dim=64)]
