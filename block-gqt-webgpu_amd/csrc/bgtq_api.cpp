@@ -959,7 +959,9 @@ double cut_long_jobs(std::vector<EncodePart> &parts, int dim, int64_t resident, 
     return tile_us(dim, rounds > 1.0 ? std::max(walk, load + rounds) : walk, load) + launches * kEncodeUploadUs;
   };
   double best = estimate(longest, parts.size());
-  if ((double)longest * (double)parts.size() <= 2.0 * (double)total) return best;
+  // (a table full of jobs has none left for parts, and the search below takes host time for each)
+  if (parts.size() >= (size_t)kEncodeJobTable || (double)longest * (double)parts.size() <= 2.0 * (double)total)
+    return best;
   const double floor = tile_us(dim, (double)((passes + resident - 1) / resident), (double)passes / (double)resident);
   if (best - floor < kEncodeUploadUs * (1.0 + (double)((parts.size() - 1) / per_launch))) return best;
   int64_t piece = 0;

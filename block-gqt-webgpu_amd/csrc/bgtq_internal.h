@@ -12,7 +12,7 @@ constexpr int kMaxDim = 128;
 constexpr int kMaxGroups = 8;
 constexpr int kMaxKvHeads = 16;
 constexpr int kEncodeJobsPerLaunch = 60;  // 64-byte jobs: the launch stays under 4 KB of kernel arguments
-constexpr int kEncodeJobTable = 4096;     // jobs in a context's device job table (thread-per-row encoders)
+constexpr int kEncodeJobTable = 4096;     // jobs in a context's device job table (calls from 16384 rows)
 
 // Device-resident calibration tables, built once on the host from the
 // reference's serialized tables (src/webgpu/layout.ts:24-31). Fixed header,
